@@ -335,6 +335,8 @@ def _stack64(case, weights, x, causal, mask):
 
 
 def exact(case, seed):
+    if work(case)["flops"] > 5e12:   # the 100,000-token block: half a minute in float64
+        return None
     inputs = _inputs(case, seed)
     kind = case["kind"]
     with torch.inference_mode():
