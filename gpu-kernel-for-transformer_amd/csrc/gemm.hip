@@ -211,6 +211,14 @@ __device__ __forceinline__ void slab_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// The same with this wave's LDS writes completed first: the barrier alone does
+// not wait for them (nor does the compiler, for this target), so a wave could
+// read what another wave's write in flight has not yet put there.
+__device__ __forceinline__ void lds_slab_barrier() {
+  __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14));  // vmcnt(63) expcnt(7) lgkmcnt(0)
+  slab_barrier();
+}
+
 __device__ __forceinline__ int row128_offset(int r, int c) { return r * 128 + ((c ^ (r & 7)) << 4); }
 
 // V of a packed QKV projection written transposed per head for the long-
@@ -344,7 +352,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_dma_kernel(
           for (int e = 0; e < 4; ++e) vs[(col + e) * BM + p] = to_half_pinned(acc[i][j][e] + b[e]);
         }
       }
-      slab_barrier();
+      lds_slab_barrier();
       constexpr int NT = 64 * NW, CPF = BM / 8;  // 16-byte chunks per staged feature row
       static_assert((BN * CPF) % NT == 0, "whole rounds of chunks");
 #pragma unroll
@@ -389,7 +397,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_dma_kernel(
       *reinterpret_cast<half4_t*>(cs + row * BN + 8 * ((col / 8) ^ (row & SW)) + (col & 7)) = h;
     }
   }
-  slab_barrier();
+  lds_slab_barrier();
   constexpr int NT = 64 * NW;
   static_assert((BM * CPR) % NT == 0, "whole rounds of 16-byte chunks");
 #pragma unroll
