@@ -52,6 +52,8 @@ XB_LINEAR_DMA_128x256 = 2
 XB_LINEAR_DMA_128x128 = 3
 XB_LINEAR_NT_128x128 = 4
 XB_LINEAR_NT_64x64 = 5
+XB_LINEAR_ROWS = 6
+XB_LINEAR_DMA_64x64 = 7
 XB_ATTN_W4_Q16 = 0
 XB_ATTN_W4_Q32 = 1
 XB_ATTN_W4_Q64 = 2

@@ -224,7 +224,8 @@ def resolve_shape_execution_plan(
             and d % 128 == 0 and d >= 256):
         widths = {_capi.XB_LINEAR_DMA_256x256: 256, _capi.XB_LINEAR_DMA_128x256: 256, _capi.XB_LINEAR_DMA_128x128: 128}
         if d % widths.get(qkv, d + 1) != 0:
-            qkv = _capi.XB_LINEAR_DMA_256x256 if d % 256 == 0 else _capi.XB_LINEAR_DMA_128x128
+            wide = d % 256 == 0 and qkv in (_capi.XB_LINEAR_DMA_256x256, _capi.XB_LINEAR_DMA_256x192)
+            qkv = _capi.XB_LINEAR_DMA_256x256 if wide else _capi.XB_LINEAR_DMA_128x128
         attn = _capi.XB_ATTN_PINGPONG_VT
     lin = lambda v: _variant_name(lib, _capi.XB_OP_LINEAR, v)  # noqa: E731
     return ShapeExecutionPlan(

@@ -37,6 +37,8 @@ extern "C" const char* xb_variant_name(int op, int variant) {
         case XB_LINEAR_DMA_128x128: return "mfma_gemm_dma_128x128";
         case XB_LINEAR_NT_128x128: return "mfma_gemm_nt_128x128";
         case XB_LINEAR_NT_64x64: return "mfma_gemm_nt_64x64";
+        case XB_LINEAR_ROWS: return "mfma_gemm_rows";
+        case XB_LINEAR_DMA_64x64: return "mfma_gemm_dma_64x64";
         default: return nullptr;
       }
     case XB_OP_ATTENTION:

@@ -9,9 +9,10 @@
 // computes GELU with tanh (triton_fused_ffn.py:198-213); the baseline it must
 // match uses exact erf (torch_transformer_benchmark.py:286), as done here.
 //
-// Two kernels:
-//  * gemm_dma_kernel (K % 64 == 0, K >= 256): 8 waves, up to 256 x 256 tiles,
+// Three kernels:
+//  * gemm_dma_kernel (K % 64 == 0, K >= 256): 64 x 64 up to 256 x 256 tiles,
 //    direct global -> LDS loads; used for the D >= 256 projections and FFN.
+//  * gemm_rows_kernel (M <= 32, K % 32 == 0, N % 16 == 0): decode steps.
 //  * gemm_nt_kernel (any K % 8 == 0): 4 waves in a 2 x 2 grid, tiles of A and
 //    W go global -> registers -> padded LDS, double buffered; the epilogue
 //    stages the FP16 tile through LDS so the stores to C are full 16-byte row
@@ -38,20 +39,23 @@ __device__ __forceinline__ int xcd_contiguous_tile(int b, int nb) {
 }
 
 // Tile coordinates of the direct-to-LDS kernel: tiles are ordered in bands of
-// four row blocks, column by column inside a band, and each XCD takes a
-// contiguous range of that order (xcd_contiguous_tile).  One round of 32
-// tiles on an XCD then covers 4 row blocks x 8 column blocks instead of 2 x 16
-// (row-major), which for the QKV projection (N = 3072) reads 5 MB of distinct
-// operands per round instead of 7 MB through that XCD's 4 MB L2, and the next
-// round keeps the same A rows.  Measured, outputs bitwise equal: 8192 x 3072
-// x 1024 (256 x 192 tiles) 62.5 -> 60.3-61.6 us, 3.2M x 3072 x 1024 (256 x
-// 256) 20.9 -> 19.6 ms, 3.2M x 1024 x 1024 7.23 -> 7.08 ms.
-constexpr int kGemmBandRows = 4;
+// 1024 rows (four row blocks of 256), column by column inside a band, and
+// each XCD takes a contiguous range of that order (xcd_contiguous_tile).  One
+// round of 32 256 x 256 tiles on an XCD then covers 4 row blocks x 8 column
+// blocks instead of 2 x 16 (row-major), which for the QKV projection (N =
+// 3072) reads 5 MB of distinct operands per round instead of 7 MB through
+// that XCD's 4 MB L2, and the next round keeps the same A rows.  Measured,
+// outputs bitwise equal: 3.2M x 3072 x 1024 (256 x 256) 20.9 -> 19.6 ms, 3.2M
+// x 1024 x 1024 7.23 -> 7.08 ms; lower tiles with the same band height
+// instead of four row blocks: 65536 x 3072 x 1024 (128 x 192) 438 -> 419 us,
+// 65536 x 2304 x 768 (64 x 64) 405 -> 368 us.
+template <int BM>
 __device__ __forceinline__ void banded_tile(int tile, int tiles_m, int tiles_n, int& tm, int& tn) {
-  const int band = tile / (kGemmBandRows * tiles_n);
-  const int l = tile - band * kGemmBandRows * tiles_n;
-  const int rows = min(kGemmBandRows, tiles_m - band * kGemmBandRows);  // the last band may be shorter
-  tm = band * kGemmBandRows + l % rows;
+  constexpr int kBandRows = 1024 / BM;
+  const int band = tile / (kBandRows * tiles_n);
+  const int l = tile - band * kBandRows * tiles_n;
+  const int rows = min(kBandRows, tiles_m - band * kBandRows);  // the last band may be shorter
+  tm = band * kBandRows + l % rows;
   tn = l / rows;
 }
 
@@ -178,14 +182,21 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_nt_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Large-tile kernel for K % 64 == 0.  8 waves (2 per SIMD) share a BM x BN
+// Large-tile kernel for K % 64 == 0.  Up to 8 waves share a BM x BN
 // tile; each wave owns a (BM/WGM) x (BN/WGN) sub-tile with its FP32
 // accumulators in VGPRs.  Operands reach LDS by direct global -> LDS loads
 // (global_load_lds_dwordx4), one 64-wide K slab at a time, in a ring of ST
 // slab stages: slab kt+ST is requested as soon as every wave has read slab
-// kt, so ST-1 slabs are in flight while one is consumed.  With one block per
-// CU nothing else hides the memory latency, so the ring depth is what keeps
-// the MFMAs fed when the grid is a single round of tiles.
+// kt, so ST-1 slabs are in flight while one is consumed.
+//
+// What is left over is each tile's start (the first slab's latency) and end
+// (the output stores), which nothing hides while a CU holds one tile: for
+// 8192 x 3072 x 1024 time against K put 17 of 55 us there.  So the tiles below
+// 256 x 256 are eight waves of at most 128 registers and at most 80 KB of LDS,
+// and a CU runs two of them, one starting or storing while the other
+// multiplies: 8192 x 3072 x 1024 54.5 -> 50.2 us (256 x 192 by one block ->
+// two of 128 x 192), 3001 x 3072 x 1024 26.1 -> 23.2 us, 8192 x 1024 x 1024
+// 21.0 -> 19.4 us (128 x 128 by four waves -> by eight).
 //
 // LDS slab layout: the A rows (BM) and then the W rows (BN), 128 bytes each
 // (64 halves = eight 16-byte chunks).  Chunk c of row r lives at slot
@@ -247,7 +258,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_dma_kernel(
   static_assert(ST >= 2 && ST * SLAB <= 160 * 1024 && (ST - 1) * SPW < 64, "slab ring");
   __shared__ __attribute__((aligned(1024))) char smem[ST * SLAB];
   int tile_m, tile_n;
-  banded_tile(xcd_contiguous_tile(blockIdx.x, gridDim.x), gridDim.x / tiles_n, tiles_n, tile_m, tile_n);
+  banded_tile<BM>(xcd_contiguous_tile(blockIdx.x, gridDim.x), gridDim.x / tiles_n, tiles_n, tile_m, tile_n);
   const int m0 = tile_m * BM, n0 = tile_n * BN;
   const int lane = threadIdx.x % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -411,6 +422,86 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_dma_kernel(
   }
 }
 
+// ---------------------------------------------------------------------------
+// Few-row kernel (M <= 32: decode steps, short prompts).  The product is then
+// a single pass over the weights, so what counts is how many CUs pull them
+// and how much each has in flight: a 128 x 128 tile at M = 4 put N = 1024 on
+// 8 CUs, each waiting on one slab at a time (13 us).  Here a block owns 16
+// output columns and its waves split K, 256 of it each, so the block's whole
+// weight slab (and the activations) is requested in the first instructions,
+// straight into registers.  The partial sums are not added up: wave w starts
+// its products from wave w - 1's accumulator (handed over in LDS), which
+// keeps one chain over K per output, the same products in the same order and
+// so the same bits as every other tile; a row's result does not depend on how
+// many rows are in the call.  Row groups of 16 follow each other down the
+// chain.
+constexpr int kRowsMax = 32, kRowsSteps = 8, kRowsMaxK = 16 * kRowsSteps * 32;
+
+template <int RG, int EPI>
+__global__ __launch_bounds__(1024) void gemm_rows_kernel(
+    const half_t* __restrict__ A, const half_t* __restrict__ W,
+    const float* __restrict__ bias, half_t* __restrict__ C, int M, int N, int K) {
+  __shared__ float4_t hand[16][RG][kWave];
+  const int lane = threadIdx.x % kWave, g = lane / 16, r16 = lane % 16;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int waves = blockDim.x / kWave;
+  const int n0 = blockIdx.x * 16;
+  const int steps = min(kRowsSteps, K / 32 - wave * kRowsSteps);  // >= 1: waves = ceil(K / 256)
+  const half_t* wrow = W + (int64_t)(n0 + r16) * K + wave * (kRowsSteps * 32) + 8 * g;
+  const half_t* arow = A + wave * (kRowsSteps * 32) + 8 * g;
+  half8_t wf[kRowsSteps], af[RG][kRowsSteps];
+  // Steps past the end repeat the last one's loads and are not multiplied.
+  auto load_a = [&](int rg) {
+    const half_t* p = arow + (int64_t)min(16 * rg + r16, M - 1) * K;
+#pragma unroll
+    for (int s = 0; s < kRowsSteps; ++s) af[rg][s] = *reinterpret_cast<const half8_t*>(p + 32 * min(s, steps - 1));
+  };
+#pragma unroll
+  for (int s = 0; s < kRowsSteps; ++s) wf[s] = *reinterpret_cast<const half8_t*>(wrow + 32 * min(s, steps - 1));
+  load_a(0);
+  if constexpr (RG > 1) load_a(1);
+  float b[4] = {0.f, 0.f, 0.f, 0.f};
+  if (wave == waves - 1 && bias != nullptr) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) b[e] = bias[n0 + 4 * g + e];
+  }
+  // Every wave passes waves + RG - 1 barriers; row group rg is at wave w
+  // between the barriers w + rg and w + rg + 1.
+  for (int i = 0; i < wave; ++i) lds_slab_barrier();
+#pragma unroll
+  for (int rg = 0; rg < RG; ++rg) {
+    float4_t acc = {0.f, 0.f, 0.f, 0.f};
+    if (wave > 0) acc = hand[wave - 1][rg][lane];
+#pragma unroll
+    for (int s = 0; s < kRowsSteps; ++s)
+      if (s < steps) acc = mfma16x16x32(wf[s], af[rg][s], acc);
+    if (wave + 1 < waves) {
+      hand[wave][rg][lane] = acc;
+    } else if (16 * rg + r16 < M) {  // lane: row r16, columns 4g .. 4g + 3
+      half4_t h;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float v = acc[e] + b[e];
+        if constexpr (EPI == XB_EPI_BIAS_GELU) v = gelu_erf(v);
+        h[e] = to_half_pinned(v);
+      }
+      *reinterpret_cast<half4_t*>(C + (int64_t)(16 * rg + r16) * N + n0 + 4 * g) = h;
+    }
+    lds_slab_barrier();
+  }
+  for (int i = wave + 1; i < waves; ++i) lds_slab_barrier();
+}
+
+template <int EPI>
+static hipError_t launch_gemm_rows(const half_t* a, const half_t* w, const float* bias, half_t* c,
+                                   int64_t m, int n, int k, hipStream_t s) {
+  const dim3 grid((unsigned)(n / 16)), block((unsigned)(kWave * ((k + 255) / 256)));
+  const int rows = (int)m;
+  if (m <= 16) hipLaunchKernelGGL((gemm_rows_kernel<1, EPI>), grid, block, 0, s, a, w, bias, c, rows, n, k);
+  else hipLaunchKernelGGL((gemm_rows_kernel<2, EPI>), grid, block, 0, s, a, w, bias, c, rows, n, k);
+  return hipGetLastError();
+}
+
 template <int BM, int BN, int WGM, int WGN, int EPI, int ST, bool VT = false>
 static hipError_t launch_gemm_dma(const half_t* a, const half_t* w, const float* bias, half_t* c,
                                   int64_t m, int n, int k, hipStream_t s, VtOut vo = {}) {
@@ -431,55 +522,71 @@ static hipError_t launch_gemm(const half_t* a, const half_t* w, const float* bia
   return hipGetLastError();
 }
 
-// Tile variants (XB_LINEAR_*): the gemm_dma_kernel tiles need K % 64 == 0
-// and K >= 256 (256 x 192 also N % 192 == 0); the gemm_nt_kernel tiles take
-// any K % 8 == 0.
+// Variants (XB_LINEAR_*): the gemm_dma_kernel tiles need K % 64 == 0 and K >=
+// 256 (256 x 192 also N % 192 == 0); the gemm_nt_kernel tiles take any K % 8
+// == 0; gemm_rows_kernel a few rows.
 static bool linear_variant_fits(int variant, int64_t m, int n, int k) {
-  (void)m;
   const bool dma = k % 64 == 0 && k >= 256;
   switch (variant) {
-    case XB_LINEAR_DMA_256x256: case XB_LINEAR_DMA_128x256: case XB_LINEAR_DMA_128x128: return dma;
+    case XB_LINEAR_DMA_256x256: case XB_LINEAR_DMA_128x256: case XB_LINEAR_DMA_128x128:
+    case XB_LINEAR_DMA_64x64: return dma;
     case XB_LINEAR_DMA_256x192: return dma && n % 192 == 0;
     case XB_LINEAR_NT_128x128: case XB_LINEAR_NT_64x64: return true;
+    case XB_LINEAR_ROWS: return m <= kRowsMax && n % 16 == 0 && k % 32 == 0 && k <= kRowsMaxK;
     default: return false;
   }
 }
 
-// The library's choice for a shape.  With the DMA tiles one block runs per
-// CU, so the cost is taken as rounds of 256 tiles x tile area, the 256 x 256
-// tile ~15% cheaper per output (fewer LDS bytes per MFMA); 256 x 192 sits
-// between them and fills whole rounds where 256 x 256 leaves half a round
-// idle (M = 8192, N = 3072: 54 vs 60 us).  With the banded tile order a
-// 128 x 128 round on an XCD reads about 3 MB of distinct operands at N =
-// 1024, inside its 4 MB L2, and costs ~5% less per output than 128 x 256:
-// a sweep (us, 256x256 / 128x256 / 128x128) of 8192 x 1024 x 1024 gave
-// 31.4 / 22.5 / 21.2, 16384 x 1024 35.4 / 40.9 / 39.6, 3.2M x 1024
-// 7311 / 8542 / 8052, and the factors below reproduce every best choice of
-// that sweep (also 4096 x 1024, 4096 / 8192 / 3.2M x 3072).
+// The library's choice for a shape.  Up to kRowsMax rows the few-row kernel is
+// the faster one at every N and K it takes.  A DMA tile costs rounds of one
+// tile per CU, r = ceil(tiles / 256), times what a tile costs a busy CU; the
+// microseconds below are at K = 1024 (all of them grow with K alike) and
+// reproduce a sweep over 777 to 65536 rows, N 512 to 4096, K 512 to 4096 to
+// within 10 %, or pick a tile within 10 % of its best.  64 x 64 tiles read the
+// most operand bytes per output but start and end in the least time and are
+// the only ones with a block for every CU at a few hundred rows (1500 x 1024:
+// 8.2 us against 13.1 with 128 x 128); 128 x 192 pairs (XB_LINEAR_DMA_256x192)
+// are the cheapest per output up to 16384 rows, 256 x 256 beyond.
 static int select_linear(int64_t m, int n, int k) {
+  if (linear_variant_fits(XB_LINEAR_ROWS, m, n, k)) return XB_LINEAR_ROWS;
   auto tiles = [&](int64_t bm, int64_t bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
+  auto rounds = [&](int64_t bm, int64_t bn) { return (double)((tiles(bm, bn) + 255) / 256); };
   if (k % 64 == 0 && k >= 256) {
-    const int64_t big = (tiles(256, 256) + 255) / 256 * 65536 * 85 / 100;
-    const int64_t wide = n % 192 == 0 ? (tiles(256, 192) + 255) / 256 * 49152 * 90 / 100 : INT64_MAX;
-    const int64_t mid = (tiles(128, 256) + 255) / 256 * 32768;
-    const int64_t small = (tiles(128, 128) + 255) / 256 * 16384 * 95 / 100;
+    const double big = 32.0 * rounds(256, 256) - 1.0;
+    const double wide = n % 192 == 0 ? 12.0 * rounds(128, 192) : 1e30;
+    const double mid = 8.6 * rounds(128, 128) + 2.5;
+    const double small = 3.1 * rounds(64, 64) + 1.5;
     if (big <= wide && big <= mid && big <= small) return XB_LINEAR_DMA_256x256;
     if (wide <= mid && wide <= small) return XB_LINEAR_DMA_256x192;
-    if (mid <= small) return XB_LINEAR_DMA_128x256;
-    return XB_LINEAR_DMA_128x128;
+    return mid <= small ? XB_LINEAR_DMA_128x128 : XB_LINEAR_DMA_64x64;
   }
   return tiles(128, 128) >= 512 ? XB_LINEAR_NT_128x128 : XB_LINEAR_NT_64x64;
+}
+
+// 64 x 64 tiles: two slabs ahead (a ring of three) where the grid is at most a
+// round, or two with a long K -- the operands of such a product are too much
+// for the L2s and its blocks too few to hide each other's misses (1500 x 768 x
+// 3072 24.2 -> 20.3 us, 777 x 1024 x 4096 30.4 -> 19.6) -- else a ring of two,
+// which lets five blocks share a CU (8192 x 1024 x 1024 28.1 against 25.8 us).
+template <int EPI>
+static hipError_t launch_gemm_64(const half_t* a, const half_t* w, const float* bias, half_t* c,
+                                 int64_t m, int n, int k, hipStream_t s) {
+  const int64_t tiles = ((m + 63) / 64) * ((n + 63) / 64);
+  if (tiles <= 256 || (tiles <= 512 && k >= 2048)) return launch_gemm_dma<64, 64, 4, 2, EPI, 3>(a, w, bias, c, m, n, k, s);
+  return launch_gemm_dma<64, 64, 2, 2, EPI, 2>(a, w, bias, c, m, n, k, s);
 }
 
 template <int EPI>
 static hipError_t run_gemm(int variant, const half_t* a, const half_t* w, const float* bias, half_t* c,
                            int64_t m, int n, int k, hipStream_t s) {
   switch (variant) {
-    case XB_LINEAR_DMA_256x256: return launch_gemm_dma<256, 256, 4, 2, EPI, 2>(a, w, bias, c, m, n, k, s);
-    case XB_LINEAR_DMA_256x192: return launch_gemm_dma<256, 192, 4, 2, EPI, 2>(a, w, bias, c, m, n, k, s);
+    case XB_LINEAR_DMA_256x256: return launch_gemm_dma<256, 256, 2, 4, EPI, 2>(a, w, bias, c, m, n, k, s);
+    case XB_LINEAR_DMA_256x192: return launch_gemm_dma<128, 192, 2, 4, EPI, 2>(a, w, bias, c, m, n, k, s);  // two per CU
     case XB_LINEAR_DMA_128x256: return launch_gemm_dma<128, 256, 2, 4, EPI, 2>(a, w, bias, c, m, n, k, s);
-    case XB_LINEAR_DMA_128x128: return launch_gemm_dma<128, 128, 2, 2, EPI, 2>(a, w, bias, c, m, n, k, s);
+    case XB_LINEAR_DMA_128x128: return launch_gemm_dma<128, 128, 2, 4, EPI, 2>(a, w, bias, c, m, n, k, s);
+    case XB_LINEAR_DMA_64x64: return launch_gemm_64<EPI>(a, w, bias, c, m, n, k, s);
     case XB_LINEAR_NT_128x128: return launch_gemm<128, 128, 2, 2, EPI>(a, w, bias, c, m, n, k, s);
+    case XB_LINEAR_ROWS: return launch_gemm_rows<EPI>(a, w, bias, c, m, n, k, s);
     default: return launch_gemm<64, 64, 2, 2, EPI>(a, w, bias, c, m, n, k, s);
   }
 }
@@ -537,7 +644,8 @@ extern "C" int xb_linear_qkv_vt(const void* a, const void* w, const float* bias,
   if (seq_len % 32 != 0 || head_dim % 8 != 0 || k % 64 != 0 || k < 256) return XB_ERR_UNSUPPORTED_SHAPE;
   if (variant == XB_VARIANT_AUTO) {
     variant = select_linear(m, n, k);
-    if (variant == XB_LINEAR_DMA_256x192 || d % 256 != 0) variant = d % 256 == 0 ? XB_LINEAR_DMA_256x256 : XB_LINEAR_DMA_128x128;
+    if (variant == XB_LINEAR_DMA_256x192) variant = XB_LINEAR_DMA_256x256;
+    if (variant != XB_LINEAR_DMA_256x256 || d % 256 != 0) variant = XB_LINEAR_DMA_128x128;
   }
   int bn = 0;
   switch (variant) {
@@ -557,11 +665,11 @@ extern "C" int xb_linear_qkv_vt(const void* a, const void* w, const float* bias,
   hipError_t e;
   switch (variant) {
     case XB_LINEAR_DMA_256x256:
-      e = launch_gemm_dma<256, 256, 4, 2, XB_EPI_BIAS, 2, true>(A, Wt, bias, Cc, m, n, k, s, vo); break;
+      e = launch_gemm_dma<256, 256, 2, 4, XB_EPI_BIAS, 2, true>(A, Wt, bias, Cc, m, n, k, s, vo); break;
     case XB_LINEAR_DMA_128x256:
       e = launch_gemm_dma<128, 256, 2, 4, XB_EPI_BIAS, 2, true>(A, Wt, bias, Cc, m, n, k, s, vo); break;
     default:
-      e = launch_gemm_dma<128, 128, 2, 2, XB_EPI_BIAS, 2, true>(A, Wt, bias, Cc, m, n, k, s, vo); break;
+      e = launch_gemm_dma<128, 128, 2, 4, XB_EPI_BIAS, 2, true>(A, Wt, bias, Cc, m, n, k, s, vo); break;
   }
   return (int)e;
 }

@@ -65,13 +65,16 @@ const char* xb_strerror(int code);
 #define XB_OP_LINEAR 0
 #define XB_OP_ATTENTION 1
 #define XB_OP_FUSED_D128 2
-/* xb_linear_v: gemm_dma_kernel tiles (K % 64 == 0, K >= 256) and gemm_nt_kernel tiles (any K % 8 == 0). */
+/* xb_linear_v: gemm_dma_kernel tiles (DMA: K % 64 == 0, K >= 256), gemm_nt_kernel tiles (NT: any K % 8 == 0)
+ * and gemm_rows_kernel (ROWS). */
 #define XB_LINEAR_DMA_256x256 0
-#define XB_LINEAR_DMA_256x192 1   /* also N % 192 == 0 */
+#define XB_LINEAR_DMA_256x192 1   /* two 128 x 192 blocks per CU; also N % 192 == 0 */
 #define XB_LINEAR_DMA_128x256 2
 #define XB_LINEAR_DMA_128x128 3
 #define XB_LINEAR_NT_128x128 4
 #define XB_LINEAR_NT_64x64 5
+#define XB_LINEAR_ROWS 6          /* gemm_rows_kernel: M <= 32, N % 16 == 0, K % 32 == 0, K <= 4096 */
+#define XB_LINEAR_DMA_64x64 7
 /* xb_attention_v: waves per block x queries per block. */
 #define XB_ATTN_W4_Q16 0     /* head_dim 256                              */
 #define XB_ATTN_W4_Q32 1     /* head_dim <= 128                           */

@@ -151,6 +151,46 @@ def test_linear_every_variant(pkg, cuda, m, n, k, gelu):
         pkg.linear(ag[:, :k], wg[:n - 128], None, variant=capi.XB_LINEAR_DMA_256x192)
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 16, 32), (4, 3072, 1024), (15, 48, 256), (16, 1024, 288), (17, 768, 3072),
+                                   (32, 4096, 1024), (31, 528, 4096), (2, 384, 128)])
+@pytest.mark.parametrize("gelu", [False, True])
+def test_linear_few_rows(pkg, cuda, m, n, k, gelu):
+    """The few-row kernel on both sides of a 16-row group, with one wave to
+    sixteen in its K chain and a last wave that owns less than 256 of K: within
+    the FP32 reference's tolerance and bit for bit what the tiles give, so a
+    row does not depend on the row count of its call."""
+    capi = pkg._capi
+    a = torch.randn(m, k, generator=_gen(m + n)).half()
+    w = (torch.randn(n, k, generator=_gen(k)) * k**-0.5).half()
+    bias = torch.randn(n, generator=_gen(n)) * 0.1
+    ref = a.float() @ w.float().T + bias
+    if gelu:
+        ref = F.gelu(ref, approximate="none")
+    assert capi.lib().xb_select_linear(m, n, k, 0) == capi.XB_LINEAR_ROWS
+    ag, wg, bg = a.to(cuda), w.to(cuda), bias.to(cuda)
+    out = pkg.linear(ag, wg, bg, gelu=gelu)
+    torch.testing.assert_close(out.cpu().float(), ref, atol=2e-3, rtol=2e-3)
+    tile = capi.XB_LINEAR_DMA_128x128 if k % 64 == 0 and k >= 256 else capi.XB_LINEAR_NT_64x64
+    assert torch.equal(out, pkg.linear(ag, wg, bg, gelu=gelu, variant=tile))
+    with pytest.raises(RuntimeError, match="code -10"):   # 33 rows are not its shape
+        pkg.linear(torch.zeros(33, k, dtype=F16, device=cuda), wg, bg, variant=capi.XB_LINEAR_ROWS)
+
+
+@pytest.mark.parametrize("m,n,k", [(63, 64, 256), (65, 72, 320), (2000, 2304, 768), (777, 1024, 4096), (1500, 768, 3072)])
+def test_linear_small_tiles(pkg, cuda, m, n, k):
+    """64 x 64 tiles (both ring depths, several blocks per CU, ragged edges): every
+    call gives the bits of the 128 x 128 tiles.  Blocks that share a CU delay each
+    other's LDS writes, so the epilogue must wait for them before it reads the tile."""
+    capi = pkg._capi
+    a = torch.randn(m, k, generator=_gen(m + n)).half().to(cuda)
+    w = (torch.randn(n, k, generator=_gen(k)) * k**-0.5).half().to(cuda)
+    bias = torch.randn(n, generator=_gen(n)).to(cuda)
+    ref = pkg.linear(a, w, bias, variant=capi.XB_LINEAR_DMA_128x128)
+    torch.testing.assert_close(ref.cpu().float(), a.cpu().float() @ w.cpu().float().T + bias.cpu(), atol=4e-3, rtol=2e-3)
+    for _ in range(5):
+        assert torch.equal(pkg.linear(a, w, bias, variant=capi.XB_LINEAR_DMA_64x64), ref)
+
+
 def test_linear_without_bias_and_batched_shape(pkg, cuda):
     a = torch.randn(3, 5, 64, generator=_gen(1)).half()
     w = (torch.randn(32, 64, generator=_gen(2)) * 0.125).half()
