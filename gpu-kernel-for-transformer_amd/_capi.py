@@ -87,12 +87,33 @@ EXPORTED_SYMBOLS = (
     "xb_fused_forward_d128",
     "xb_fused_forward_d128_workspace_bytes",
     "xb_fused_forward_d128_ws",
+    "xb_stack_workspace_bytes",
+    "xb_stack_forward",
 )
 
 _vp = ctypes.c_void_p
 _i32 = ctypes.c_int32
 _i64 = ctypes.c_int64
 _f32 = ctypes.c_float
+
+
+class XbBlock(ctypes.Structure):
+    """xb_block of include/xblock.h."""
+
+    _fields_ = ([(name, _vp) for name in (
+        "qkv_w", "out_w", "ffn_in_w", "ffn_out_w", "qkv_b", "out_b", "ffn_in_b", "ffn_out_b",
+        "norm1_g", "norm1_b", "norm2_g", "norm2_b")]
+        + [(name, _f32) for name in ("norm1_eps", "norm2_eps", "scale")]
+        + [(name, _i32) for name in ("norm1_affine", "norm2_affine")])
+
+
+class XbStack(ctypes.Structure):
+    """xb_stack of include/xblock.h."""
+
+    _fields_ = ([("blocks", ctypes.POINTER(XbBlock)), ("final_g", _vp), ("final_b", _vp), ("final_eps", _f32)]
+                + [(name, _i32) for name in ("final_affine", "layers", "heads", "head_dim", "ffn_dim", "causal")])
+
+
 _SIGNATURES = {
     "xb_abi_version": (ctypes.c_int, []),
     "xb_strerror": (ctypes.c_char_p, [ctypes.c_int]),
@@ -134,6 +155,12 @@ _SIGNATURES = {
     "xb_fused_forward_d128_ws": (
         ctypes.c_int,
         [_vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _i64, _vp, _i32, _vp, _i64, _i32, _i32, _vp],
+    ),
+    "xb_stack_workspace_bytes": (_i64, [_i32, _i64, _i32, _i32, _i32, ctypes.c_int, _i64]),
+    "xb_stack_forward": (
+        ctypes.c_int,
+        [_vp, _vp, _vp, _vp, _i32, _i64, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+         _vp, _i64, _i64, _vp, _i64, _vp],
     ),
 }
 

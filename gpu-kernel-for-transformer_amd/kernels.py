@@ -15,6 +15,7 @@ on torch's current stream, and never synchronise: they are capture-safe.
 
 from __future__ import annotations
 
+import ctypes
 import threading
 import weakref
 from functools import lru_cache
@@ -510,6 +511,53 @@ def kv_cache_workspace_bytes(batch: int, chunk: int, num_heads: int, head_dim: i
     if need < 0:
         check(int(need), "xb_attention_kv_cache_workspace_bytes")
     return int(need)
+
+
+def recording() -> bool:
+    """Whether a LaunchRecorder is active: launches then go one by one through the wrappers above."""
+    return LaunchRecorder._active is not None
+
+
+@lru_cache(maxsize=256)
+def _stack_workspace_bytes(batch: int, seq_len: int, heads: int, head_dim: int, ffn_dim: int, attention_variant: int) -> int:
+    return int(lib().xb_stack_workspace_bytes(batch, seq_len, heads, head_dim, ffn_dim, attention_variant, -1))
+
+
+def stack_forward(
+    x: torch.Tensor,
+    stack: _capi.XbStack,
+    variants: Tuple[int, int, int, int, int],
+    out: torch.Tensor,
+    token_valid: Optional[torch.Tensor] = None,
+    caches=None,
+    cache_start: int = 0,
+    cache_capacity: int = 0,
+) -> torch.Tensor:
+    """The per-op forward of a whole stack in one native call (xb_stack_forward).
+
+    x and out: contiguous float32 [B, S, D]; token_valid: contiguous uint8 [B,
+    S] or None; variants: (qkv, out, ffn_in, ffn_out, attention) of the
+    execution plan.  caches: a ctypes array of each layer's k_cache and v_cache
+    pointers, or None.  The workspace is one allocation of torch's caching
+    allocator on the current stream, given back when the call has been issued.
+    """
+    _require_device(x, "stack_forward")
+    batch, seq_len, _ = x.shape
+    if caches is None:
+        need = _stack_workspace_bytes(batch, seq_len, stack.heads, stack.head_dim, stack.ffn_dim, variants[4])
+    else:
+        need = int(lib().xb_stack_workspace_bytes(batch, seq_len, stack.heads, stack.head_dim, stack.ffn_dim,
+                                                  variants[4], cache_start))
+    if need < 0:
+        check(need, "xb_stack_workspace_bytes")
+    workspace = torch.empty(need, device=x.device, dtype=torch.uint8)
+    check(
+        lib().xb_stack_forward(
+            ctypes.addressof(stack), x.data_ptr(), out.data_ptr(), _ptr(token_valid), batch, seq_len, *variants,
+            caches, cache_start, cache_capacity, workspace.data_ptr(), need, stream_handle(x.device)),
+        "xb_stack_forward",
+    )
+    return out
 
 
 def pack_linear_fragments(weight: torch.Tensor, natural: bool = False, scale: float = 1.0) -> torch.Tensor:

@@ -39,6 +39,7 @@ reference (TTB:503-508) there is no sequence-length limit: the key mask is a
 
 from __future__ import annotations
 
+import ctypes
 import dataclasses
 import operator
 from typing import Dict, Optional, Tuple
@@ -278,12 +279,55 @@ class UserOptimizedTransformer(nn.Module):
             cache[index] = cached
         return cached[1]
 
+    def _native_stack(self) -> Optional[Tuple[_capi.XbStack, object, object]]:
+        """(xb_stack, its xb_block array, the tensors they point into), cached by parameter version.
+
+        None when a LayerNorm has no weight or bias: the wrappers then raise
+        for it.  The descriptors are written once and only read afterwards, so
+        forwards of several threads may share them.
+        """
+        params, norms = self._tree()
+        attentions = self.__dict__["_tree_cache"][3]
+        for norm in norms:  # read on each call: setting one to None calls no registration hook
+            registered = norm._parameters
+            if registered.get("weight") is None or registered.get("bias") is None:
+                return None
+        settings = ([n.eps for n in norms], [a.scale for a in attentions])
+        try:
+            key = (tuple(map(_VERSION_OF, params)), tuple(map(torch.Tensor.data_ptr, params)), settings)
+        except RuntimeError:  # inference-mode parameters have no version counter: never reuse
+            key = None
+        cached = self.__dict__.get("_native_stack_cache")
+        if key is not None and cached is not None and cached[0] == key:
+            return cached[1]
+        cfg = self.config
+        blocks = (_capi.XbBlock * len(self.layers))()
+        weights = [self._layer_weights(i) for i in range(len(self.layers))]
+        for block, layer, w in zip(blocks, self.layers, weights):
+            for name in _LayerWeights.__slots__:
+                setattr(block, name, getattr(w, name).data_ptr())
+            for which, norm in (("norm1", layer.norm1), ("norm2", layer.norm2)):
+                setattr(block, which + "_g", norm.weight.data_ptr())
+                setattr(block, which + "_b", norm.bias.data_ptr())
+                setattr(block, which + "_eps", norm.eps)
+                setattr(block, which + "_affine", int(self._layer_norm_uses_affine(norm)))
+            block.scale = layer.attention.scale
+        final = self.final_norm
+        stack = _capi.XbStack(blocks=blocks, final_g=final.weight.data_ptr(), final_b=final.bias.data_ptr(),
+                              final_eps=final.eps, final_affine=int(self._layer_norm_uses_affine(final)),
+                              layers=len(self.layers), heads=cfg.num_heads, head_dim=cfg.head_dim,
+                              ffn_dim=cfg.ffn_dim, causal=int(cfg.causal))
+        value = (stack, blocks, weights)
+        self.__dict__["_native_stack_cache"] = (key, value)
+        return value
+
     def _tree(self) -> Tuple[Tuple[nn.Parameter, ...], Tuple[nn.LayerNorm, ...]]:
         """(parameters, LayerNorm modules) of this model, re-walked after any registration."""
         cached = self.__dict__.get("_tree_cache")
         if cached is None or cached[0] != _TREE_GENERATION[0]:
             cached = (_TREE_GENERATION[0], tuple(self.parameters()),
-                      tuple(m for m in self.modules() if isinstance(m, nn.LayerNorm)))
+                      tuple(m for m in self.modules() if isinstance(m, nn.LayerNorm)),
+                      tuple(layer.attention for layer in self.layers))
             self.__dict__["_tree_cache"] = cached
         return cached[1], cached[2]
 
@@ -477,16 +521,10 @@ class UserOptimizedTransformer(nn.Module):
                                               split=plan.fused_variant == _capi.XB_FUSED_SPLIT,
                                               strict=self._strict_handoff_checks)
 
-        def attend_with(key_valid: Optional[torch.Tensor]):
-            def attend(index: int, layer: TransformerBlockParameters, qkv: torch.Tensor) -> torch.Tensor:
-                return kernels.attention(qkv, cfg.num_heads, key_valid=key_valid, causal=cfg.causal,
-                                         scale=layer.attention.scale, variant=plan.attention_variant)
-            return attend
-
         streams = self._overlap_streams(x)
         if streams is not None and torch.cuda.is_current_stream_capturing():
-            return self._per_op_forward_overlapped(x, attend_with, plan, streams, out, token_valid)
-        return self._per_op_forward(x, attend_with(token_valid), plan, out=out, token_valid=token_valid)
+            return self._per_op_forward_overlapped(x, plan, streams, out, token_valid)
+        return self._per_op_forward(x, plan, out=out, token_valid=token_valid)
 
     # A small per-op forward captured into a hipGraph runs as two half-batches
     # on two streams forked from the capturing stream and joined back into it.
@@ -536,7 +574,7 @@ class UserOptimizedTransformer(nn.Module):
                           for h, p in zip(halves, own))
         return f"two half-batch streams under capture ({names}); QKV and attention as planned"
 
-    def _per_op_forward_overlapped(self, x: torch.Tensor, attend_with, plan: ShapeExecutionPlan,
+    def _per_op_forward_overlapped(self, x: torch.Tensor, plan: ShapeExecutionPlan,
                                    streams: Tuple[torch.cuda.Stream, torch.cuda.Stream],
                                    out: Optional[torch.Tensor], token_valid: Optional[torch.Tensor]) -> torch.Tensor:
         """_per_op_forward of each half of the batch on its own stream, joined back into the current one."""
@@ -552,8 +590,7 @@ class UserOptimizedTransformer(nn.Module):
                                             ffn_out_variant=own.ffn_out_variant)
             stream.wait_stream(main)
             with torch.cuda.stream(stream):
-                self._per_op_forward(x[start:end], attend_with(valid), half_plan, out=out[start:end],
-                                     token_valid=valid)
+                self._per_op_forward(x[start:end], half_plan, out=out[start:end], token_valid=valid)
         for stream in streams:
             main.wait_stream(stream)
         return out
@@ -581,30 +618,50 @@ class UserOptimizedTransformer(nn.Module):
             elif tuple(cached[0].shape) != expected or cached[0].device != x.device:
                 raise RuntimeError(
                     "KV cache does not match this input; reset it before changing batch size, device, or dtype")
-        need = kernels.kv_cache_workspace_bytes(batch, chunk, cfg.num_heads, cfg.head_dim, start) if start else 0
-        workspace = torch.empty(need, device=x.device, dtype=torch.uint8) if need else None
-
-        def attend(index: int, layer: TransformerBlockParameters, qkv: torch.Tensor) -> torch.Tensor:
-            k_cache, v_cache = self._kv_cache[index]
-            kernels.kv_cache_append(qkv, k_cache, v_cache, cfg.num_heads, start)
-            if start == 0:
-                return kernels.attention(qkv, cfg.num_heads, causal=True, scale=layer.attention.scale)
-            return kernels.attention_kv_cache(qkv, k_cache, v_cache, cfg.num_heads, start,
-                                              scale=layer.attention.scale, workspace=workspace)
-
         plan = self.execution_plan(batch, chunk, per_op=True)
         if not plan.runnable:
             raise ValueError(f"no gfx950 kernel sequence for this input: {plan.forward_strategy}")
-        output = self._per_op_forward(x, attend, plan)
+        output = self._per_op_forward(x, plan, cache_start=start)
         self._kv_cache_length = start + chunk
         return output
 
-    def _per_op_forward(self, x: torch.Tensor, attend, plan: ShapeExecutionPlan, out: Optional[torch.Tensor] = None,
-                        token_valid: Optional[torch.Tensor] = None) -> torch.Tensor:
-        """LN -> per layer (QKV GEMM, attend(index, layer, qkv), out GEMM, residual LN, FFN) -> final LN."""
+    def _per_op_forward(self, x: torch.Tensor, plan: ShapeExecutionPlan, out: Optional[torch.Tensor] = None,
+                        token_valid: Optional[torch.Tensor] = None, cache_start: Optional[int] = None) -> torch.Tensor:
+        """LN -> per layer (QKV GEMM, attention, out GEMM, residual LN, FFN) -> final LN, issued natively.
+
+        cache_start: None, or the position in the KV cache of x's first token.
+        While a LaunchRecorder is active the same launches go through the
+        wrappers one by one, so that each is bracketed by its events.
+        """
+        native = None if kernels.recording() else self._native_stack()
+        if native is None:
+            return self._per_op_forward_stepwise(x, plan, out, token_valid, cache_start)
+        if out is None:
+            out = torch.empty_like(x)
+        variants = (plan.qkv_variant, plan.out_variant, plan.ffn_in_variant, plan.ffn_out_variant,
+                    plan.attention_variant)
+        if cache_start is None:
+            return kernels.stack_forward(x, native[0], variants, out, token_valid=token_valid)
+        pointers = [t.data_ptr() for index in range(len(self.layers)) for t in self._kv_cache[index]]
+        return kernels.stack_forward(x, native[0], variants, out, caches=(ctypes.c_void_p * len(pointers))(*pointers),
+                                     cache_start=cache_start, cache_capacity=self.config.seq_len)
+
+    def _attend_stepwise(self, index: int, qkv: torch.Tensor, plan: ShapeExecutionPlan,
+                         token_valid: Optional[torch.Tensor], cache_start: Optional[int]) -> torch.Tensor:
+        heads, scale = self.config.num_heads, self.layers[index].attention.scale
+        if cache_start is not None:
+            k_cache, v_cache = self._kv_cache[index]
+            kernels.kv_cache_append(qkv, k_cache, v_cache, heads, cache_start)
+            if cache_start:
+                return kernels.attention_kv_cache(qkv, k_cache, v_cache, heads, cache_start, scale=scale)
+        return kernels.attention(qkv, heads, key_valid=token_valid, causal=self.config.causal, scale=scale,
+                                 variant=plan.attention_variant)
+
+    def _per_op_forward_stepwise(self, x: torch.Tensor, plan: ShapeExecutionPlan, out: Optional[torch.Tensor],
+                                 token_valid: Optional[torch.Tensor], cache_start: Optional[int]) -> torch.Tensor:
+        """_per_op_forward, one wrapper call per launch."""
         cfg = self.config
         batch, seq_len, d_model = x.shape
-        rows = batch * seq_len
         dev = x.device
         f16 = torch.float16
         num_layers = len(self.layers)
@@ -629,7 +686,7 @@ class UserOptimizedTransformer(nn.Module):
                 context = kernels.attention_vt(qkv, vt, cfg.num_heads, scale=layer.attention.scale)
             else:
                 qkv = kernels.linear(norm, w.qkv_w, w.qkv_b, variant=plan.qkv_variant)
-                context = attend(index, layer, qkv)
+                context = self._attend_stepwise(index, qkv, plan, token_valid, cache_start)
             update = kernels.linear(context, w.out_w, w.out_b, variant=plan.out_variant)
             residual_in, norm2 = kernels.fused_residual_layer_norm(
                 residual_in, update, layer.norm2.weight, layer.norm2.bias, layer.norm2.eps, f16,

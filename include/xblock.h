@@ -379,6 +379,48 @@ int xb_fused_forward_d128_ws(const float* x, float* y, const void* wpack,
                              int32_t spin_limit, int32_t fault_flags,
                              void* stream);
 
+/*
+ * The whole per-op forward in one call: LayerNorm, then per layer QKV
+ * projection, attention, output projection, residual LayerNorm, FFN, residual
+ * LayerNorm, the last one final_norm in FP32 -- exactly the entry points above
+ * in the order of _forward_cuda_fused_norm (torch_transformer_benchmark.py:
+ * 1092-1148), each called with the variant given for it, so the results are
+ * theirs bit for bit.  x, y: [batch, seq_len, heads * head_dim] FP32 (y may not
+ * be x); the intermediates live in `workspace` (16-byte aligned, at least
+ * xb_stack_workspace_bytes, contents don't matter).
+ *   token_valid: [batch, seq_len] bytes or NULL, as key_valid of xb_attention
+ *     and the row mask of the final LayerNorm (XB_MASK_OUTPUT).
+ *   attention_variant: XB_ATTN_* (XB_ATTN_PINGPONG_VT: V handed over
+ *     transposed, xb_linear_qkv_vt) or XB_VARIANT_AUTO.
+ *   caches: NULL, or k_cache, v_cache of each layer in turn (2 * layers
+ *     pointers, xb_kv_cache_append's layout); the call then appends its tokens
+ *     at cache_start and attends over everything cached (cache_start 0: within
+ *     its own projection).  Needs causal, and token_valid NULL.
+ */
+typedef struct xb_block {
+  const void *qkv_w, *out_w, *ffn_in_w, *ffn_out_w;          /* FP16 [3D, D], [D, D], [F, D], [D, F] */
+  const float *qkv_b, *out_b, *ffn_in_b, *ffn_out_b;         /* FP32 */
+  const float *norm1_g, *norm1_b, *norm2_g, *norm2_b;        /* FP32 [D] */
+  float norm1_eps, norm2_eps, scale;                         /* scale: of the attention scores */
+  int32_t norm1_affine, norm2_affine;                        /* 0: gamma == 1 and beta == 0 */
+} xb_block;
+typedef struct xb_stack {
+  const xb_block* blocks;
+  const float *final_g, *final_b;
+  float final_eps;
+  int32_t final_affine, layers, heads, head_dim, ffn_dim, causal;
+} xb_stack;
+int64_t xb_stack_workspace_bytes(int32_t batch, int64_t seq_len, int32_t heads,
+                                 int32_t head_dim, int32_t ffn_dim,
+                                 int attention_variant, int64_t cache_start /* < 0: no cache */);
+int xb_stack_forward(const xb_stack* stack, const float* x, float* y,
+                     const uint8_t* token_valid, int32_t batch, int64_t seq_len,
+                     int qkv_variant, int out_variant, int ffn_in_variant,
+                     int ffn_out_variant, int attention_variant,
+                     void* const* caches, int64_t cache_start,
+                     int64_t cache_capacity, void* workspace,
+                     int64_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

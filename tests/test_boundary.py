@@ -309,3 +309,32 @@ def test_captured_overlap_is_described(pkg):
         assert pkg.UserOptimizedTransformer(c).captured_overlap(c.batch_size, c.seq_len) is None
     odd = pkg.UserOptimizedTransformer(pkg.TransformerConfig(7, 64, 1024, 4, 1024, 1, True))
     assert "4 sequences" in odd.captured_overlap(7, 64, padded=True) and "3 sequences" in odd.captured_overlap(7, 64)
+
+
+def test_stack_forward_argument_checks(capi):
+    """xb_stack_forward refuses bad sizes, missing pointers and a small workspace before any launch."""
+    import ctypes
+
+    lib = capi.lib()
+    need = lib.xb_stack_workspace_bytes(2, 8, 4, 16, 64, -1, -1)
+    rows, d = 16, 64
+    # residual (FP32), norm, update, then qkv with ctx, in whose place the FFN hidden state goes
+    assert need == rows * d * (4 + 2 + 2 + 6 + 2)
+    assert lib.xb_stack_workspace_bytes(2, 8, 4, 16, 4096, -1, -1) == rows * (d * 8 + 2 * 4096)
+    assert lib.xb_stack_workspace_bytes(2, 8, 4, 16, 64, -1, 100) == \
+        need + (lib.xb_attention_kv_cache_workspace_bytes(2, 8, 4, 16, 100) + 255) // 256 * 256
+    assert lib.xb_stack_workspace_bytes(2, 8, 0, 16, 64, -1, -1) == -2
+    blocks = (capi.XbBlock * 1)()
+    stack = capi.XbStack(blocks=blocks, layers=1, heads=4, head_dim=16, ffn_dim=64, causal=1)
+    ref = ctypes.addressof(stack)
+
+    def call(x=16, y=16, batch=2, ws=256, ws_bytes=need, valid=None, caches=None, start=0):
+        return lib.xb_stack_forward(ref, x, y, valid, batch, 8, -1, -1, -1, -1, -1, caches, start, 8, ws, ws_bytes, None)
+
+    assert call(batch=0) == 0
+    assert call(x=None) == -1 and call(y=None) == -1 and call(ws=None) == -1
+    assert call(ws_bytes=need - 1) == -7 and call(ws=8) == -5
+    assert call(batch=-1) == -2
+    assert call(valid=16, caches=16) == -2 and call(caches=16, start=-1) == -2
+    stack.layers = 0
+    assert call() == -2

@@ -772,3 +772,58 @@ def test_random_geometries_against_oracle(pkg, cuda, geom):
         out = optimized(x.to(cuda), mask.to(cuda)).cpu()
     plan = optimized.execution_plan(b, s, padded=padded)
     _check(ref, out, f"random geometry {geom} plan {plan.forward_strategy}")
+
+
+@pytest.mark.parametrize("geom,causal,padded", [
+    ((3, 70, 64, 4, 96, 3), True, False), ((3, 70, 64, 4, 96, 3), False, True), ((2, 129, 256, 8, 2048, 2), True, True),
+    ((2, 4128, 256, 4, 256, 1), True, False),      # V handed over transposed
+    ((1, 1, 512, 8, 512, 2), True, False)])
+def test_native_sequence_is_the_stepwise_one(pkg, cuda, geom, causal, padded):
+    """The native call issues the launches the wrappers issue one by one: the same
+    bits, with padding, without the causal mask, with an FFN wider and narrower
+    than the buffers it reuses, and after a parameter or an eps has changed."""
+    config = pkg.TransformerConfig(*geom, causal)
+    torch.manual_seed(sum(geom))
+    model = pkg.UserOptimizedTransformer(config).to(cuda).eval()
+    x = torch.randn(geom[0], geom[1], geom[2], generator=torch.Generator().manual_seed(5)).to(cuda)
+    valid = None
+    if padded:
+        valid = torch.ones(geom[0], geom[1], dtype=torch.uint8, device=cuda)
+        valid[0, geom[1] // 2:] = 0
+    plan = model.execution_plan(geom[0], geom[1], padded=padded)
+
+    def both():
+        with torch.no_grad():
+            out = model(x, valid)
+            assert torch.equal(out, model._per_op_forward_stepwise(x, plan, None, valid, None))
+        return out
+
+    first = both()
+    model.layers[0].norm2.eps = 0.25
+    second = both()
+    with torch.no_grad():
+        model.layers[0].ffn_out.weight.mul_(0.5)
+        model.final_norm.bias.add_(1.0)
+    third = both()
+    assert not torch.equal(first, second) and not torch.equal(second, third)
+
+
+@pytest.mark.parametrize("prompt,chunks", [(1, (1, 1)), (40, (1, 16, 17, 1)), (0, (5, 1))])
+def test_native_sequence_with_kv_cache(pkg, cuda, prompt, chunks):
+    """KV-cached steps: native and stepwise issue give the same outputs and caches."""
+    steps = [c for c in (prompt, *chunks) if c]
+    config = pkg.TransformerConfig(3, sum(steps) + 2, 256, 4, 512, 2, True)
+    torch.manual_seed(7)
+    models = [pkg.UserOptimizedTransformer(config).to(cuda).eval() for _ in range(2)]
+    models[1].load_state_dict(models[0].state_dict())
+    for m in models:
+        m.enable_kv_cache(True)
+    models[1]._native_stack = lambda: None
+    for i, c in enumerate(steps):
+        x = torch.randn(3, c, 256, generator=torch.Generator().manual_seed(i)).to(cuda)
+        with torch.no_grad():
+            assert torch.equal(models[0](x), models[1](x)), (i, c)
+    used = sum(steps)
+    for a, b in zip(models[0]._kv_cache.values(), models[1]._kv_cache.values()):
+        for s, t in zip(a, b):
+            assert torch.equal(s[:, :, :used], t[:, :, :used])
