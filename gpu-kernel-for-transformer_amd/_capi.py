@@ -87,6 +87,8 @@ EXPORTED_SYMBOLS = (
     "xb_fused_forward_d128",
     "xb_fused_forward_d128_workspace_bytes",
     "xb_fused_forward_d128_ws",
+    "xb_select_row_block",
+    "xb_row_block",
     "xb_stack_workspace_bytes",
     "xb_stack_forward",
 )
@@ -101,7 +103,7 @@ class XbBlock(ctypes.Structure):
     """xb_block of include/xblock.h."""
 
     _fields_ = ([(name, _vp) for name in (
-        "qkv_w", "out_w", "ffn_in_w", "ffn_out_w", "qkv_b", "out_b", "ffn_in_b", "ffn_out_b",
+        "qkv_w", "out_w", "ffn_in_w", "ffn_out_w", "packed", "qkv_b", "out_b", "ffn_in_b", "ffn_out_b",
         "norm1_g", "norm1_b", "norm2_g", "norm2_b")]
         + [(name, _f32) for name in ("norm1_eps", "norm2_eps", "scale")]
         + [(name, _i32) for name in ("norm1_affine", "norm2_affine")])
@@ -156,6 +158,8 @@ _SIGNATURES = {
         ctypes.c_int,
         [_vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _i64, _vp, _i32, _vp, _i64, _i32, _i32, _vp],
     ),
+    "xb_select_row_block": (ctypes.c_int, [_i32, _i32]),
+    "xb_row_block": (ctypes.c_int, [_vp, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp]),
     "xb_stack_workspace_bytes": (_i64, [_i32, _i64, _i32, _i32, _i32, ctypes.c_int, _i64]),
     "xb_stack_forward": (
         ctypes.c_int,

@@ -128,6 +128,7 @@ class ShapeExecutionPlan:
     ffn_in_variant: int = -1
     ffn_out_variant: int = -1
     attention_variant: int = -1
+    row_block: bool = False  # everything between two attentions in one kernel (xb_row_block)
 
     @property
     def fused(self) -> bool:
@@ -170,6 +171,7 @@ def resolve_shape_execution_plan(
     masked: bool = False,
     fused_allowed: bool = True,
     transposed_v_allowed: bool = True,
+    row_block_allowed: bool = True,
 ) -> ShapeExecutionPlan:
     """The gfx950 plan for a forward of [batch, seq_len] (default: the config's own shape).
 
@@ -178,7 +180,9 @@ def resolve_shape_execution_plan(
     conditions beyond the shape (the toggle, LayerNorm eps 1e-5 with affine
     parameters).  transposed_v_allowed: the ping-pong attention may take V
     transposed from the QKV GEMM (xb_linear_qkv_vt / xb_attention_causal_vt;
-    not for KV-cached steps, which attend through the cache).  The kernel choices are the library's (xb_select_*); only a
+    not for KV-cached steps, which attend through the cache).
+    row_block_allowed: narrow models may run everything between two attentions
+    as one kernel (xb_row_block).  The kernel choices are the library's (xb_select_*); only a
     batch whose working set exceeds CHUNK_BUDGET_FRACTION of HBM is chunked.
     Without the library the plan stays "unresolved" (the forward then raises).
     """
@@ -207,6 +211,18 @@ def resolve_shape_execution_plan(
             projection_strategy=f"{name}: MFMA GEMMs, weights staged in LDS",
         )
     rows = (chunk or b) * s
+    if row_block_allowed and lib.xb_select_row_block(d, f) == 0:
+        attn = lib.xb_select_attention(chunk or b, s, h, d // h, int(masked))
+        if attn >= 0:
+            return ShapeExecutionPlan(
+                official_shape_id=shape_id, batch=b, seq_len=s, masked=masked, batch_chunk_size=chunk,
+                forward_strategy="row_blocks (LayerNorm and QKV, then per layer attention and one kernel from its "
+                                 "output projection to the next QKV)",
+                ffn_strategy="row_block: MFMA GEMMs + erf GELU in registers",
+                attention_strategy=_variant_name(lib, _capi.XB_OP_ATTENTION, attn),
+                projection_strategy="row_block: MFMA GEMMs, weights staged in LDS",
+                attention_variant=attn, row_block=True,
+            )
     qkv = lib.xb_select_linear(rows, 3 * d, d, _capi.XB_EPI_BIAS)
     out = lib.xb_select_linear(rows, d, d, _capi.XB_EPI_BIAS)
     ffn_in = lib.xb_select_linear(rows, f, d, _capi.XB_EPI_BIAS_GELU)

@@ -438,17 +438,6 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_kernel(const AttnArgs a)
   }
 }
 
-// dma16 issued from inline assembly: the compiler does not see this LDS
-// write, so it adds no wait for it before later LDS reads (it cannot tell the
-// ring buffer being filled from the one being read, and would wait before
-// every read).  The caller waits itself (vmcnt) before the barrier that
-// publishes the tile.  Any wait the compiler does emit for its own loads only
-// waits longer, since it counts fewer operations in flight than there are.
-__device__ __forceinline__ void dma16_untracked(const void* src_lane, void* lds_wave_base) {
-  const uint32_t lds = (uint32_t)(uintptr_t)(lds_void_t*)lds_wave_base;
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src_lane), "s"(lds) : "memory", "m0");
-}
-
 // Ping-pong variant for long sequences (head_dim 64, no key mask): 8 waves in
 // two groups of four, A = waves 0-3 and B = waves 4-7, one wave of each per
 // SIMD.  Per 64-key tile a wave runs an MFMA phase (PV of the previous tile,

@@ -99,4 +99,15 @@ __device__ __forceinline__ void dma16(const void* src_lane, void* lds_wave_base)
   __builtin_amdgcn_global_load_lds((global_void_t*)src_lane, (lds_void_t*)lds_wave_base, 16, 0, 0);
 }
 
+// dma16 issued from inline assembly: the compiler does not see this LDS
+// write, so it adds no wait for it before later LDS reads (it cannot tell the
+// ring buffer being filled from the one being read, and would wait before
+// every read).  The caller waits itself (vmcnt) before the barrier that
+// publishes the tile.  Any wait the compiler does emit for its own loads only
+// waits longer, since it counts fewer operations in flight than there are.
+__device__ __forceinline__ void dma16_untracked(const void* src_lane, void* lds_wave_base) {
+  const uint32_t lds = (uint32_t)(uintptr_t)(lds_void_t*)lds_wave_base;
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src_lane), "s"(lds) : "memory", "m0");
+}
+
 }  // namespace xb

@@ -93,6 +93,34 @@ extern "C" int xb_stack_forward(const xb_stack* st, const float* x, float* y, co
   const bool transposed_v = !cached && attention_variant == XB_ATTN_PINGPONG_VT;
 
   const xb_block* b = st->blocks;
+  bool row_blocks = true;
+  for (int i = 0; i < st->layers; ++i) row_blocks = row_blocks && b[i].packed != nullptr;
+  // Append and attend: layer i's context from qkv.
+  auto attend = [&](int i) -> int {
+    const float scale = st->blocks[i].scale;
+    if (cached) {
+      const int bad = xb_kv_cache_append(qkv, caches[2 * i], caches[2 * i + 1], batch, seq_len, heads, hd, cache_start,
+                                         cache_capacity, stream);
+      if (bad) return bad;
+      if (cache_start > 0)
+        return xb_attention_kv_cache(qkv, caches[2 * i], caches[2 * i + 1], ctx, batch, seq_len, heads, hd,
+                                     cache_start, cache_capacity, scale, decode, l.bytes - l.decode, stream);
+    }
+    return xb_attention_v(qkv, ctx, token_valid, batch, seq_len, heads, hd, scale, st->causal, attention_variant, stream);
+  };
+  if (row_blocks) {
+    // The residual stream alternates between its buffer and the place of
+    // norm and update, which this path does not use.
+    float* streams[2] = {residual, static_cast<float*>(norm)};
+    const float* in = x;
+    e = xb_row_block(st, -1, x, nullptr, nullptr, qkv, nullptr, nullptr, rows, stream);
+    for (int i = 0; i < st->layers && !e; ++i) {
+      e = attend(i);
+      if (!e) e = xb_row_block(st, i, in, ctx, streams[i & 1], qkv, y, token_valid, rows, stream);
+      in = streams[i & 1];
+    }
+    return e;
+  }
   e = xb_layernorm(x, b->norm1_g, b->norm1_b, norm, XB_F16, rows, d, b->norm1_eps, b->norm1_affine, stream);
   const float* res_in = x;
   for (int i = 0; i < st->layers && !e; ++i, ++b) {
@@ -101,17 +129,7 @@ extern "C" int xb_stack_forward(const xb_stack* st, const float* x, float* y, co
       if (!e) e = xb_attention_causal_vt(qkv, vt, ctx, batch, seq_len, heads, hd, b->scale, stream);
     } else {
       e = xb_linear_v(norm, b->qkv_w, b->qkv_b, qkv, rows, 3 * d, d, XB_EPI_BIAS, qkv_variant, stream);
-      if (!e && cached)
-        e = xb_kv_cache_append(qkv, caches[2 * i], caches[2 * i + 1], batch, seq_len, heads, hd, cache_start,
-                               cache_capacity, stream);
-      if (!e) {
-        if (cached && cache_start > 0)
-          e = xb_attention_kv_cache(qkv, caches[2 * i], caches[2 * i + 1], ctx, batch, seq_len, heads, hd, cache_start,
-                                    cache_capacity, b->scale, decode, l.bytes - l.decode, stream);
-        else
-          e = xb_attention_v(qkv, ctx, token_valid, batch, seq_len, heads, hd, b->scale, st->causal,
-                             attention_variant, stream);
-      }
+      if (!e) e = attend(i);
     }
     if (!e) e = xb_linear_v(ctx, b->out_w, b->out_b, update, rows, d, d, XB_EPI_BIAS, out_variant, stream);
     if (!e)

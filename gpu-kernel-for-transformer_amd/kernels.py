@@ -560,18 +560,53 @@ def stack_forward(
     return out
 
 
-def pack_linear_fragments(weight: torch.Tensor, natural: bool = False, scale: float = 1.0) -> torch.Tensor:
-    """FP16 fragment-major copy of `scale * weight` (nn.Linear [n, k]) for the fused kernel.
+def row_block(
+    stack: _capi.XbStack,
+    layer: int,
+    residual: torch.Tensor,
+    ctx: Optional[torch.Tensor] = None,
+    residual_out: Optional[torch.Tensor] = None,
+    qkv: Optional[torch.Tensor] = None,
+    out: Optional[torch.Tensor] = None,
+    row_valid: Optional[torch.Tensor] = None,
+) -> None:
+    """One xb_row_block launch: layer -1 starts a narrow model's forward (LayerNorm 1 and QKV of layer
+    0), layer i runs from its attention context to layer i + 1's QKV, or to the final LayerNorm in `out`."""
+    _require_device(residual, "row_block")
+    d = stack.heads * stack.head_dim
+    rows = residual.numel() // d
+    lead = tuple(residual.shape[:-1])
+    for t, shape, dtype, what in ((residual, residual.shape, torch.float32, "residual"), (ctx, (*lead, d), torch.float16, "ctx"),
+                                  (residual_out, residual.shape, torch.float32, "residual_out"),
+                                  (qkv, (*lead, 3 * d), torch.float16, "qkv"), (out, residual.shape, torch.float32, "out")):
+        if t is not None:
+            _check_buffer(t, shape, dtype, residual.device, what)
+    valid = None if row_valid is None else _byte_mask(row_valid, rows, residual.device, "row_valid")
+    check(
+        _launch(f"row_block_{d}", lambda: lib().xb_row_block(
+            ctypes.addressof(stack), layer, residual.data_ptr(), _ptr(ctx), _ptr(residual_out), _ptr(qkv), _ptr(out),
+            _ptr(valid), rows, stream_handle(residual.device))),
+        "xb_row_block",
+    )
+
+
+def pack_linear_fragments(weight: torch.Tensor, natural: bool = False, scale: float = 1.0,
+                          out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """FP16 fragment-major copy of `scale * weight` (nn.Linear [n, k]) for the fused kernels.
 
     natural=False gives the permuted k order used against register-resident
     activations, natural=True the plain order used against LDS-resident ones.
+    `out`: n * k contiguous float16 entries to write (allocated when not given).
     """
     _require_device(weight, "pack_linear_fragments")
     if weight.ndim != 2:
         raise ValueError("weight must be 2-D")
     w = weight.detach().float().contiguous()
     n, k = w.shape
-    out = torch.empty(n * k, device=w.device, dtype=torch.float16)
+    if out is None:
+        out = torch.empty(n * k, device=w.device, dtype=torch.float16)
+    else:
+        _check_buffer(out, (n * k,), torch.float16, w.device, "out")
     check(
         _launch("pack_fragments", lambda: lib().xb_pack_linear_fragments(
             w.data_ptr(), out.data_ptr(), n, k, _capi.XB_PACK_NATURAL if natural else _capi.XB_PACK_PERMUTED,

@@ -135,6 +135,25 @@ class _LayerWeights:
             self.ffn_out_b = layer.ffn_out.bias.float().contiguous()
 
 
+class _RowBlockWeights:
+    """One block's weights fragment-packed for xb_row_block, and its FP32 biases."""
+
+    __slots__ = ("packed", "qkv_b", "out_b", "ffn_in_b", "ffn_out_b")
+
+    def __init__(self, layer: TransformerBlockParameters) -> None:
+        att = layer.attention
+        linears = (att.q_proj, att.k_proj, att.v_proj, att.out_proj, layer.ffn_in, layer.ffn_out)
+        with torch.no_grad():
+            sizes = [lin.weight.numel() for lin in linears]
+            self.packed = torch.empty(sum(sizes), device=att.q_proj.weight.device, dtype=torch.float16)
+            for lin, part in zip(linears, self.packed.split(sizes)):
+                kernels.pack_linear_fragments(lin.weight, out=part)
+            self.qkv_b = torch.cat((att.q_proj.bias, att.k_proj.bias, att.v_proj.bias), 0).float().contiguous()
+            self.out_b = att.out_proj.bias.float().contiguous()
+            self.ffn_in_b = layer.ffn_in.bias.float().contiguous()
+            self.ffn_out_b = layer.ffn_out.bias.float().contiguous()
+
+
 class UserOptimizedTransformer(nn.Module):
     """Drop-in for the reference's UserOptimizedTransformer (TTB:320-1148), HIP-only."""
 
@@ -179,12 +198,13 @@ class UserOptimizedTransformer(nn.Module):
         eligibility (the enable_fused_stack toggle, LayerNorm eps and affine);
         per_op=True asks for the per-op sequence (KV-cached steps).
         """
-        key = (int(batch), int(seq_len), bool(padded), self._fused_stack_eligible() and not per_op, bool(per_op))
+        key = (int(batch), int(seq_len), bool(padded), self._fused_stack_eligible() and not per_op, bool(per_op),
+               self._fused_stack_enabled)
         plans = self.__dict__.setdefault("_plans", {})
         plan = plans.get(key)
         if plan is None:
             plan = resolve_shape_execution_plan(self.config, batch, seq_len, masked=padded, fused_allowed=key[3],
-                                                transposed_v_allowed=not per_op)
+                                                transposed_v_allowed=not per_op, row_block_allowed=key[5])
             plans[key] = plan
         return plan
 
@@ -226,9 +246,9 @@ class UserOptimizedTransformer(nn.Module):
         self._attention_fp16_accumulation_enabled = bool(enabled)
 
     def enable_fused_stack(self, enabled: bool = True) -> None:
-        """Use the one-kernel whole-stack forward where its shape contract holds.
+        """Use the one-kernel whole-stack forward where its shape contract holds, and row blocks for narrow models.
 
-        With it disabled every shape runs the per-op kernel sequence; the two
+        With it disabled every shape runs the per-op kernel sequence; the
         paths compute the same math (FP16 operands, FP32 accumulation).
         """
         self._fused_stack_enabled = bool(enabled)
@@ -279,8 +299,11 @@ class UserOptimizedTransformer(nn.Module):
             cache[index] = cached
         return cached[1]
 
-    def _native_stack(self) -> Optional[Tuple[_capi.XbStack, object, object]]:
+    def _native_stack(self, row_block: bool) -> Optional[Tuple[_capi.XbStack, object, object]]:
         """(xb_stack, its xb_block array, the tensors they point into), cached by parameter version.
+
+        row_block: with fragment-packed weights for xb_row_block instead of
+        the FP16 copies the GEMMs read.
 
         None when a LayerNorm has no weight or bias: the wrappers then raise
         for it.  The descriptors are written once and only read afterwards, so
@@ -292,7 +315,7 @@ class UserOptimizedTransformer(nn.Module):
             registered = norm._parameters
             if registered.get("weight") is None or registered.get("bias") is None:
                 return None
-        settings = ([n.eps for n in norms], [a.scale for a in attentions])
+        settings = (row_block, [n.eps for n in norms], [a.scale for a in attentions])
         try:
             key = (tuple(map(_VERSION_OF, params)), tuple(map(torch.Tensor.data_ptr, params)), settings)
         except RuntimeError:  # inference-mode parameters have no version counter: never reuse
@@ -302,9 +325,10 @@ class UserOptimizedTransformer(nn.Module):
             return cached[1]
         cfg = self.config
         blocks = (_capi.XbBlock * len(self.layers))()
-        weights = [self._layer_weights(i) for i in range(len(self.layers))]
+        weights = [_RowBlockWeights(layer) if row_block else self._layer_weights(i)
+                   for i, layer in enumerate(self.layers)]
         for block, layer, w in zip(blocks, self.layers, weights):
-            for name in _LayerWeights.__slots__:
+            for name in w.__slots__:
                 setattr(block, name, getattr(w, name).data_ptr())
             for which, norm in (("norm1", layer.norm1), ("norm2", layer.norm2)):
                 setattr(block, which + "_g", norm.weight.data_ptr())
@@ -633,7 +657,7 @@ class UserOptimizedTransformer(nn.Module):
         While a LaunchRecorder is active the same launches go through the
         wrappers one by one, so that each is bracketed by its events.
         """
-        native = None if kernels.recording() else self._native_stack()
+        native = None if kernels.recording() else self._native_stack(plan.row_block)
         if native is None:
             return self._per_op_forward_stepwise(x, plan, out, token_valid, cache_start)
         if out is None:
@@ -660,6 +684,9 @@ class UserOptimizedTransformer(nn.Module):
     def _per_op_forward_stepwise(self, x: torch.Tensor, plan: ShapeExecutionPlan, out: Optional[torch.Tensor],
                                  token_valid: Optional[torch.Tensor], cache_start: Optional[int]) -> torch.Tensor:
         """_per_op_forward, one wrapper call per launch."""
+        native = self._native_stack(True) if plan.row_block else None
+        if native is not None:
+            return self._row_block_forward_stepwise(x, native[0], plan, out, token_valid, cache_start)
         cfg = self.config
         batch, seq_len, d_model = x.shape
         dev = x.device
@@ -705,6 +732,23 @@ class UserOptimizedTransformer(nn.Module):
                 mask_mode=_capi.XB_MASK_OUTPUT if last and token_valid is not None else 0,
             )
         return norm
+
+    def _row_block_forward_stepwise(self, x: torch.Tensor, stack: _capi.XbStack, plan: ShapeExecutionPlan,
+                                    out: Optional[torch.Tensor], token_valid: Optional[torch.Tensor],
+                                    cache_start: Optional[int]) -> torch.Tensor:
+        if out is None:
+            out = torch.empty_like(x)
+        qkv = torch.empty((*x.shape[:2], 3 * x.shape[2]), device=x.device, dtype=torch.float16)
+        kernels.row_block(stack, -1, x, qkv=qkv)
+        residual = x
+        for index in range(len(self.layers)):
+            context = self._attend_stepwise(index, qkv, plan, token_valid, cache_start)
+            last = index == len(self.layers) - 1
+            updated = None if last else torch.empty_like(x)
+            kernels.row_block(stack, index, residual, ctx=context, residual_out=updated, qkv=None if last else qkv,
+                              out=out if last else None, row_valid=token_valid if last else None)
+            residual = updated
+        return out
 
 
 def forward_flops(config: TransformerConfig, batch: Optional[int] = None, seq_len: Optional[int] = None) -> float:

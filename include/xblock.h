@@ -385,7 +385,9 @@ int xb_fused_forward_d128_ws(const float* x, float* y, const void* wpack,
  * LayerNorm, the last one final_norm in FP32 -- exactly the entry points above
  * in the order of _forward_cuda_fused_norm (torch_transformer_benchmark.py:
  * 1092-1148), each called with the variant given for it, so the results are
- * theirs bit for bit.  x, y: [batch, seq_len, heads * head_dim] FP32 (y may not
+ * theirs bit for bit.  If every block has `packed` weights, the attention is
+ * launched as above and everything between two attentions by xb_row_block (the
+ * other FP16 weights may then be NULL, and the linear variants are not used).  x, y: [batch, seq_len, heads * head_dim] FP32 (y may not
  * be x); the intermediates live in `workspace` (16-byte aligned, at least
  * xb_stack_workspace_bytes, contents don't matter).
  *   token_valid: [batch, seq_len] bytes or NULL, as key_valid of xb_attention
@@ -399,6 +401,8 @@ int xb_fused_forward_d128_ws(const float* x, float* y, const void* wpack,
  */
 typedef struct xb_block {
   const void *qkv_w, *out_w, *ffn_in_w, *ffn_out_w;          /* FP16 [3D, D], [D, D], [F, D], [D, F] */
+  const void* packed;        /* xb_row_block: Wq Wk Wv Wo W1 W2 fragment-packed (XB_PACK_PERMUTED, scale 1),
+                                back to back, or NULL */
   const float *qkv_b, *out_b, *ffn_in_b, *ffn_out_b;         /* FP32 */
   const float *norm1_g, *norm1_b, *norm2_g, *norm2_b;        /* FP32 [D] */
   float norm1_eps, norm2_eps, scale;                         /* scale: of the attention scores */
@@ -410,6 +414,25 @@ typedef struct xb_stack {
   float final_eps;
   int32_t final_affine, layers, heads, head_dim, ffn_dim, causal;
 } xb_stack;
+
+/*
+ * Everything between two attentions of a narrow model in one kernel
+ * (xb_select_row_block: XB_OK for d_model 32, 64 or 128 with ffn_dim a multiple
+ * of it, up to 4 times, at 128 up to 8 times).  layer -1: qkv = the packed QKV
+ * projection of layer 0's LayerNorm 1 of `residual` (= the input).  layer i:
+ * from its attention context ctx [rows, D] FP16, output projection, residual
+ * add, LayerNorm 2, FFN, residual add; then, before the last layer, the new
+ * residual stream goes to residual_out (not `residual`) and layer i + 1's QKV
+ * projection to qkv; after the last one the final LayerNorm goes to y (rows
+ * whose row_valid byte is 0 as zeros; row_valid may be NULL).  Same math as
+ * the entry points it stands for, with FP16 operands, FP32 sums and residual
+ * stream, and no FP16 rounding of the residual updates.
+ */
+int xb_select_row_block(int32_t d_model, int32_t ffn_dim);
+int xb_row_block(const xb_stack* stack, int32_t layer, const float* residual,
+                 const void* ctx, float* residual_out, void* qkv, float* y,
+                 const uint8_t* row_valid, int64_t rows, void* stream);
+
 int64_t xb_stack_workspace_bytes(int32_t batch, int64_t seq_len, int32_t heads,
                                  int32_t head_dim, int32_t ffn_dim,
                                  int attention_variant, int64_t cache_start /* < 0: no cache */);

@@ -775,7 +775,9 @@ def test_random_geometries_against_oracle(pkg, cuda, geom):
 
 
 @pytest.mark.parametrize("geom,causal,padded", [
-    ((3, 70, 64, 4, 96, 3), True, False), ((3, 70, 64, 4, 96, 3), False, True), ((2, 129, 256, 8, 2048, 2), True, True),
+    ((3, 70, 64, 4, 96, 3), True, False), ((3, 70, 64, 4, 96, 3), False, True),
+    ((3, 70, 64, 4, 128, 3), False, True), ((2, 200, 128, 4, 256, 2), True, True),   # row blocks
+    ((2, 129, 256, 8, 2048, 2), True, True),
     ((2, 4128, 256, 4, 256, 1), True, False),      # V handed over transposed
     ((1, 1, 512, 8, 512, 2), True, False)])
 def test_native_sequence_is_the_stepwise_one(pkg, cuda, geom, causal, padded):
@@ -818,7 +820,7 @@ def test_native_sequence_with_kv_cache(pkg, cuda, prompt, chunks):
     models[1].load_state_dict(models[0].state_dict())
     for m in models:
         m.enable_kv_cache(True)
-    models[1]._native_stack = lambda: None
+    models[1]._native_stack = lambda row_block: None
     for i, c in enumerate(steps):
         x = torch.randn(3, c, 256, generator=torch.Generator().manual_seed(i)).to(cuda)
         with torch.no_grad():
@@ -827,3 +829,46 @@ def test_native_sequence_with_kv_cache(pkg, cuda, prompt, chunks):
     for a, b in zip(models[0]._kv_cache.values(), models[1]._kv_cache.values()):
         for s, t in zip(a, b):
             assert torch.equal(s[:, :, :used], t[:, :, :used])
+
+
+@pytest.mark.parametrize("geom", [
+    (1, 1, 32, 4, 32, 1), (3, 21, 32, 4, 128, 2), (64, 128, 32, 4, 32, 4), (2, 65, 64, 4, 64, 3), (5, 100, 64, 1, 256, 2),
+    (1, 130, 128, 4, 128, 2), (2, 300, 128, 1, 1024, 2), (130, 127, 128, 16, 128, 2),     # 1-block waves of eight
+    (257, 129, 128, 4, 128, 2), (1100, 31, 64, 8, 128, 1)])                               # two blocks per wave
+@pytest.mark.parametrize("causal,padded", [(True, False), (True, True), (False, False)])
+def test_row_blocks(pkg, cuda, geom, causal, padded):
+    """Narrow models' row-block path at every width, FFN multiple and tile, with ragged
+    last blocks: against the oracle, close to the per-op kernels (which differ by the FP16 rounding
+    of the residual updates), and each sequence's rows independent of the batch."""
+    b, s, d = geom[:3]
+    config = pkg.TransformerConfig(*geom, causal)
+    torch.manual_seed(sum(geom))
+    baseline = BaselineTransformer(config).eval()
+    model = pkg.UserOptimizedTransformer(config)
+    copy_model_weights(baseline, model)
+    with torch.no_grad():
+        for i, (a, c) in enumerate(zip(baseline.parameters(), model.parameters())):
+            if a.ndim == 1:   # LayerNorm affine and biases that matter
+                a.add_(0.1 * torch.randn(a.shape, generator=torch.Generator().manual_seed(i)))
+                c.copy_(a)
+    model = model.to(cuda).eval()
+    assert model.execution_plan(b, s, padded=padded, per_op=True).row_block
+    x = torch.randn(b, s, d, generator=torch.Generator().manual_seed(1))
+    mask = torch.ones(b, s, dtype=torch.bool)
+    if padded:
+        mask[0, (s + 1) // 2:] = False
+    plan = model.execution_plan(b, s, padded=padded and s > 1, per_op=True)
+    valid = mask.to(torch.uint8).to(cuda) if not bool(mask.all()) else None
+    xg = x.to(cuda)
+    with torch.no_grad():
+        out = model._per_op_forward(xg, plan, token_valid=valid)
+        few = min(b, 4)
+        ref = baseline(x[:few], mask[:few])
+        result = compare_outputs(ref, out[:few].cpu())
+        assert result.passed, result.summary()
+        model.enable_fused_stack(False)
+        per_op = model._per_op_forward(xg, model.execution_plan(b, s, padded=valid is not None), token_valid=valid)
+        model.enable_fused_stack(True)
+        assert float((out - per_op).abs().max()) < 2e-2 and float((out - per_op).norm() / per_op.norm()) < 1e-3
+        alone = model._per_op_forward(xg[:1].contiguous(), plan, token_valid=None if valid is None else valid[:1].contiguous())
+        assert torch.equal(alone, out[:1])
