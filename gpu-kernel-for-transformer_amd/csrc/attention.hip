@@ -9,7 +9,7 @@
 // is the [B, S, D] row layout the output projection consumes (this removes
 // the reference's transpose + reshape copy, torch_transformer_benchmark.py:809).
 //
-// Work decomposition: one 256-thread block = 4 waves handles BQ = 64*NQ
+// Work decomposition: one 256-thread block = 4 waves handles BQ = 64*NQ (NQ = 1, 2 or 4)
 // consecutive queries of one head; wave w owns queries [16*NQ*w, 16*NQ*(w+1)).
 // K and V tiles of BKEYS keys are double buffered in LDS, both row-major: the
 // next tile's global loads are in flight while the current tile is consumed,
@@ -32,7 +32,8 @@
 // of the MFMA as one extra O^T block whose V^T rows are all ones, and m_run is
 // only moved (and O rescaled) on the first tile and when a tile's maximum
 // exceeds it by more than 8 (probabilities then stay <= 2^8, exact enough in
-// FP16); the decision is wave-uniform.  Only tiles that straddle the diagonal
+// FP16); the decision is made per block of 16 queries, so a query's result is
+// the same bit for bit whichever variant's wave holds it.  Only tiles that straddle the diagonal
 // pay for the mask.
 #include <algorithm>
 #include <atomic>
@@ -114,16 +115,22 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_kernel(const AttnArgs a)
   // One-wave split blocks keep a single LDS tile (the next one waits in
   // registers), so more of them fit on a CU.
   constexpr int NBUF = SPLIT ? 1 : 2;
+  constexpr int AHEAD = SPLIT || HD >= 256 || NQ > 2 ? 1 : 2;
   static_assert(NT >= BKEYS, "one thread per key stages the validity bytes");
 
   __shared__ __attribute__((aligned(16))) half_t k_lds[NBUF][BKEYS * LDK];
   __shared__ __attribute__((aligned(16))) half_t v_lds[NBUF][BKEYS * LDV];
   __shared__ __attribute__((aligned(16))) uint8_t kv_lds[NBUF][BKEYS];  // key validity of the tile
 
-  // Heaviest query tiles (most keys under the causal mask) are issued first.
+  // Heaviest query tiles (most keys under the causal mask) are issued first;
+  // the tiles of one (batch, head) run on one XCD, whose L2 then holds that
+  // head's K and V for all of them (dealt round-robin, every L2 streamed every
+  // head's: B = 1, S = 8000, 16 heads of 64 246 -> 174 us, B = 8, S = 2048
+  // padded 173 -> 136 us; ping-pong kernel at S = 32768 2928 -> 2025 us).
   const int per_bh = SPLIT ? a.n_splits : a.q_tiles;
-  const int bh = blockIdx.x / per_bh;
-  const int sub = blockIdx.x % per_bh;
+  const int block = xcd_contiguous_tile(blockIdx.x, gridDim.x);
+  const int bh = block / per_bh;
+  const int sub = block % per_bh;
   const int qt = SPLIT ? 0 : (CAUSAL ? a.q_tiles - 1 - sub : sub);
   const int b = bh / a.H, h = bh % a.H;
   const int S_q = a.S_q, S_k = a.S_k, q_offset = a.q_offset;
@@ -188,59 +195,69 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_kernel(const AttnArgs a)
   }
   const half8_t ones8 = {1, 1, 1, 1, 1, 1, 1, 1};
 
+  const int k_begin = SPLIT ? sub * a.split_keys : 0;
+  int key_end = CAUSAL ? min(S_k, q_offset + q0 + BQ) : S_k;
+  if constexpr (SPLIT) key_end = min(key_end, k_begin + a.split_keys);
+  const int n_tiles = key_end > k_begin ? (key_end - k_begin + BKEYS - 1) / BKEYS : 0;
+
+  // Tile loads, unconditional: rows from key_end on repeat row key_end - 1
+  // (their scores are masked, and that row is in the last tile anyway), also
+  // when the whole tile lies past the end.  A load under any condition would
+  // make the compiler wait for every load in flight, the tile after next
+  // included, where it should wait for the next tile's only (B = 1, S = 1500,
+  // 12 heads of 64: 22.4 -> 20.1 us; B = 8, S = 2048, 16 heads, padded: 136 ->
+  // 124 us).
   // Key validity travels with the tile (0 past S as well).
   const uint8_t* kvb = KEYMASK ? a.key_valid + (int64_t)b * S_k : nullptr;
-  uint8_t kvreg = 0;
-  half8_t kreg[CH], vreg[CH];
-  auto gload = [&](int k0) {
-    if (KEYMASK && tid < BKEYS) {
-      const int key = k0 + tid;
-      kvreg = key < S_k ? kvb[key] : (uint8_t)0;
+  uint8_t kvreg[AHEAD] = {};
+  half8_t kreg[AHEAD][CH], vreg[AHEAD][CH];
+  auto gload = [&](int t, auto set) {
+    constexpr int R = decltype(set)::value;
+    const int k0 = k_begin + t * BKEYS;
+    const int key_last = max(key_end - 1, 0);
+    if constexpr (KEYMASK) {
+      const int key = k0 + tid % BKEYS;
+      const uint8_t v = kvb[min(key, key_last)];
+      kvreg[R] = key < key_end ? v : (uint8_t)0;
     }
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
-      const int id = tid + NT * j;
-      kreg[j] = zero8;
-      vreg[j] = zero8;
-      if (id < BKEYS * CPK) {
-        const int key = k0 + id / CPK, c = (id % CPK) * 8;
-        if (key < S_k) {
-          const half8_t* kp = reinterpret_cast<const half8_t*>(kbase + key * k_rstride + c);
-          const half8_t* vp = reinterpret_cast<const half8_t*>(vbase + key * k_rstride + c);
-          if constexpr (SPLIT) {
-            // Decode streams each cached row exactly once: non-temporal loads
-            // keep it from displacing reusable lines (87% vs 77% of HBM peak
-            // on a 100k-token cache).
-            kreg[j] = __builtin_nontemporal_load(kp);
-            vreg[j] = __builtin_nontemporal_load(vp);
-          } else {
-            kreg[j] = *kp;
-            vreg[j] = *vp;
-          }
-        }
+      const int id = min(tid + NT * j, BKEYS * CPK - 1);
+      const int key = min(k0 + id / CPK, key_last), c = (id % CPK) * 8;
+      const half8_t* kp = reinterpret_cast<const half8_t*>(kbase + key * k_rstride + c);
+      const half8_t* vp = reinterpret_cast<const half8_t*>(vbase + key * k_rstride + c);
+      if constexpr (SPLIT) {
+        // Decode streams each cached row exactly once: non-temporal loads
+        // keep it from displacing reusable lines (87% vs 77% of HBM peak
+        // on a 100k-token cache).
+        kreg[R][j] = __builtin_nontemporal_load(kp);
+        vreg[R][j] = __builtin_nontemporal_load(vp);
+      } else {
+        kreg[R][j] = *kp;
+        vreg[R][j] = *vp;
       }
     }
   };
-  auto sstore = [&](int buf) {
-    if (KEYMASK && tid < BKEYS) kv_lds[buf][tid] = kvreg;
+  auto sstore = [&](int buf, auto set) {
+    constexpr int R = decltype(set)::value;
+    if (KEYMASK && tid < BKEYS) kv_lds[buf][tid] = kvreg[R];
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
       const int id = tid + NT * j;
       if (id < BKEYS * CPK) {
         const int r = id / CPK, c = (id % CPK) * 8;
-        *reinterpret_cast<half8_t*>(&k_lds[buf][r * LDK + c]) = kreg[j];
-        *reinterpret_cast<half8_t*>(&v_lds[buf][r * LDV + c]) = vreg[j];
+        *reinterpret_cast<half8_t*>(&k_lds[buf][r * LDK + c]) = kreg[R][j];
+        *reinterpret_cast<half8_t*>(&v_lds[buf][r * LDV + c]) = vreg[R][j];
       }
     }
   };
 
-  const int k_begin = SPLIT ? sub * a.split_keys : 0;
-  int key_end = CAUSAL ? min(S_k, q_offset + q0 + BQ) : S_k;
-  if constexpr (SPLIT) key_end = min(key_end, k_begin + a.split_keys);
-  const int n_tiles = key_end > k_begin ? (key_end - k_begin + BKEYS - 1) / BKEYS : 0;
+  constexpr std::integral_constant<int, 0> kSet0{};
+  constexpr std::integral_constant<int, AHEAD - 1> kSet1{};
   if (n_tiles > 0) {
-    gload(k_begin);
-    sstore(0);
+    gload(0, kSet0);
+    if constexpr (AHEAD == 2) gload(1, kSet1);
+    sstore(0, kSet0);
   }
 #pragma unroll
   for (int qb = 0; qb < NQ; ++qb)
@@ -252,10 +269,11 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_kernel(const AttnArgs a)
       qf[qb][ks] = q_ok(qb, ks) ? v : zero8;
     }
   __syncthreads();
-  for (int t = 0; t < n_tiles; ++t) {
+  // Tile t; register set `free` held it and takes tile t + AHEAD, set `next` holds tile t + 1 by its end.
+  auto step = [&](int t, auto free, auto next) {
     const int cur = NBUF == 1 ? 0 : t & 1;
     const int k0 = k_begin + t * BKEYS;
-    if (t + 1 < n_tiles) gload(k0 + BKEYS);
+    gload(t + AHEAD, free);
 
     // Wave-uniform skip: every key of this tile lies above this wave's diagonal.
     if (!CAUSAL || k0 <= q_offset + qw0 + QPW - 1) {
@@ -332,6 +350,9 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_kernel(const AttnArgs a)
 #pragma unroll
           for (int jb = 0; jb < KB; ++jb)
             m = fmaxf(m, fmaxf(fmaxf(s[jb][qb][0], s[jb][qb][1]), fmaxf(s[jb][qb][2], s[jb][qb][3])));
+          // Decided per block of 16 queries, not per wave: a query's result then
+          // does not depend on how many blocks its wave holds.
+          if (!__any((TRACK ? !m_set[qb] : t == 0) || m > 8.0f)) continue;
           const float mx = quad_group_max(m);
           // Until a query has seen a key its o and lacc are exactly zero: the
           // offset jumps to the first finite maximum and nothing is rescaled
@@ -377,8 +398,16 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_kernel(const AttnArgs a)
 
     __builtin_amdgcn_s_setprio(0);
     if constexpr (NBUF == 1) __syncthreads();  // the tile is read completely before it is replaced
-    if (t + 1 < n_tiles) sstore(NBUF == 1 ? 0 : cur ^ 1);
+    sstore(NBUF == 1 ? 0 : cur ^ 1, next);
     __syncthreads();
+  };
+  if constexpr (AHEAD == 2) {
+    for (int t = 0; t < n_tiles; t += 2) {
+      step(t, kSet0, kSet1);
+      if (t + 1 < n_tiles) step(t + 1, kSet1, kSet0);
+    }
+  } else {
+    for (int t = 0; t < n_tiles; ++t) step(t, kSet0, kSet0);
   }
 
   if constexpr (SPLIT) {
@@ -477,8 +506,9 @@ __global__ __launch_bounds__(512, 1) void attn_pp_kernel(const AttnArgs a) {
   __shared__ __attribute__((aligned(16))) half8_t q_lds[NW][NQ][KSTEPS][kWave];
 
   const int per_bh = a.q_tiles;
-  const int bh = blockIdx.x / per_bh;
-  const int sub = blockIdx.x % per_bh;
+  const int block = xcd_contiguous_tile(blockIdx.x, gridDim.x);
+  const int bh = block / per_bh;
+  const int sub = block % per_bh;
   const int qt = CAUSAL ? a.q_tiles - 1 - sub : sub;  // heaviest query tiles first
   const int b = bh / a.H, h = bh % a.H;
   const int S_q = a.S_q, S_k = a.S_k, q_offset = a.q_offset;
@@ -700,6 +730,7 @@ __global__ __launch_bounds__(512, 1) void attn_pp_kernel(const AttnArgs a) {
 #pragma unroll
         for (int jb = 0; jb < KB; ++jb)
           m = fmaxf(m, fmaxf(fmaxf(s[jb][qb][0], s[jb][qb][1]), fmaxf(s[jb][qb][2], s[jb][qb][3])));
+        if (!__any(t == 0 || m > 8.0f)) continue;  // per block of 16 queries, as attn_kernel
         const float mx = quad_group_max(m);
         // Tile 0 shows every query key 0, so its maximum is finite: the offset
         // jumps there with nothing to rescale; later sh >= 0 and corr <= 1.
@@ -858,13 +889,13 @@ static hipError_t launch_attn_pp(AttnArgs a, int B, int causal, hipStream_t s) {
   return hipGetLastError();
 }
 
-constexpr int kPingPongMinQueries = 4096;  // query ranges from here on take the ping-pong kernel
 constexpr int kCUs = 256;  // MI355X compute units
 
 // Kernel variants (XB_ATTN_*) and the head widths each is built for.
 static bool attention_variant_fits(int variant, int hd, bool masked) {
   switch (variant) {
-    case XB_ATTN_W4_Q16: case XB_ATTN_W8_Q16: return hd == 256;
+    case XB_ATTN_W4_Q16: return true;
+    case XB_ATTN_W8_Q16: return hd == 256;
     case XB_ATTN_W4_Q32: return hd <= 128;
     case XB_ATTN_W4_Q64: return hd <= 64;
     case XB_ATTN_PINGPONG: return hd == 64 && !masked;
@@ -872,18 +903,32 @@ static bool attention_variant_fits(int variant, int hd, bool masked) {
   }
 }
 
-// The library's choice.  head_dim 256 up to 128 queries: one 8-wave block
-// takes all of them, so each K/V row is fetched once per (batch, head)
-// instead of by two 64-query blocks (cfg3's geometry: 16.7 vs 18.6 us) -- when
-// the B*H blocks still fill the GPU.  head_dim 64 without a key mask from
-// kPingPongMinQueries on: the ping-pong kernel.  Other long ranges take 64
-// queries per wave (each K/V fragment read from LDS then feeds 4 MFMAs);
-// short ones keep 32 so a block does not outgrow S_q.
+// The library's choice; every variant of a head width gives the same bits.
+// head_dim 256 up to 128 queries: one 8-wave block takes all of them, so each
+// K/V row is fetched once per (batch, head) instead of by two 64-query blocks
+// (cfg3's geometry: 16.7 vs 18.6 us) -- when the B*H blocks still fill the
+// GPU.  Otherwise more queries per wave mean fewer LDS reads per product (each
+// K/V fragment read feeds 1, 2 or 4 MFMAs) but fewer, longer blocks, and what
+// counts while the GPU is not full is the longest block.  Measured (us, 16 /
+// 32 / 64 queries per wave, head_dim 64 unless said): B = 1, S = 1500, 12
+// heads 20.1 / 24.3 / 36.6; 1 x 4000 x 16 79.6 / 85.4 / 117; 2 x 2907 x 16
+// 64.6 / 61.6 / 78.3; 8 x 2048 x 16 145 / 125 / 153; 8 x 4096 x 16 - / 347 /
+// 344; 1 x 16384 x 16 751 / 601 / 534; head_dim 128, 3 x 446 x 8 10.9 / 14.8,
+// 16 x 1024 x 8 76.8 / 69.1.  So 16 up to 640 blocks of 128 queries, 64 from
+// 16384 queries or 2048 blocks of at least 4096 queries on.  The ping-pong
+// kernel (head_dim 64, no key mask) is ahead from 16384 queries on (1 x 16384
+// x 16 530 us, 1 x 32768 x 16 2025 against 2073) and behind below (8 x 4096 x
+// 16 388 against 344, 1 x 8000 x 16 206 against 177); with 32 heads and more
+// it keeps the plans past 4096 queries, where it is within 2 to 9 % (2 x 4128
+// x 16 120 with V handed over transposed, 126 without, against 117; 4 x 8192 x
+// 16 629 and 643 against 620).
 static int select_attention(int64_t B, int S_q, int H, int hd, bool masked) {
   if (hd >= 256) return S_q <= 128 && B * H >= kCUs ? XB_ATTN_W8_Q16 : XB_ATTN_W4_Q16;
+  if (hd == 64 && !masked && (S_q >= 16384 || (S_q > 4096 && B * H >= 32))) return XB_ATTN_PINGPONG;
+  if ((S_q + 127) / 128 * B * H <= 640) return XB_ATTN_W4_Q16;
   if (hd >= 128) return XB_ATTN_W4_Q32;
-  if (hd == 64 && !masked && S_q >= kPingPongMinQueries) return XB_ATTN_PINGPONG;
-  return S_q >= 1024 ? XB_ATTN_W4_Q64 : XB_ATTN_W4_Q32;
+  const bool many = S_q >= 16384 || (S_q >= 4096 && (S_q + 255) / 256 * B * H >= 2048);
+  return many ? XB_ATTN_W4_Q64 : XB_ATTN_W4_Q32;
 }
 
 template <int HD>
@@ -892,8 +937,10 @@ static hipError_t run_attn(int variant, const AttnArgs& a, int B, int causal, hi
     if (variant == XB_ATTN_W8_Q16) return launch_attn<HD, 1, 8>(a, B, causal, s);
     return launch_attn<HD, 1>(a, B, causal, s);
   } else if constexpr (HD >= 128) {
+    if (variant == XB_ATTN_W4_Q16) return launch_attn<HD, 1>(a, B, causal, s);
     return launch_attn<HD, 2>(a, B, causal, s);
   } else {
+    if (variant == XB_ATTN_W4_Q16) return launch_attn<HD, 1>(a, B, causal, s);
     if constexpr (HD == 64) {
       if (variant == XB_ATTN_PINGPONG) return launch_attn_pp<HD>(a, B, causal, s);
     }

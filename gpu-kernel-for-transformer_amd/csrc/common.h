@@ -99,6 +99,14 @@ __device__ __forceinline__ void dma16(const void* src_lane, void* lds_wave_base)
   __builtin_amdgcn_global_load_lds((global_void_t*)src_lane, (lds_void_t*)lds_wave_base, 16, 0, 0);
 }
 
+// Blocks are dispatched round-robin over the 8 XCDs (block b -> XCD b % 8).
+// Renumber so that each XCD walks a contiguous range of tiles: neighbouring
+// tiles share their A rows, which then stay in that XCD's L2.
+__device__ __forceinline__ int xcd_contiguous_tile(int b, int nb) {
+  const int q = nb / 8, r = nb % 8, x = b % 8;
+  return x * q + (x < r ? x : r) + b / 8;
+}
+
 // dma16 issued from inline assembly: the compiler does not see this LDS
 // write, so it adds no wait for it before later LDS reads (it cannot tell the
 // ring buffer being filled from the one being read, and would wait before

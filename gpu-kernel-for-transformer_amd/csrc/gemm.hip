@@ -30,14 +30,6 @@ namespace xb {
 constexpr int kGemmBK = 64;
 constexpr int kGemmLDK = kGemmBK + 8;  // padded LDS row (halves): 144 bytes
 
-// Blocks are dispatched round-robin over the 8 XCDs (block b -> XCD b % 8).
-// Renumber so that each XCD walks a contiguous range of tiles: neighbouring
-// tiles share their A rows, which then stay in that XCD's L2.
-__device__ __forceinline__ int xcd_contiguous_tile(int b, int nb) {
-  const int q = nb / 8, r = nb % 8, x = b % 8;
-  return x * q + (x < r ? x : r) + b / 8;
-}
-
 // Tile coordinates of the direct-to-LDS kernel: tiles are ordered in bands of
 // 1024 rows (four row blocks of 256), column by column inside a band, and
 // each XCD takes a contiguous range of that order (xcd_contiguous_tile).  One

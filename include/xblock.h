@@ -76,7 +76,7 @@ const char* xb_strerror(int code);
 #define XB_LINEAR_ROWS 6          /* gemm_rows_kernel: M <= 32, N % 16 == 0, K % 32 == 0, K <= 4096 */
 #define XB_LINEAR_DMA_64x64 7
 /* xb_attention_v: waves per block x queries per block. */
-#define XB_ATTN_W4_Q16 0     /* head_dim 256                              */
+#define XB_ATTN_W4_Q16 0     /* any head_dim                              */
 #define XB_ATTN_W4_Q32 1     /* head_dim <= 128                           */
 #define XB_ATTN_W4_Q64 2     /* head_dim <= 64                            */
 #define XB_ATTN_W8_Q16 3     /* head_dim 256                              */

@@ -457,6 +457,30 @@ def test_attention_every_variant(pkg, cuda, causal, hd, b, s, h, variants):
 
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("hd,s", [(8, 65), (16, 200), (32, 700), (64, 130), (64, 1025), (128, 333)])
+def test_attention_variants_give_the_same_bits(pkg, cuda, hd, s, causal, masked):
+    """16, 32 and 64 queries per wave agree bit for bit, with scores that move the
+    softmax offset late and for single queries, holes in the mask, and one to
+    many key tiles; so a sequence's rows do not depend on the batch it is in."""
+    capi = pkg._capi
+    b, h = 2, 3
+    qkv = torch.randn(b, s, 3, h, hd, generator=_gen(hd + s))
+    qkv[:, s // 2, 1] *= 6.0       # a key some queries score far above everything before it (std 6)
+    qkv = qkv.view(b, s, 3 * h * hd).half()
+    valid = torch.rand(b, s, generator=_gen(s)) > 0.3 if masked else None
+    ref = _attention_reference(qkv, h, valid, causal)
+    qg, vg = qkv.to(cuda), None if valid is None else valid.to(cuda)
+    names = ["XB_ATTN_W4_Q16", "XB_ATTN_W4_Q32"] + (["XB_ATTN_W4_Q64"] if hd <= 64 else [])
+    outs = [pkg.attention(qg, h, key_valid=vg, causal=causal, variant=getattr(capi, n)) for n in names]
+    # Q is rounded to FP16 once more with the scale (2^-11 relative): a score of 24 (4 std) is off by up to
+    # 24 * 2^-11 = 0.012, its probability p by 0.012 p (1 - p) <= 0.003, times |v| differences of up to 8.
+    torch.testing.assert_close(outs[0].cpu().float(), ref, atol=2.4e-2, rtol=0)
+    for n, o in zip(names[1:], outs[1:]):
+        assert torch.equal(o, outs[0]), n
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("masked", [False, True])
 def test_attention_hd256_short_one_block_per_head(pkg, cuda, causal, masked):
     """cfg3's geometry (B*H = 256 heads of S = 128, head_dim 256) takes one 8-wave
     block per head; slices of two sequences (8 heads) take the 4-wave blocks.
