@@ -75,11 +75,11 @@ struct AttnArgs {
   const half_t* v;
   half_t* out;
   const uint8_t* key_valid;  // [B, S_k] bytes (KEYMASK only)
-  float* ws_o;               // split partials: [B*H][splits][BQ][HD] (SPLIT only)
-  float2* ws_ml;             // split partials: [B*H][splits][BQ] (offset, row sum)
+  float* ws_o;               // split partials: [B*H][splits][ws_rows][HD] (SPLIT only)
+  float2* ws_ml;             // split partials: [B*H][splits][ws_rows] (offset, row sum)
   int64_t q_bstride, k_bstride, k_hstride, o_bstride;
   int q_rstride, k_rstride, o_rstride;
-  int H, S_q, S_k, q_offset, q_tiles, n_splits, split_keys;
+  int H, S_q, S_k, q_offset, q_tiles, n_splits, split_keys, ws_rows;
   float scale_log2;
   // Ping-pong kernel only: V transposed per head by the QKV GEMM,
   // vt[b][h][d][p] (rows of vt_row elements, key order inside each 32-key
@@ -114,8 +114,9 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_kernel(const AttnArgs a)
   constexpr bool TRACK = KEYMASK || SPLIT;  // a query may see no key in its first tile
   // One-wave split blocks keep a single LDS tile (the next one waits in
   // registers), so more of them fit on a CU.
-  constexpr int NBUF = SPLIT ? 1 : 2;
-  constexpr int AHEAD = SPLIT || HD >= 256 || NQ > 2 ? 1 : 2;
+  constexpr bool DECODE = SPLIT && NW == 1;
+  constexpr int NBUF = DECODE ? 1 : 2;
+  constexpr int AHEAD = DECODE || HD >= 256 || NQ > 2 ? 1 : 2;
   static_assert(NT >= BKEYS, "one thread per key stages the validity bytes");
 
   __shared__ __attribute__((aligned(16))) half_t k_lds[NBUF][BKEYS * LDK];
@@ -127,11 +128,12 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_kernel(const AttnArgs a)
   // head's K and V for all of them (dealt round-robin, every L2 streamed every
   // head's: B = 1, S = 8000, 16 heads of 64 246 -> 174 us, B = 8, S = 2048
   // padded 173 -> 136 us; ping-pong kernel at S = 32768 2928 -> 2025 us).
-  const int per_bh = SPLIT ? a.n_splits : a.q_tiles;
+  const int per_bh = SPLIT ? a.n_splits * a.q_tiles : a.q_tiles;
   const int block = xcd_contiguous_tile(blockIdx.x, gridDim.x);
   const int bh = block / per_bh;
   const int sub = block % per_bh;
-  const int qt = SPLIT ? 0 : (CAUSAL ? a.q_tiles - 1 - sub : sub);
+  const int split = SPLIT ? sub / a.q_tiles : 0;
+  const int qt = CAUSAL ? a.q_tiles - 1 - sub % a.q_tiles : sub % a.q_tiles;
   const int b = bh / a.H, h = bh % a.H;
   const int S_q = a.S_q, S_k = a.S_k, q_offset = a.q_offset;
   const half_t* base = a.q + (int64_t)b * a.q_bstride + (int64_t)h * HD;
@@ -195,7 +197,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_kernel(const AttnArgs a)
   }
   const half8_t ones8 = {1, 1, 1, 1, 1, 1, 1, 1};
 
-  const int k_begin = SPLIT ? sub * a.split_keys : 0;
+  const int k_begin = SPLIT ? split * a.split_keys : 0;
   int key_end = CAUSAL ? min(S_k, q_offset + q0 + BQ) : S_k;
   if constexpr (SPLIT) key_end = min(key_end, k_begin + a.split_keys);
   const int n_tiles = key_end > k_begin ? (key_end - k_begin + BKEYS - 1) / BKEYS : 0;
@@ -226,7 +228,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_kernel(const AttnArgs a)
       const int key = min(k0 + id / CPK, key_last), c = (id % CPK) * 8;
       const half8_t* kp = reinterpret_cast<const half8_t*>(kbase + key * k_rstride + c);
       const half8_t* vp = reinterpret_cast<const half8_t*>(vbase + key * k_rstride + c);
-      if constexpr (SPLIT) {
+      if constexpr (DECODE) {
         // Decode streams each cached row exactly once: non-temporal loads
         // keep it from displacing reusable lines (87% vs 77% of HBM peak
         // on a 100k-token cache).
@@ -413,18 +415,18 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_kernel(const AttnArgs a)
   if constexpr (SPLIT) {
     // Unnormalised partial of this key range: o, the offset m_run (-inf when
     // the range showed the query no key) and the row sum.
-    const int64_t slot = (int64_t)bh * a.n_splits + sub;
+    const int64_t slot = (int64_t)bh * a.n_splits + split;
 #pragma unroll
     for (int qb = 0; qb < NQ; ++qb) {
       const int q = qw0 + 16 * qb + r16;
       if (q >= S_q) continue;
-      float* wo = a.ws_o + (slot * BQ + q) * HD;
+      float* wo = a.ws_o + (slot * a.ws_rows + q) * HD;
 #pragma unroll
       for (int hb = 0; hb < HB; ++hb) {
         const int d = 16 * hb + 4 * g;
         if (d < HD) *reinterpret_cast<float4_t*>(wo + d) = o[hb][qb];
       }
-      if (g == 0) a.ws_ml[slot * BQ + q] = make_float2(m_set[qb] ? m_run[qb] : -INFINITY, lacc[qb][0]);
+      if (g == 0) a.ws_ml[slot * a.ws_rows + q] = make_float2(m_set[qb] ? m_run[qb] : -INFINITY, lacc[qb][0]);
     }
     return;
   }
@@ -814,41 +816,64 @@ __global__ __launch_bounds__(512, 1) void attn_pp_kernel(const AttnArgs a) {
 
 // Merges the key-range partials of attn_kernel<..., SPLIT>: per (batch, head,
 // query) M = max_s m_s, out = sum_s 2^(m_s - M) o_s / sum_s 2^(m_s - M) l_s.
-// One thread per 8 context columns.
+// One block per query: the splits' weights are formed side by side, then HD /
+// 4 threads walk a row and 1024 / HD rows are in flight at once.  (One thread
+// per 8 columns walking the splits one after the other waited for each load
+// in turn: with the split kernel, B = 4, 16 heads of 64, 517 keys 15.3 -> 9.7
+// us, B = 1, 20,001 keys 100 -> 19.5 us.)
+constexpr int kMaxSplits = 2048;
 template <int HD>
-__global__ __launch_bounds__(256) void attn_split_combine(const AttnArgs a, int BQ, int64_t total) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= total) return;
-  constexpr int C8 = HD / 8;
-  const int c = (int)(idx % C8);
-  const int64_t rest = idx / C8;
-  const int q = (int)(rest % a.S_q);
-  const int64_t bh = rest / a.S_q;
-  const int b = (int)(bh / a.H), h = (int)(bh % a.H);
-  const float2* ml = a.ws_ml + bh * a.n_splits * BQ + q;
+__global__ __launch_bounds__(256) void attn_split_combine(const AttnArgs a) {
+  constexpr int C4 = HD / 4, R = 256 / C4;
+  __shared__ float w[kMaxSplits];
+  __shared__ float red[2][4];
+  __shared__ float4_t part[256];
+  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+  const int q = blockIdx.x % a.S_q;
+  const int64_t bh = blockIdx.x / a.S_q;
+  const int b = (int)(bh / a.H), h = (int)(bh % a.H), n = a.n_splits;
+  const float2* ml = a.ws_ml + bh * n * a.ws_rows + q;
+  const float* wo = a.ws_o + (bh * n * a.ws_rows + q) * HD + 4 * (tid % C4);
   float m = -INFINITY;
-  for (int s = 0; s < a.n_splits; ++s) m = fmaxf(m, ml[(int64_t)s * BQ].x);
-  float l = 0.f, acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < a.n_splits; ++s) {
-    const float2 p = ml[(int64_t)s * BQ];
-    if (p.x == -INFINITY) continue;
-    const float w = __builtin_amdgcn_exp2f(p.x - m);
-    l = fmaf(w, p.y, l);
-    const float* wo = a.ws_o + ((bh * a.n_splits + s) * BQ + q) * HD + 8 * c;
-    const float4_t lo = *reinterpret_cast<const float4_t*>(wo);
-    const float4_t hi = *reinterpret_cast<const float4_t*>(wo + 4);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      acc[i] = fmaf(w, lo[i], acc[i]);
-      acc[4 + i] = fmaf(w, hi[i], acc[4 + i]);
-    }
+  for (int s = tid; s < n; s += 256) m = fmaxf(m, ml[(int64_t)s * a.ws_rows].x);
+  m = group_max<kWave>(m);
+  if (lane == 0) red[0][wave] = m;
+  __syncthreads();
+  m = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
+  if (m == -INFINITY) m = 0.f;  // no split saw a key: every weight is 0
+  float l = 0.f;
+  for (int s = tid; s < n; s += 256) {
+    const float2 p = ml[(int64_t)s * a.ws_rows];
+    const float e = __builtin_amdgcn_exp2f(p.x - m);
+    w[s] = e;
+    l = fmaf(e, p.y, l);
   }
-  const float inv = l > 0.f ? 1.f / l : 0.f;
-  half8_t r;
+  l = group_sum<kWave>(l);
+  if (lane == 0) red[1][wave] = l;
+  __syncthreads();
+  l = (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]);
+  float4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int s = tid / C4; s < n; s += R) {
+    const float e = w[s];
+    const float4_t v = *reinterpret_cast<const float4_t*>(wo + (int64_t)s * a.ws_rows * HD);
 #pragma unroll
-  for (int i = 0; i < 8; ++i) r[i] = (half_t)(acc[i] * inv);
-  *reinterpret_cast<half8_t*>(a.out + (int64_t)b * a.o_bstride + (int64_t)q * a.o_rstride +
-                              (int64_t)h * HD + 8 * c) = r;
+    for (int i = 0; i < 4; ++i) acc[i] = e == 0.f ? acc[i] : fmaf(e, v[i], acc[i]);
+  }
+  part[tid] = acc;
+  __syncthreads();
+#pragma unroll
+  for (int k = R / 2; k > 0; k /= 2) {
+    if (tid < k * C4) part[tid] += part[tid + k * C4];
+    __syncthreads();
+  }
+  if (tid < C4) {
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    half4_t r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = (half_t)(part[tid][i] * inv);
+    *reinterpret_cast<half4_t*>(a.out + (int64_t)b * a.o_bstride + (int64_t)q * a.o_rstride + (int64_t)h * HD + 4 * tid) = r;
+  }
 }
 
 template <int HD, int NQ, int NW = 4>
@@ -960,51 +985,68 @@ static hipError_t dispatch_attn(const AttnArgs& a, int B, int causal, hipStream_
 constexpr int kDecodeQueries = 16;
 constexpr int64_t kDecodeTargetBlocks = 2048;
 
-struct DecodeGeometry {
-  int n_splits, split_keys;
-  int64_t o_bytes, bytes;  // partial o, then (offset, sum) pairs
+struct SplitGeometry {
+  int n_splits, split_keys, rows;  // rows: partial rows per (batch, head, split)
+  int64_t o_bytes, bytes;          // partial o, then (offset, sum) pairs; 0 bytes: no split
 };
 
-// Bytes of one split's partials for one (batch, head): kDecodeQueries rows of
-// HD FP32 outputs plus an (offset, sum) pair each.
-static int64_t decode_split_bytes(int HD) {
-  return (int64_t)kDecodeQueries * (HD * (int64_t)sizeof(float) + (int64_t)sizeof(float2));
+// Bytes of one split's partials for one (batch, head).
+static int64_t split_partial_bytes(int64_t rows, int HD) {
+  return rows * (HD * (int64_t)sizeof(float) + (int64_t)sizeof(float2));
 }
 
 // The split count is also capped so that the partials fit the no-allocation
 // entry point's static scratch whenever one split per (batch, head) does:
 // both entry points then run the same geometry and give the same bits.
-static DecodeGeometry decode_geometry(int B, int H, int S_k, int HD) {
+//
+// Chunks of more than kDecodeQueries tokens split their keys only where their
+// blocks of 64 queries would leave most of the GPU idle (kChunkTargetBlocks:
+// three per CU) over at least kChunkMinTiles key tiles per split; 0 bytes
+// otherwise.  B = 1, 16 heads of 64: 100 tokens over a cache of 50,000 789 -> 54
+// us, 512 over 8,000 139 -> 50 us.
+constexpr int64_t kChunkTargetBlocks = 768;
+constexpr int kChunkMinTiles = 8;
+static SplitGeometry split_geometry(int B, int H, int64_t chunk, int S_k, int HD) {
   const int bk = HD >= 256 ? 32 : 64;
   const int tiles = (S_k + bk - 1) / bk;
   const int64_t bh = (int64_t)B * H;
-  const int64_t fit = std::max<int64_t>(1, XB_DECODE_SCRATCH_BYTES / (bh * decode_split_bytes(HD)));
-  const int64_t want = std::min<int64_t>(std::min<int64_t>(tiles, fit),
-                                         std::max<int64_t>(1, (kDecodeTargetBlocks + bh - 1) / bh));
+  const bool decode = chunk <= kDecodeQueries;
+  SplitGeometry g = {};
+  g.rows = decode ? kDecodeQueries : (int)chunk;
+  const int64_t fit = std::max<int64_t>(1, XB_DECODE_SCRATCH_BYTES / (bh * split_partial_bytes(g.rows, HD)));
+  const int64_t blocks = decode ? bh : bh * ((chunk + 63) / 64);
+  const int64_t target = decode ? kDecodeTargetBlocks : kChunkTargetBlocks;
+  int64_t want = std::min<int64_t>(std::min<int64_t>(tiles, fit), std::max<int64_t>(1, (target + blocks - 1) / blocks));
+  if (!decode) want = std::min<int64_t>(want, tiles / kChunkMinTiles);
+  if (!decode && want < 2) return g;
+  want = std::min<int64_t>(want, kMaxSplits);
   const int tiles_per = (int)((tiles + want - 1) / want);
-  DecodeGeometry g;
   g.split_keys = tiles_per * bk;
   g.n_splits = (S_k + g.split_keys - 1) / g.split_keys;
-  const int64_t slots = bh * g.n_splits * kDecodeQueries;
+  const int64_t slots = bh * g.n_splits * g.rows;
   g.o_bytes = slots * HD * (int64_t)sizeof(float);
   g.bytes = g.o_bytes + slots * (int64_t)sizeof(float2);
   return g;
 }
 
 template <int HD>
-static hipError_t launch_decode(AttnArgs a, int B, const DecodeGeometry& geo, void* workspace, hipStream_t s) {
-  static_assert(AttnCfg<HD, 1, 1>::BQ == kDecodeQueries, "one wave of 16 queries");
+static hipError_t launch_split(AttnArgs a, int B, const SplitGeometry& geo, void* workspace, hipStream_t s) {
+  static_assert(AttnCfg<HD, 1, 1>::BQ == kDecodeQueries && AttnCfg<HD, 1>::BQ == 64, "queries per block");
+  const bool decode = a.S_q <= kDecodeQueries;
   a.n_splits = geo.n_splits;
   a.split_keys = geo.split_keys;
+  a.ws_rows = geo.rows;
+  a.q_tiles = decode ? 1 : (a.S_q + 63) / 64;
   a.ws_o = static_cast<float*>(workspace);
   a.ws_ml = reinterpret_cast<float2*>(static_cast<char*>(workspace) + geo.o_bytes);
-  const int64_t blocks = (int64_t)B * a.H * geo.n_splits;
-  if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((attn_kernel<HD, 1, 1, true, false, true>), dim3((unsigned)blocks), dim3(64), 0, s, a);
-  const int64_t total = (int64_t)B * a.H * a.S_q * (HD / 8);
-  const int64_t cblocks = (total + 255) / 256;
-  if (cblocks > 0x7fffffffLL) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((attn_split_combine<HD>), dim3((unsigned)cblocks), dim3(256), 0, s, a, kDecodeQueries, total);
+  const int64_t blocks = (int64_t)B * a.H * geo.n_splits * a.q_tiles;
+  const int64_t queries = (int64_t)B * a.H * a.S_q;
+  if (blocks > 0x7fffffffLL || queries > 0x7fffffffLL) return hipErrorInvalidValue;
+  if (decode)
+    hipLaunchKernelGGL((attn_kernel<HD, 1, 1, true, false, true>), dim3((unsigned)blocks), dim3(64), 0, s, a);
+  else
+    hipLaunchKernelGGL((attn_kernel<HD, 1, 4, true, false, true>), dim3((unsigned)blocks), dim3(256), 0, s, a);
+  hipLaunchKernelGGL((attn_split_combine<HD>), dim3((unsigned)queries), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
@@ -1165,13 +1207,14 @@ extern "C" int64_t xb_attention_kv_cache_workspace_bytes(int32_t batch, int64_t 
                                                          int32_t head_dim, int64_t start) {
   const int bad = check_cache_args(batch, chunk, heads, head_dim, start, start + chunk);
   if (bad) return bad;
-  if (batch == 0 || chunk == 0 || chunk > kDecodeQueries) return 0;
-  return decode_geometry(batch, heads, (int)(start + chunk), head_dim).bytes;
+  if (batch == 0 || chunk == 0) return 0;
+  return split_geometry(batch, heads, chunk, (int)(start + chunk), head_dim).bytes;
 }
 
 // The cached-attention call behind xb_attention_kv_cache and its no-allocation
-// variant.  `workspace_of(bytes, &ptr)` supplies the decode partials' memory
-// (or an error code) once the call has been validated and sized.
+// variant.  `workspace_of(bytes, optional, &ptr)` supplies the split partials'
+// memory (or an error code; or, where optional, nothing) once the call has been
+// validated and sized.
 template <typename WorkspaceOf>
 static int attention_kv_cache(const void* qkv, const void* k_cache, const void* v_cache, void* out, int32_t batch,
                               int64_t chunk, int32_t heads, int32_t head_dim, int64_t start, int64_t capacity,
@@ -1200,13 +1243,15 @@ static int attention_kv_cache(const void* qkv, const void* k_cache, const void* 
   a.q_offset = (int)start;
   a.scale_log2 = scale * 1.44269504088896340736f;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (chunk > kDecodeQueries)
-    return (int)by_head_dim(head_dim, [&](auto hd) { return dispatch_attn<decltype(hd)::value>(a, batch, 1, s); });
-  const DecodeGeometry geo = decode_geometry(batch, heads, a.S_k, head_dim);
+  const SplitGeometry geo = split_geometry(batch, heads, chunk, a.S_k, head_dim);
   void* workspace = nullptr;
-  const int got = workspace_of(geo.bytes, &workspace);
-  if (got != XB_OK) return got;
-  return (int)by_head_dim(head_dim, [&](auto hd) { return launch_decode<decltype(hd)::value>(a, batch, geo, workspace, s); });
+  if (geo.bytes > 0) {
+    const int got = workspace_of(geo.bytes, chunk > kDecodeQueries, &workspace);
+    if (got != XB_OK) return got;
+  }
+  if (workspace == nullptr)  // a long chunk that needs no split, or whose caller brought no workspace
+    return (int)by_head_dim(head_dim, [&](auto hd) { return dispatch_attn<decltype(hd)::value>(a, batch, 1, s); });
+  return (int)by_head_dim(head_dim, [&](auto hd) { return launch_split<decltype(hd)::value>(a, batch, geo, workspace, s); });
 }
 
 extern "C" int xb_attention_kv_cache(const void* qkv, const void* k_cache, const void* v_cache, void* out,
@@ -1214,7 +1259,8 @@ extern "C" int xb_attention_kv_cache(const void* qkv, const void* k_cache, const
                                      int64_t capacity, float scale, void* workspace, int64_t workspace_bytes,
                                      void* stream) {
   return attention_kv_cache(qkv, k_cache, v_cache, out, batch, chunk, heads, head_dim, start, capacity, scale, stream,
-                            [&](int64_t need, void** ptr) {
+                            [&](int64_t need, bool optional, void** ptr) {
+                              if (optional && (!workspace || workspace_bytes < need)) return XB_OK;
                               if (!workspace) return XB_ERR_NULL_POINTER;
                               if (workspace_bytes < need) return XB_ERR_WORKSPACE;
                               if ((uintptr_t)workspace & 15u) return XB_ERR_MISALIGNED;
@@ -1270,8 +1316,8 @@ extern "C" int xb_attention_kv_cache_noalloc(const void* qkv, const void* k_cach
                                              int32_t batch, int64_t chunk, int32_t heads, int32_t head_dim,
                                              int64_t start, int64_t capacity, float scale, void* stream) {
   return attention_kv_cache(qkv, k_cache, v_cache, out, batch, chunk, heads, head_dim, start, capacity, scale, stream,
-                            [&](int64_t need, void** ptr) {
-                              if (need > XB_DECODE_SCRATCH_BYTES) return XB_ERR_SCRATCH_TOO_SMALL;
+                            [&](int64_t need, bool optional, void** ptr) {
+                              if (need > XB_DECODE_SCRATCH_BYTES) return optional ? XB_OK : XB_ERR_SCRATCH_TOO_SMALL;
                               return scratch_address(static_cast<hipStream_t>(stream), ptr);
                             });
 }

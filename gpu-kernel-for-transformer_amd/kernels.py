@@ -466,7 +466,8 @@ def attention_kv_cache(
 
     Call after kv_cache_append for the same chunk (TTB:747-765).  `workspace`
     (uint8, at least kv_cache_workspace_bytes) is allocated here when not
-    given; decode chunks of up to 16 tokens need one.  no_alloc=True calls
+    given; decode chunks of up to 16 tokens need one, longer ones over a long
+    cache use it.  no_alloc=True calls
     xb_attention_kv_cache_noalloc instead, whose partials live in the
     library's static per-GPU scratch (with `out` given, nothing is
     allocated); calls that overlap in time on one GPU must not use it.
@@ -497,7 +498,7 @@ def attention_kv_cache(
     ws_ptr = workspace.data_ptr() if need else None
     ws_bytes = workspace.numel() * workspace.element_size() if need else 0
     check(
-        _launch(f"attention_kv_hd{head_dim}{'_decode' if need else ''}", lambda: lib().xb_attention_kv_cache(
+        _launch(f"attention_kv_hd{head_dim}{'_decode' if chunk <= 16 else ''}", lambda: lib().xb_attention_kv_cache(
             qkv.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), batch, chunk, num_heads,
             head_dim, int(start), capacity, float(scale), ws_ptr, ws_bytes, stream_handle(qkv.device))),
         "xb_attention_kv_cache",
@@ -506,7 +507,7 @@ def attention_kv_cache(
 
 
 def kv_cache_workspace_bytes(batch: int, chunk: int, num_heads: int, head_dim: int, start: int) -> int:
-    """Workspace bytes xb_attention_kv_cache needs (0 for chunks longer than 16 tokens)."""
+    """Workspace bytes xb_attention_kv_cache needs (decode) or can use (chunks longer than 16 tokens; may be 0)."""
     need = lib().xb_attention_kv_cache_workspace_bytes(batch, chunk, num_heads, head_dim, int(start))
     if need < 0:
         check(int(need), "xb_attention_kv_cache_workspace_bytes")

@@ -226,8 +226,10 @@ int xb_attention_causal_vt(const void* qkv, const void* vt, void* out,
  * start + chunk <= capacity, else XB_ERR_BAD_SIZE (the reference raises
  * ValueError, TTB:434-438).  A chunk of at most 16 tokens (decode) splits
  * the keys over the GPU and needs a caller-provided workspace of
- * xb_attention_kv_cache_workspace_bytes(...) bytes (16-byte aligned; 0 for
- * longer chunks, which need none); a smaller one gives XB_ERR_WORKSPACE.
+ * xb_attention_kv_cache_workspace_bytes(...) bytes (16-byte aligned); a
+ * smaller one gives XB_ERR_WORKSPACE.  Longer chunks need none: with the bytes
+ * the function gives (0 where there is nothing to gain) they split the keys
+ * too, with less or NULL they don't.
  */
 int xb_kv_cache_append(const void* qkv, void* k_cache, void* v_cache,
                        int32_t batch, int64_t chunk, int32_t heads,

@@ -658,6 +658,34 @@ def test_decode_long_cache(pkg, cuda, b, heads, hd, start):
     torch.testing.assert_close(out.cpu().float(), ref, atol=2e-3, rtol=1e-2)
 
 
+@pytest.mark.parametrize("b,heads,hd,start,chunk", [
+    (1, 2, 64, 6000, 17), (2, 2, 64, 5000, 130), (1, 3, 8, 4095, 64), (1, 2, 128, 3001, 100), (1, 1, 256, 2100, 33),
+    (1, 2, 32, 2047, 300)])
+def test_chunk_over_long_cache(pkg, cuda, b, heads, hd, start, chunk):
+    """Chunks of more than 16 tokens over a long cache split the keys when given the
+    workspace for it: against the reference, next to the unsplit call without
+    one, and the no-allocation call runs the same split."""
+    lib = pkg._capi.lib()
+    length = start + chunk
+    qkv = torch.randn(b, length, 3 * heads * hd, generator=_gen(start)).half()
+    kc, vc = _fill_cache(pkg, qkv, heads, length, [start, chunk], cuda)
+    t = qkv.float().view(b, length, 3, heads, hd).permute(2, 0, 3, 1, 4)
+    scores = (t[0][:, :, start:] @ t[1].transpose(2, 3).contiguous()) * hd**-0.5
+    late = torch.arange(length)[None, :] > torch.arange(start, length)[:, None]
+    ref = (torch.softmax(scores.masked_fill(late, float("-inf")), -1) @ t[2]).transpose(1, 2).reshape(b, chunk, heads * hd)
+    need = pkg.kernels.kv_cache_workspace_bytes(b, chunk, heads, hd, start)
+    assert need > 0
+    q = qkv[:, start:].contiguous().to(cuda)
+    out = pkg.attention_kv_cache(q, kc, vc, heads, start)
+    torch.testing.assert_close(out.cpu().float(), ref, atol=2e-3, rtol=1e-2)
+    plain = torch.empty_like(out)
+    code = lib.xb_attention_kv_cache(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), plain.data_ptr(), b, chunk, heads, hd,
+                                     start, length, hd**-0.5, None, 0, pkg._capi.stream_handle(q.device))
+    assert code == 0
+    torch.testing.assert_close(plain.cpu().float(), ref, atol=2e-3, rtol=1e-2)
+    assert torch.equal(pkg.attention_kv_cache(q, kc, vc, heads, start, no_alloc=True), out)
+
+
 def test_decode_workspace_too_small(pkg, cuda):
     b, heads, hd, start = 1, 2, 64, 300
     qkv_full = torch.randn(b, start + 1, 3 * heads * hd, generator=_gen(3)).half()
