@@ -97,6 +97,35 @@ def test_layer_norm_errors(pkg, cuda):
         pkg.layer_norm(x.cpu(), torch.ones(128), torch.zeros(128), 1e-5, F16)
 
 
+@pytest.mark.parametrize("cols", [768, 1536, 3072, 4096])
+@pytest.mark.parametrize("mode", [0, 1, 2, 4])
+def test_layer_norm_vector_widths(pkg, cuda, cols, mode):
+    """Widths that use the vector kernel when the pointers are 16-byte aligned and
+    the per-row kernel otherwise: both match the FP32 reference and take every row mask."""
+    rows = 7
+    x = torch.randn(rows, cols, generator=_gen(cols))
+    u = torch.randn(rows, cols, generator=_gen(cols + 1)).half()
+    g, b = torch.randn(cols, generator=_gen(2)), torch.randn(cols, generator=_gen(3))
+    valid = torch.tensor([1, 0, 1, 1, 0, 1, 1], dtype=torch.uint8)
+    drop = (valid == 0)[:, None]
+    s = x + torch.where(drop & bool(mode & 1), torch.zeros(()), u.float())
+    s = torch.where(drop & bool(mode & 2), torch.zeros(()), s)
+    ref = torch.where(drop & bool(mode & 4), torch.zeros(()), F.layer_norm(s, (cols,), g, b, 1e-5))
+    gg, bg, vg = g.to(cuda), b.to(cuda), valid.to(cuda)
+    for shift in (0, 1):   # 0: aligned; 1: off by one element
+        def place(t):
+            flat = torch.empty(t.numel() + 8, dtype=t.dtype, device=cuda)[shift:shift + t.numel()]
+            flat.copy_(t.flatten())
+            return flat.view(t.shape)
+        res, out = pkg.fused_residual_layer_norm(place(x), place(u), gg, bg, 1e-5, F32, row_valid=vg if mode else None,
+                                                 mask_mode=mode)
+        torch.testing.assert_close(res.cpu(), s, atol=0, rtol=0)
+        torch.testing.assert_close(out.cpu(), ref, atol=2e-5, rtol=2e-5)
+        if not mode:
+            plain = pkg.layer_norm(place(x), gg, bg, 1e-5, F16)
+            torch.testing.assert_close(plain.cpu().float(), F.layer_norm(x, (cols,), g, b, 1e-5), atol=2e-3, rtol=2e-3)
+
+
 # ----------------------------------------------------------------------------- GEMM
 @pytest.mark.parametrize(
     "m,n,k",
