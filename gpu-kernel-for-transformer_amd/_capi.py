@@ -87,6 +87,8 @@ EXPORTED_SYMBOLS = (
     "xb_fused_forward_d128",
     "xb_fused_forward_d128_workspace_bytes",
     "xb_fused_forward_d128_ws",
+    "xb_select_norm_linear",
+    "xb_norm_linear",
     "xb_select_row_block",
     "xb_row_block",
     "xb_stack_workspace_bytes",
@@ -157,6 +159,12 @@ _SIGNATURES = {
     "xb_fused_forward_d128_ws": (
         ctypes.c_int,
         [_vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _i64, _vp, _i32, _vp, _i64, _i32, _i32, _vp],
+    ),
+    "xb_select_norm_linear": (ctypes.c_int, [_i64, _i32, _i32]),
+    "xb_norm_linear": (
+        ctypes.c_int,
+        [_vp, _vp, _vp, _vp, _f32, ctypes.c_int, _vp, _vp, _vp, _vp, _i64, _i32, _i32, ctypes.c_int,
+         _vp, _vp, _i32, _i64, _i64, _i64, _vp],
     ),
     "xb_select_row_block": (ctypes.c_int, [_i32, _i32]),
     "xb_row_block": (ctypes.c_int, [_vp, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp]),

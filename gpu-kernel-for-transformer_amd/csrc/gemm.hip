@@ -429,11 +429,33 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_dma_kernel(
 // chain.
 constexpr int kRowsMax = 32, kRowsSteps = 8, kRowsMaxK = 16 * kRowsSteps * 32;
 
-template <int RG, int EPI>
+//
+// CH > 0 (xb_norm_linear, M <= 8, K = 256 CH): the activations are LN(x +
+// upd), computed here by every block, a row per wave at a time in
+// ln_rows_kernel's order (the same bits), while the weights are on their way;
+// block 0 also writes x + upd.  A decode step's LayerNorms were launches of
+// 4.4 us for a few KB.  KV columns also go to the caches, which saves the
+// append's launch.
+struct RowsExtra {
+  const float* x;          // [M, K] residual stream; not res_out (every block reads it)
+  const half_t* upd;       // [M, K] or NULL
+  const float *gamma, *beta;
+  float* res_out;          // x + upd, or NULL
+  float eps;
+  int affine;
+  half_t *k_cache, *v_cache;  // NULL: none; N = 3D then
+  int heads, head_dim, chunk; // M = batch * chunk
+  int64_t start, capacity;
+};
+constexpr int kNormRowsMax = 8;
+
+template <int RG, int EPI, int CH>
 __global__ __launch_bounds__(1024) void gemm_rows_kernel(
     const half_t* __restrict__ A, const half_t* __restrict__ W,
-    const float* __restrict__ bias, half_t* __restrict__ C, int M, int N, int K) {
+    const float* __restrict__ bias, half_t* __restrict__ C, int M, int N, int K, RowsExtra ex) {
   __shared__ float4_t hand[16][RG][kWave];
+  constexpr int LDN = CH * 256 + 8;
+  __shared__ __attribute__((aligned(16))) half_t normed[CH > 0 ? kNormRowsMax * LDN : 8];
   const int lane = threadIdx.x % kWave, g = lane / 16, r16 = lane % 16;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int waves = blockDim.x / kWave;
@@ -450,8 +472,65 @@ __global__ __launch_bounds__(1024) void gemm_rows_kernel(
   };
 #pragma unroll
   for (int s = 0; s < kRowsSteps; ++s) wf[s] = *reinterpret_cast<const half8_t*>(wrow + 32 * min(s, steps - 1));
-  load_a(0);
-  if constexpr (RG > 1) load_a(1);
+  if constexpr (CH == 0) {
+    load_a(0);
+    if constexpr (RG > 1) load_a(1);
+  } else {
+    constexpr int D = CH * 256;
+    for (int row = wave; row < M; row += waves) {
+      float v[CH][4];
+      float4_t gm[CH], bt[CH];
+#pragma unroll
+      for (int c = 0; c < CH; ++c) {
+        const int col = (c * kWave + lane) * 4;
+        const float4_t x4 = *reinterpret_cast<const float4_t*>(ex.x + (int64_t)row * D + col);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[c][i] = x4[i];
+        if (ex.upd != nullptr) {
+          const half4_t u = *reinterpret_cast<const half4_t*>(ex.upd + (int64_t)row * D + col);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[c][i] += (float)u[i];
+        }
+        if (ex.affine) {
+          gm[c] = *reinterpret_cast<const float4_t*>(ex.gamma + col);
+          bt[c] = *reinterpret_cast<const float4_t*>(ex.beta + col);
+        }
+      }
+      if (ex.res_out != nullptr && blockIdx.x == 0) {
+#pragma unroll
+        for (int c = 0; c < CH; ++c)
+          *reinterpret_cast<float4_t*>(ex.res_out + (int64_t)row * D + (c * kWave + lane) * 4) =
+              float4_t{v[c][0], v[c][1], v[c][2], v[c][3]};
+      }
+      float s = 0.f;
+#pragma unroll
+      for (int c = 0; c < CH; ++c)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s += v[c][i];
+      const float mean = group_sum<kWave>(s) * (1.0f / D);
+      float q = 0.f;
+#pragma unroll
+      for (int c = 0; c < CH; ++c)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          v[c][i] -= mean;
+          q += v[c][i] * v[c][i];
+        }
+      const float rstd = rsqrtf(group_sum<kWave>(q) * (1.0f / D) + ex.eps);
+#pragma unroll
+      for (int c = 0; c < CH; ++c) {
+        half4_t h;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          h[i] = (half_t)(ex.affine ? v[c][i] * rstd * gm[c][i] + bt[c][i] : v[c][i] * rstd);
+        *reinterpret_cast<half4_t*>(normed + row * LDN + (c * kWave + lane) * 4) = h;
+      }
+    }
+    lds_slab_barrier();
+    const half_t* p = normed + min(r16, M - 1) * LDN + wave * (kRowsSteps * 32) + 8 * g;
+#pragma unroll
+    for (int st = 0; st < kRowsSteps; ++st) af[0][st] = *reinterpret_cast<const half8_t*>(p + 32 * st);
+  }
   float b[4] = {0.f, 0.f, 0.f, 0.f};
   if (wave == waves - 1 && bias != nullptr) {
 #pragma unroll
@@ -478,6 +557,15 @@ __global__ __launch_bounds__(1024) void gemm_rows_kernel(
         h[e] = to_half_pinned(v);
       }
       *reinterpret_cast<half4_t*>(C + (int64_t)(16 * rg + r16) * N + n0 + 4 * g) = h;
+      if constexpr (CH > 0) {
+        if (ex.k_cache != nullptr && n0 >= K) {  // K = D here: a block is all Q, all K or all V
+          const int col = (n0 - K) % K + 4 * g;
+          const int64_t row = 16 * rg + r16, bt = row / ex.chunk, t = row - bt * ex.chunk;
+          const int head = col / ex.head_dim, d = col - head * ex.head_dim;
+          half_t* cache = n0 < 2 * K ? ex.k_cache : ex.v_cache;
+          *reinterpret_cast<half4_t*>(cache + ((bt * ex.heads + head) * ex.capacity + ex.start + t) * ex.head_dim + d) = h;
+        }
+      }
     }
     lds_slab_barrier();
   }
@@ -489,9 +577,27 @@ static hipError_t launch_gemm_rows(const half_t* a, const half_t* w, const float
                                    int64_t m, int n, int k, hipStream_t s) {
   const dim3 grid((unsigned)(n / 16)), block((unsigned)(kWave * ((k + 255) / 256)));
   const int rows = (int)m;
-  if (m <= 16) hipLaunchKernelGGL((gemm_rows_kernel<1, EPI>), grid, block, 0, s, a, w, bias, c, rows, n, k);
-  else hipLaunchKernelGGL((gemm_rows_kernel<2, EPI>), grid, block, 0, s, a, w, bias, c, rows, n, k);
+  if (m <= 16) hipLaunchKernelGGL((gemm_rows_kernel<1, EPI, 0>), grid, block, 0, s, a, w, bias, c, rows, n, k, RowsExtra{});
+  else hipLaunchKernelGGL((gemm_rows_kernel<2, EPI, 0>), grid, block, 0, s, a, w, bias, c, rows, n, k, RowsExtra{});
   return hipGetLastError();
+}
+
+template <int EPI>
+static hipError_t launch_norm_rows(const RowsExtra& ex, const half_t* w, const float* bias, half_t* c, int m, int n,
+                                   int k, hipStream_t s) {
+  const dim3 grid((unsigned)(n / 16)), block((unsigned)(kWave * (k / 256)));
+  switch (k / 256) {
+    case 2: hipLaunchKernelGGL((gemm_rows_kernel<1, EPI, 2>), grid, block, 0, s, nullptr, w, bias, c, m, n, k, ex); break;
+    case 3: hipLaunchKernelGGL((gemm_rows_kernel<1, EPI, 3>), grid, block, 0, s, nullptr, w, bias, c, m, n, k, ex); break;
+    case 4: hipLaunchKernelGGL((gemm_rows_kernel<1, EPI, 4>), grid, block, 0, s, nullptr, w, bias, c, m, n, k, ex); break;
+    default: hipLaunchKernelGGL((gemm_rows_kernel<1, EPI, 8>), grid, block, 0, s, nullptr, w, bias, c, m, n, k, ex); break;
+  }
+  return hipGetLastError();
+}
+
+// Widths whose LayerNorm ln_rows_kernel reduces over 64 lanes of 4 columns.
+static bool norm_rows_fit(int64_t m, int n, int k) {
+  return m <= kNormRowsMax && n % 16 == 0 && (k == 512 || k == 768 || k == 1024 || k == 2048);
 }
 
 template <int BM, int BN, int WGM, int WGN, int EPI, int ST, bool VT = false>
@@ -664,4 +770,40 @@ extern "C" int xb_linear_qkv_vt(const void* a, const void* w, const float* bias,
       e = launch_gemm_dma<128, 128, 2, 4, XB_EPI_BIAS, 2, true>(A, Wt, bias, Cc, m, n, k, s, vo); break;
   }
   return (int)e;
+}
+
+extern "C" int xb_select_norm_linear(int64_t rows, int32_t n, int32_t k) {
+  if (rows < 0 || n <= 0 || k <= 0) return XB_ERR_BAD_SIZE;
+  return norm_rows_fit(rows, n, k) ? XB_OK : XB_ERR_UNSUPPORTED_SHAPE;
+}
+
+extern "C" int xb_norm_linear(const float* residual, const void* update, const float* gamma, const float* beta,
+                              float eps, int apply_affine, float* residual_out, const void* w, const float* bias,
+                              void* c, int64_t rows, int32_t n, int32_t k, int epilogue, void* k_cache, void* v_cache,
+                              int32_t heads, int64_t chunk, int64_t start, int64_t capacity, void* stream) {
+  if (rows < 0 || n <= 0 || k <= 0) return XB_ERR_BAD_SIZE;
+  if (epilogue != XB_EPI_BIAS && epilogue != XB_EPI_BIAS_GELU) return XB_ERR_BAD_EPILOGUE;
+  if (!norm_rows_fit(rows, n, k)) return XB_ERR_UNSUPPORTED_SHAPE;
+  const bool caches = k_cache != nullptr || v_cache != nullptr;
+  if (caches) {
+    if (n != 3 * k || heads <= 0 || k % heads != 0 || (k / heads) % 8 != 0) return XB_ERR_UNSUPPORTED_SHAPE;
+    if (chunk <= 0 || rows % chunk != 0 || start < 0 || start + chunk > capacity) return XB_ERR_BAD_SIZE;
+  }
+  if (rows == 0) return XB_OK;
+  if (!residual || !w || !c || (apply_affine && (!gamma || !beta))) return XB_ERR_NULL_POINTER;
+  if (caches && (!k_cache || !v_cache)) return XB_ERR_NULL_POINTER;
+  if (residual_out == residual) return XB_ERR_BAD_SIZE;  // other blocks still read it
+  uintptr_t all = (uintptr_t)residual | (uintptr_t)update | (uintptr_t)residual_out | (uintptr_t)w | (uintptr_t)c |
+                  (uintptr_t)k_cache | (uintptr_t)v_cache;
+  if (apply_affine) all |= (uintptr_t)gamma | (uintptr_t)beta;
+  if (all & 15u) return XB_ERR_MISALIGNED;
+  const RowsExtra ex{residual, static_cast<const half_t*>(update), gamma, beta, residual_out, eps, apply_affine,
+                     static_cast<half_t*>(k_cache), static_cast<half_t*>(v_cache), heads,
+                     caches ? k / heads : 0, caches ? (int)chunk : 1, start, capacity};
+  const half_t* Wt = static_cast<const half_t*>(w);
+  half_t* Cc = static_cast<half_t*>(c);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  return (int)(epilogue == XB_EPI_BIAS_GELU
+      ? launch_norm_rows<XB_EPI_BIAS_GELU>(ex, Wt, bias, Cc, (int)rows, n, k, s)
+      : launch_norm_rows<XB_EPI_BIAS>(ex, Wt, bias, Cc, (int)rows, n, k, s));
 }

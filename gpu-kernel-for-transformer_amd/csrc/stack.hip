@@ -19,8 +19,14 @@ namespace xb {
 // Byte offsets of the intermediates, each from a 256-byte boundary.  hidden
 // (the FFN activation) takes the place of qkv and ctx, which are dead by then.
 struct StackLayout {
-  int64_t residual, norm, update, qkv, ctx, hidden, vt, decode, bytes;
+  int64_t residual, residual2, norm, update, qkv, ctx, hidden, vt, decode, bytes;
 };
+
+// A few rows (decode steps): LayerNorm in the prologue of the product that
+// follows it (xb_norm_linear), which needs a second residual buffer.
+static bool norm_in_products(int64_t rows, int d, int ffn) {
+  return xb_select_norm_linear(rows, 3 * d, d) == XB_OK && xb_select_norm_linear(rows, ffn, d) == XB_OK;
+}
 
 static int64_t aligned_up(int64_t n) { return (n + 255) / 256 * 256; }
 
@@ -38,6 +44,7 @@ static int stack_layout(int32_t batch, int64_t seq_len, int32_t heads, int32_t h
     return p;
   };
   l.residual = take(rows * d * 4);
+  l.residual2 = take(norm_in_products(rows, (int)d, ffn_dim) ? rows * d * 4 : 0);
   l.norm = take(rows * d * 2);
   l.update = take(rows * d * 2);
   l.qkv = take(rows * 3 * d * 2);
@@ -95,12 +102,13 @@ extern "C" int xb_stack_forward(const xb_stack* st, const float* x, float* y, co
   const xb_block* b = st->blocks;
   bool row_blocks = true;
   for (int i = 0; i < st->layers; ++i) row_blocks = row_blocks && b[i].packed != nullptr;
-  // Append and attend: layer i's context from qkv.
-  auto attend = [&](int i) -> int {
+  // Append (unless the projection did) and attend: layer i's context from qkv.
+  auto attend = [&](int i, bool appended) -> int {
     const float scale = st->blocks[i].scale;
     if (cached) {
-      const int bad = xb_kv_cache_append(qkv, caches[2 * i], caches[2 * i + 1], batch, seq_len, heads, hd, cache_start,
-                                         cache_capacity, stream);
+      const int bad = appended ? XB_OK
+                               : xb_kv_cache_append(qkv, caches[2 * i], caches[2 * i + 1], batch, seq_len, heads, hd,
+                                                    cache_start, cache_capacity, stream);
       if (bad) return bad;
       if (cache_start > 0)
         return xb_attention_kv_cache(qkv, caches[2 * i], caches[2 * i + 1], ctx, batch, seq_len, heads, hd,
@@ -115,11 +123,38 @@ extern "C" int xb_stack_forward(const xb_stack* st, const float* x, float* y, co
     const float* in = x;
     e = xb_row_block(st, -1, x, nullptr, nullptr, qkv, nullptr, nullptr, rows, stream);
     for (int i = 0; i < st->layers && !e; ++i) {
-      e = attend(i);
+      e = attend(i, false);
       if (!e) e = xb_row_block(st, i, in, ctx, streams[i & 1], qkv, y, token_valid, rows, stream);
       in = streams[i & 1];
     }
     return e;
+  }
+  // The few-row kernel gives the bits of every tile, but only AUTO or its own
+  // variant asks for it.
+  auto any = [](int v) { return v == XB_VARIANT_AUTO || v == XB_LINEAR_ROWS; };
+  if (norm_in_products(rows, d, f) && any(qkv_variant) && any(ffn_in_variant) && !transposed_v) {
+    float* streams[2] = {residual, reinterpret_cast<float*>(ws + l.residual2)};
+    const float* in = x;
+    const void* upd = nullptr;
+    for (int i = 0; i < st->layers && !e; ++i, ++b) {
+      // x + update of the layer before (layer 0: x itself) -> streams[0]; then + the attention's -> streams[1].
+      e = xb_norm_linear(in, upd, b->norm1_g, b->norm1_b, b->norm1_eps, b->norm1_affine, upd ? streams[0] : nullptr,
+                         b->qkv_w, b->qkv_b, qkv, rows, 3 * d, d, XB_EPI_BIAS, cached ? caches[2 * i] : nullptr,
+                         cached ? caches[2 * i + 1] : nullptr, heads, seq_len, cache_start, cache_capacity, stream);
+      if (upd) in = streams[0];
+      if (!e) e = attend(i, cached);
+      if (!e) e = xb_linear_v(ctx, b->out_w, b->out_b, update, rows, d, d, XB_EPI_BIAS, out_variant, stream);
+      if (!e)
+        e = xb_norm_linear(in, update, b->norm2_g, b->norm2_b, b->norm2_eps, b->norm2_affine, streams[1], b->ffn_in_w,
+                           b->ffn_in_b, hidden, rows, f, d, XB_EPI_BIAS_GELU, nullptr, nullptr, 0, 1, 0, 0, stream);
+      in = streams[1];
+      if (!e) e = xb_linear_v(hidden, b->ffn_out_w, b->ffn_out_b, update, rows, d, f, XB_EPI_BIAS, ffn_out_variant, stream);
+      upd = update;
+    }
+    if (e) return e;
+    return xb_residual_layernorm_masked(in, update, XB_F16, st->final_g, st->final_b, nullptr, y, XB_F32, rows, d,
+                                        st->final_eps, st->final_affine, token_valid,
+                                        token_valid ? XB_MASK_OUTPUT : 0, stream);
   }
   e = xb_layernorm(x, b->norm1_g, b->norm1_b, norm, XB_F16, rows, d, b->norm1_eps, b->norm1_affine, stream);
   const float* res_in = x;
@@ -129,7 +164,7 @@ extern "C" int xb_stack_forward(const xb_stack* st, const float* x, float* y, co
       if (!e) e = xb_attention_causal_vt(qkv, vt, ctx, batch, seq_len, heads, hd, b->scale, stream);
     } else {
       e = xb_linear_v(norm, b->qkv_w, b->qkv_b, qkv, rows, 3 * d, d, XB_EPI_BIAS, qkv_variant, stream);
-      if (!e) e = attend(i);
+      if (!e) e = attend(i, false);
     }
     if (!e) e = xb_linear_v(ctx, b->out_w, b->out_b, update, rows, d, d, XB_EPI_BIAS, out_variant, stream);
     if (!e)

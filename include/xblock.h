@@ -418,6 +418,23 @@ typedef struct xb_stack {
 } xb_stack;
 
 /*
+ * A few rows' LayerNorm and the product after it in one kernel
+ * (xb_select_norm_linear: XB_OK for up to 8 rows, n % 16 == 0 and k 512, 768,
+ * 1024 or 2048): s = residual + update (update NULL: residual), c[rows, n] =
+ * epilogue(LN(s) . w^T + bias), residual_out = s unless NULL (it may not be
+ * `residual`).  Same bits as xb_layernorm / xb_residual_layernorm followed by
+ * xb_linear.  k_cache and v_cache (NULL: none; n == 3k, rows = batch * chunk)
+ * receive the K and V columns as xb_kv_cache_append would write them.
+ */
+int xb_select_norm_linear(int64_t rows, int32_t n, int32_t k);
+int xb_norm_linear(const float* residual, const void* update, const float* gamma,
+                   const float* beta, float eps, int apply_affine,
+                   float* residual_out, const void* w, const float* bias,
+                   void* c, int64_t rows, int32_t n, int32_t k, int epilogue,
+                   void* k_cache, void* v_cache, int32_t heads, int64_t chunk,
+                   int64_t start, int64_t capacity, void* stream);
+
+/*
  * Everything between two attentions of a narrow model in one kernel
  * (xb_select_row_block: XB_OK for d_model 32, 64 or 128 with ffn_dim a multiple
  * of it, up to 4 times, at 128 up to 8 times).  layer -1: qkv = the packed QKV

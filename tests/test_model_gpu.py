@@ -810,19 +810,27 @@ def test_native_sequence_is_the_stepwise_one(pkg, cuda, geom, causal, padded):
     assert not torch.equal(first, second) and not torch.equal(second, third)
 
 
-@pytest.mark.parametrize("prompt,chunks", [(1, (1, 1)), (40, (1, 16, 17, 1)), (0, (5, 1))])
-def test_native_sequence_with_kv_cache(pkg, cuda, prompt, chunks):
-    """KV-cached steps: native and stepwise issue give the same outputs and caches."""
+@pytest.mark.parametrize("prompt,chunks", [(1, (1, 1)), (40, (1, 16, 17, 1)), (0, (5, 1)), (2, (2, 1))])
+@pytest.mark.parametrize("d,heads,ffn", [(256, 4, 512), (512, 8, 528), (768, 12, 768), (1024, 4, 1024), (2048, 16, 2048)])
+def test_native_sequence_with_kv_cache(pkg, cuda, prompt, chunks, d, heads, ffn):
+    """KV-cached steps: native and stepwise issue give the same outputs and
+    caches, also where a step's few rows take their LayerNorms and the cache
+    append into the products."""
     steps = [c for c in (prompt, *chunks) if c]
-    config = pkg.TransformerConfig(3, sum(steps) + 2, 256, 4, 512, 2, True)
+    config = pkg.TransformerConfig(3, sum(steps) + 2, d, heads, ffn, 2, True)
     torch.manual_seed(7)
     models = [pkg.UserOptimizedTransformer(config).to(cuda).eval() for _ in range(2)]
+    with torch.no_grad():
+        for i, norm in enumerate(m for m in models[0].modules() if isinstance(m, torch.nn.LayerNorm)):
+            if i % 2 == 0:   # affine and identity LayerNorms
+                norm.weight.add_(0.1 * torch.randn(d, device=cuda))
+                norm.bias.add_(0.1 * torch.randn(d, device=cuda))
     models[1].load_state_dict(models[0].state_dict())
     for m in models:
         m.enable_kv_cache(True)
     models[1]._native_stack = lambda row_block: None
     for i, c in enumerate(steps):
-        x = torch.randn(3, c, 256, generator=torch.Generator().manual_seed(i)).to(cuda)
+        x = torch.randn(3, c, d, generator=torch.Generator().manual_seed(i)).to(cuda)
         with torch.no_grad():
             assert torch.equal(models[0](x), models[1](x)), (i, c)
     used = sum(steps)
