@@ -501,7 +501,9 @@ class UserOptimizedTransformer(nn.Module):
             if valid_token_mask.dtype not in (torch.bool, torch.uint8):
                 raise ValueError("valid_token_mask must be bool or uint8")
             if x.numel() and not self._all_tokens_valid(valid_token_mask, x.shape[1]):
-                token_valid = (valid_token_mask != 0).to(torch.uint8).contiguous()
+                # Every kernel tests the mask's bytes against zero, so a bool mask is read
+                # as it is: converting it first took two launches, 11 us of a 51 us forward.
+                token_valid = valid_token_mask.contiguous().view(torch.uint8)
         if x.numel() == 0:  # no sequence or no token: an empty result, nothing launched, no cache change
             return torch.empty_like(x) if out is None else out
         x = x.contiguous()

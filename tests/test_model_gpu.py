@@ -880,3 +880,22 @@ def test_row_blocks(pkg, cuda, geom, causal, padded):
         assert float((out - per_op).abs().max()) < 2e-2 and float((out - per_op).norm() / per_op.norm()) < 1e-3
         alone = model._per_op_forward(xg[:1].contiguous(), plan, token_valid=None if valid is None else valid[:1].contiguous())
         assert torch.equal(alone, out[:1])
+
+
+@pytest.mark.parametrize("geom", [(3, 60, 128, 4, 128, 2), (3, 60, 64, 4, 64, 2), (3, 60, 256, 4, 256, 1)])
+def test_mask_forms_agree(pkg, cuda, geom):
+    """A padding mask is read as its bytes: bool, uint8 with any nonzero value and
+    strided masks give the same output, in the one-launch, row-block and per-op forms."""
+    config = pkg.TransformerConfig(*geom, True)
+    torch.manual_seed(3)
+    model = pkg.UserOptimizedTransformer(config).to(cuda).eval()
+    x = torch.randn(*geom[:3], generator=torch.Generator().manual_seed(4)).to(cuda)
+    mask = (torch.rand(geom[0], geom[1], generator=torch.Generator().manual_seed(5)) > 0.3).to(cuda)
+    mask[:, 0] = True
+    with torch.inference_mode():
+        out = model(x, mask)
+        assert torch.equal(out, model(x, mask.to(torch.uint8)))
+        assert torch.equal(out, model(x, mask.to(torch.uint8) * 200))
+        assert torch.equal(out, model(x, mask.t().contiguous().t()))
+        assert torch.equal(out, model(x, torch.stack((mask, ~mask), -1)[..., 0]))
+        assert not bool(out[~mask].any())
