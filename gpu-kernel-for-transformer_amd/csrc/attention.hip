@@ -105,8 +105,13 @@ __device__ __forceinline__ half4_t lds_read_tr16(const half_t* p) {
 // attn_split_combine; that is the decode path, which needs the whole GPU on
 // the key axis.  Without KEYMASK or SPLIT every query sees key 0 in the first
 // tile, which keeps the offset bookkeeping to a tile-index test.
-template <int HD, int NQ, int NW, bool CAUSAL, bool KEYMASK, bool SPLIT>
-__global__ __launch_bounds__(64 * NW, 8 / NW) void attn_kernel(const AttnArgs a) {
+//
+// KW > 1 (decode): KW waves, each with its own key range and LDS tile and no
+// barrier between them; their partials are merged in LDS, so the block leaves
+// one partial for KW ranges, or, when it covers all keys, the result itself
+// without the merge kernel.
+template <int HD, int NQ, int NW, bool CAUSAL, bool KEYMASK, bool SPLIT, int KW = 1>
+__global__ __launch_bounds__(64 * NW * KW, 8 / (NW * KW)) void attn_kernel(const AttnArgs a) {
   using C = AttnCfg<HD, NQ, NW>;
   constexpr int NT = C::NT, BKEYS = C::BKEYS, HDP = C::HDP, HDV = C::HDV, QPW = C::QPW, BQ = C::BQ;
   constexpr int LDK = C::LDK, LDV = C::LDV, KSTEPS = C::KSTEPS, KB = C::KB, HB = C::HB;
@@ -118,9 +123,10 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_kernel(const AttnArgs a)
   constexpr int NBUF = DECODE ? 1 : 2;
   constexpr int AHEAD = DECODE || HD >= 256 || NQ > 2 ? 1 : 2;
   static_assert(NT >= BKEYS, "one thread per key stages the validity bytes");
+  static_assert(KW == 1 || DECODE, "several key ranges per block: decode only");
 
-  __shared__ __attribute__((aligned(16))) half_t k_lds[NBUF][BKEYS * LDK];
-  __shared__ __attribute__((aligned(16))) half_t v_lds[NBUF][BKEYS * LDV];
+  __shared__ __attribute__((aligned(16))) half_t k_lds[KW * NBUF][BKEYS * LDK];
+  __shared__ __attribute__((aligned(16))) half_t v_lds[KW * NBUF][BKEYS * LDV];
   __shared__ __attribute__((aligned(16))) uint8_t kv_lds[NBUF][BKEYS];  // key validity of the tile
 
   // Heaviest query tiles (most keys under the causal mask) are issued first;
@@ -142,22 +148,33 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_kernel(const AttnArgs a)
   const half_t* vbase = a.v + (int64_t)b * a.k_bstride + (int64_t)h * a.k_hstride;
   const float scale_log2 = a.scale_log2;
 
-  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+  const int kw = KW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) : 0;  // this wave's key range
+  const int tid = KW > 1 ? threadIdx.x % kWave : threadIdx.x, wave = tid / kWave, lane = tid % kWave;
   const int g = lane / 16, r16 = lane % 16;
   const int q0 = qt * BQ;
   const int qw0 = q0 + wave * QPW;
+  // Orders the tile's LDS writes and reads: within a wave they run in order.
+  auto tile_sync = [] {
+    if constexpr (KW > 1) {
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_wave_barrier();
+      asm volatile("" ::: "memory");
+    } else {
+      __syncthreads();
+    }
+  };
 
   // Zero the padding columns of both buffers once; tile stores never touch them.
   if constexpr (HDP > HD) {
     for (int i = tid; i < NBUF * BKEYS * (HDP - HD); i += NT) {
       const int buf = i / (BKEYS * (HDP - HD)), j = i % (BKEYS * (HDP - HD));
-      k_lds[buf][(j / (HDP - HD)) * LDK + HD + j % (HDP - HD)] = (half_t)0.f;
+      k_lds[kw * NBUF + buf][(j / (HDP - HD)) * LDK + HD + j % (HDP - HD)] = (half_t)0.f;
     }
   }
   if constexpr (HDV > HD) {
     for (int i = tid; i < NBUF * BKEYS * (HDV - HD); i += NT) {
       const int buf = i / (BKEYS * (HDV - HD)), j = i % (BKEYS * (HDV - HD));
-      v_lds[buf][(j / (HDV - HD)) * LDV + HD + j % (HDV - HD)] = (half_t)0.f;
+      v_lds[kw * NBUF + buf][(j / (HDV - HD)) * LDV + HD + j % (HDV - HD)] = (half_t)0.f;
     }
   }
 
@@ -197,7 +214,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_kernel(const AttnArgs a)
   }
   const half8_t ones8 = {1, 1, 1, 1, 1, 1, 1, 1};
 
-  const int k_begin = SPLIT ? split * a.split_keys : 0;
+  const int k_begin = SPLIT ? (split * KW + kw) * a.split_keys : 0;
   int key_end = CAUSAL ? min(S_k, q_offset + q0 + BQ) : S_k;
   if constexpr (SPLIT) key_end = min(key_end, k_begin + a.split_keys);
   const int n_tiles = key_end > k_begin ? (key_end - k_begin + BKEYS - 1) / BKEYS : 0;
@@ -248,8 +265,8 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_kernel(const AttnArgs a)
       const int id = tid + NT * j;
       if (id < BKEYS * CPK) {
         const int r = id / CPK, c = (id % CPK) * 8;
-        *reinterpret_cast<half8_t*>(&k_lds[buf][r * LDK + c]) = kreg[R][j];
-        *reinterpret_cast<half8_t*>(&v_lds[buf][r * LDV + c]) = vreg[R][j];
+        *reinterpret_cast<half8_t*>(&k_lds[kw * NBUF + buf][r * LDK + c]) = kreg[R][j];
+        *reinterpret_cast<half8_t*>(&v_lds[kw * NBUF + buf][r * LDV + c]) = vreg[R][j];
       }
     }
   };
@@ -270,10 +287,10 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_kernel(const AttnArgs a)
       for (int m = 0; m < 8; ++m) v[m] = (half_t)((float)v[m] * scale_log2);
       qf[qb][ks] = q_ok(qb, ks) ? v : zero8;
     }
-  __syncthreads();
+  tile_sync();
   // Tile t; register set `free` held it and takes tile t + AHEAD, set `next` holds tile t + 1 by its end.
   auto step = [&](int t, auto free, auto next) {
-    const int cur = NBUF == 1 ? 0 : t & 1;
+    const int cur = NBUF == 1 ? kw : t & 1;
     const int k0 = k_begin + t * BKEYS;
     gload(t + AHEAD, free);
 
@@ -399,9 +416,9 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_kernel(const AttnArgs a)
     }
 
     __builtin_amdgcn_s_setprio(0);
-    if constexpr (NBUF == 1) __syncthreads();  // the tile is read completely before it is replaced
+    if constexpr (NBUF == 1) tile_sync();  // the tile is read completely before it is replaced
     sstore(NBUF == 1 ? 0 : cur ^ 1, next);
-    __syncthreads();
+    tile_sync();
   };
   if constexpr (AHEAD == 2) {
     for (int t = 0; t < n_tiles; t += 2) {
@@ -410,6 +427,55 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_kernel(const AttnArgs a)
     }
   } else {
     for (int t = 0; t < n_tiles; ++t) step(t, kSet0, kSet0);
+  }
+
+  if constexpr (KW > 1) {
+    static_assert(NQ == 1, "one block of 16 queries");
+    // Merge: (m, l) of every range, then each wave's o scaled onto the common
+    // offset, [KW][16][HD + 4] floats in the freed tiles.
+    constexpr int LDM = HD + 4;
+    static_assert(KW * 16 * LDM * 4 <= KW * NBUF * BKEYS * LDK * 2, "the partials fit in the K tiles");
+    __shared__ float2 ml[KW][16];
+    if (g == 0) ml[kw][r16] = make_float2(m_set[0] ? m_run[0] : -INFINITY, lacc[0][0]);
+    __syncthreads();
+    float m = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < KW; ++w) m = fmaxf(m, ml[w][r16].x);
+    const float m0 = m == -INFINITY ? 0.f : m;
+    const float scale = __builtin_amdgcn_exp2f(ml[kw][r16].x - m0);
+    float* const po = reinterpret_cast<float*>(&k_lds[0][0]);
+#pragma unroll
+    for (int hb = 0; hb < HB; ++hb) {
+      const int d = 16 * hb + 4 * g;
+      if (d < HD) *reinterpret_cast<float4_t*>(po + (kw * 16 + r16) * LDM + d) = o[hb][0] * scale;
+    }
+    __syncthreads();
+    const int64_t slot = (int64_t)bh * a.n_splits + split;
+    for (int e = threadIdx.x; e < S_q * (HD / 4); e += 64 * KW) {
+      const int q = e / (HD / 4), d = 4 * (e % (HD / 4));
+      float mq = -INFINITY;
+#pragma unroll
+      for (int w = 0; w < KW; ++w) mq = fmaxf(mq, ml[w][q].x);
+      const float base_m = mq == -INFINITY ? 0.f : mq;
+      float l = 0.f;
+      float4_t sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < KW; ++w) {
+        l = fmaf(__builtin_amdgcn_exp2f(ml[w][q].x - base_m), ml[w][q].y, l);
+        sum += *reinterpret_cast<const float4_t*>(po + (w * 16 + q) * LDM + d);
+      }
+      if (a.n_splits == 1) {
+        const float inv = l > 0.f ? 1.f / l : 0.f;
+        half4_t r;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = (half_t)(sum[i] * inv);
+        *reinterpret_cast<half4_t*>(a.out + (int64_t)b * a.o_bstride + (int64_t)q * a.o_rstride + (int64_t)h * HD + d) = r;
+      } else {
+        *reinterpret_cast<float4_t*>(a.ws_o + (slot * a.ws_rows + q) * HD + d) = sum;
+        if (d == 0) a.ws_ml[slot * a.ws_rows + q] = make_float2(mq, l);
+      }
+    }
+    return;
   }
 
   if constexpr (SPLIT) {
@@ -987,6 +1053,7 @@ constexpr int64_t kDecodeTargetBlocks = 2048;
 
 struct SplitGeometry {
   int n_splits, split_keys, rows;  // rows: partial rows per (batch, head, split)
+  int per_block;                   // key ranges one block merges before it writes a partial
   int64_t o_bytes, bytes;          // partial o, then (offset, sum) pairs; 0 bytes: no split
 };
 
@@ -1004,6 +1071,13 @@ static int64_t split_partial_bytes(int64_t rows, int HD) {
 // three per CU) over at least kChunkMinTiles key tiles per split; 0 bytes
 // otherwise.  B = 1, 16 heads of 64: 100 tokens over a cache of 50,000 789 -> 54
 // us, 512 over 8,000 139 -> 50 us.
+//
+// Decode blocks of four waves merge four ranges in LDS: a quarter of the
+// partials, and where one block covers a (batch, head) -- four ranges or fewer
+// are wanted, or the cache is at most kOneBlockTiles key tiles long, which its
+// waves walk in three or fewer steps -- no merge launch at all (B = 4, 16
+// heads of 64, 517 keys 9.7 -> 7.8 us, B = 32, 501 keys 17.0 -> 12.8 us).
+constexpr int kDecodeWaves = 4, kOneBlockTiles = 12;
 constexpr int64_t kChunkTargetBlocks = 768;
 constexpr int kChunkMinTiles = 8;
 static SplitGeometry split_geometry(int B, int H, int64_t chunk, int S_k, int HD) {
@@ -1023,7 +1097,16 @@ static SplitGeometry split_geometry(int B, int H, int64_t chunk, int S_k, int HD
   const int tiles_per = (int)((tiles + want - 1) / want);
   g.split_keys = tiles_per * bk;
   g.n_splits = (S_k + g.split_keys - 1) / g.split_keys;
-  const int64_t slots = bh * g.n_splits * g.rows;
+  g.per_block = 1;
+  if (decode && tiles > 1) {
+    if (tiles <= kOneBlockTiles) {
+      g.split_keys = (tiles + kDecodeWaves - 1) / kDecodeWaves * bk;
+      g.per_block = kDecodeWaves;
+    } else if (g.n_splits >= 3) {
+      g.per_block = kDecodeWaves;
+    }
+  }
+  const int64_t slots = bh * g.n_splits * g.rows;  // room for a partial per range
   g.o_bytes = slots * HD * (int64_t)sizeof(float);
   g.bytes = g.o_bytes + slots * (int64_t)sizeof(float2);
   return g;
@@ -1033,19 +1116,24 @@ template <int HD>
 static hipError_t launch_split(AttnArgs a, int B, const SplitGeometry& geo, void* workspace, hipStream_t s) {
   static_assert(AttnCfg<HD, 1, 1>::BQ == kDecodeQueries && AttnCfg<HD, 1>::BQ == 64, "queries per block");
   const bool decode = a.S_q <= kDecodeQueries;
-  a.n_splits = geo.n_splits;
+  const int64_t keys_per_block = (int64_t)geo.split_keys * geo.per_block;
+  a.n_splits = (int)((a.S_k + keys_per_block - 1) / keys_per_block);  // <= geo.n_splits, which the workspace is sized for
   a.split_keys = geo.split_keys;
   a.ws_rows = geo.rows;
   a.q_tiles = decode ? 1 : (a.S_q + 63) / 64;
   a.ws_o = static_cast<float*>(workspace);
   a.ws_ml = reinterpret_cast<float2*>(static_cast<char*>(workspace) + geo.o_bytes);
-  const int64_t blocks = (int64_t)B * a.H * geo.n_splits * a.q_tiles;
+  const int64_t blocks = (int64_t)B * a.H * a.n_splits * a.q_tiles;
   const int64_t queries = (int64_t)B * a.H * a.S_q;
   if (blocks > 0x7fffffffLL || queries > 0x7fffffffLL) return hipErrorInvalidValue;
-  if (decode)
+  if (geo.per_block == kDecodeWaves)
+    hipLaunchKernelGGL((attn_kernel<HD, 1, 1, true, false, true, kDecodeWaves>), dim3((unsigned)blocks),
+                       dim3(64 * kDecodeWaves), 0, s, a);
+  else if (decode)
     hipLaunchKernelGGL((attn_kernel<HD, 1, 1, true, false, true>), dim3((unsigned)blocks), dim3(64), 0, s, a);
   else
     hipLaunchKernelGGL((attn_kernel<HD, 1, 4, true, false, true>), dim3((unsigned)blocks), dim3(256), 0, s, a);
+  if (geo.per_block == kDecodeWaves && a.n_splits == 1) return hipGetLastError();  // merged by its block
   hipLaunchKernelGGL((attn_split_combine<HD>), dim3((unsigned)queries), dim3(256), 0, s, a);
   return hipGetLastError();
 }
