@@ -132,7 +132,14 @@ extern "C" int xb_stack_forward(const xb_stack* st, const float* x, float* y, co
   // The few-row kernel gives the bits of every tile, but only AUTO or its own
   // variant asks for it.
   auto any = [](int v) { return v == XB_VARIANT_AUTO || v == XB_LINEAR_ROWS; };
-  if (norm_in_products(rows, d, f) && any(qkv_variant) && any(ffn_in_variant) && !transposed_v) {
+  // Nor does it take the unaligned inputs that some widths' LayerNorms do.
+  uintptr_t vectors = (uintptr_t)x;
+  for (int i = 0; i < st->layers; ++i) {
+    if (b[i].norm1_affine) vectors |= (uintptr_t)b[i].norm1_g | (uintptr_t)b[i].norm1_b;
+    if (b[i].norm2_affine) vectors |= (uintptr_t)b[i].norm2_g | (uintptr_t)b[i].norm2_b;
+  }
+  const bool aligned = (vectors & 15u) == 0;
+  if (aligned && norm_in_products(rows, d, f) && any(qkv_variant) && any(ffn_in_variant) && !transposed_v) {
     float* streams[2] = {residual, reinterpret_cast<float*>(ws + l.residual2)};
     const float* in = x;
     const void* upd = nullptr;

@@ -547,7 +547,9 @@ class UserOptimizedTransformer(nn.Module):
                                               split=plan.fused_variant == _capi.XB_FUSED_SPLIT,
                                               strict=self._strict_handoff_checks)
 
-        streams = self._overlap_streams(x)
+        # Not for row blocks: nine short launches gain nothing from running beside nine more
+        # (64 x 128 tokens of width 32: 47 us in one stream, 82 us in two).
+        streams = None if plan.row_block else self._overlap_streams(x)
         if streams is not None and torch.cuda.is_current_stream_capturing():
             return self._per_op_forward_overlapped(x, plan, streams, out, token_valid)
         return self._per_op_forward(x, plan, out=out, token_valid=token_valid)
@@ -592,7 +594,8 @@ class UserOptimizedTransformer(nn.Module):
         the FFN (see _OVERLAP_MAX_TOKENS); this names them.
         """
         plan = self.execution_plan(batch, seq_len, padded=padded)
-        if plan.fused or batch < 2 or batch * seq_len > self._OVERLAP_MAX_TOKENS or self._kv_cache_enabled:
+        if (plan.fused or plan.row_block or batch < 2 or batch * seq_len > self._OVERLAP_MAX_TOKENS
+                or self._kv_cache_enabled):
             return None
         halves = sorted({(batch + 1) // 2, batch // 2}, reverse=True)
         own = [self.execution_plan(h, seq_len, padded=padded, per_op=True) for h in halves]
@@ -659,6 +662,8 @@ class UserOptimizedTransformer(nn.Module):
         While a LaunchRecorder is active the same launches go through the
         wrappers one by one, so that each is bracketed by its events.
         """
+        if plan.row_block and self.config.d_model == 32 and x.data_ptr() % 16:
+            x = x.clone()  # this width's LayerNorm takes any alignment, the row blocks 16 bytes
         native = None if kernels.recording() else self._native_stack(plan.row_block)
         if native is None:
             return self._per_op_forward_stepwise(x, plan, out, token_valid, cache_start)

@@ -899,3 +899,32 @@ def test_mask_forms_agree(pkg, cuda, geom):
         assert torch.equal(out, model(x, mask.t().contiguous().t()))
         assert torch.equal(out, model(x, torch.stack((mask, ~mask), -1)[..., 0]))
         assert not bool(out[~mask].any())
+
+
+@pytest.mark.parametrize("geom", [(2, 9, 32, 4, 32, 2), (1, 3, 768, 12, 768, 2), (2, 40, 768, 12, 768, 1)])
+def test_unaligned_input_and_norms(pkg, cuda, geom):
+    """Widths whose LayerNorm never asked for 16-byte alignment still take inputs and
+    LayerNorm parameters that start anywhere."""
+    config = pkg.TransformerConfig(*geom, True)
+    torch.manual_seed(9)
+    model = pkg.UserOptimizedTransformer(config).to(cuda).eval()
+    d = geom[2]
+
+    def off_by_one(t):
+        flat = torch.empty(t.numel() + 4, device=cuda)[1:1 + t.numel()]
+        return flat.copy_(t.flatten()).view(t.shape)
+
+    with torch.no_grad():
+        model.layers[0].norm2.weight.add_(0.25)
+        x = torch.randn(*geom[:3], device=cuda)
+        ref = model(x)
+        shifted = off_by_one(x)
+        assert shifted.data_ptr() % 16 and shifted.is_contiguous()
+        out = model(shifted)
+        torch.testing.assert_close(out, ref, atol=2e-2, rtol=0)
+        assert float((out - ref).norm() / ref.norm()) < 1e-3
+        for norm in (model.layers[0].norm1, model.layers[0].norm2):
+            norm.weight.data = off_by_one(norm.weight.data)
+            norm.bias.data = off_by_one(norm.bias.data)
+        out = model(x)
+        assert float((out - ref).norm() / ref.norm()) < 1e-3
