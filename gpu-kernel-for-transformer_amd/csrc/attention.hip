@@ -1005,7 +1005,8 @@ static bool attention_variant_fits(int variant, int hd, bool masked) {
 // heads 20.1 / 24.3 / 36.6; 1 x 4000 x 16 79.6 / 85.4 / 117; 2 x 2907 x 16
 // 64.6 / 61.6 / 78.3; 8 x 2048 x 16 145 / 125 / 153; 8 x 4096 x 16 - / 347 /
 // 344; 1 x 16384 x 16 751 / 601 / 534; head_dim 128, 3 x 446 x 8 10.9 / 14.8,
-// 16 x 1024 x 8 76.8 / 69.1.  So 16 up to 640 blocks of 128 queries, 64 from
+// 16 x 1024 x 8 76.8 / 69.1; 56 x 47 x 16 6.6 / 8.7 (half of each block idle).
+// So 16 up to 64 queries or 640 blocks of 128 queries, 64 from
 // 16384 queries or 2048 blocks of at least 4096 queries on.  The ping-pong
 // kernel (head_dim 64, no key mask) is ahead from 16384 queries on (1 x 16384
 // x 16 530 us, 1 x 32768 x 16 2025 against 2073) and behind below (8 x 4096 x
@@ -1016,7 +1017,7 @@ static bool attention_variant_fits(int variant, int hd, bool masked) {
 static int select_attention(int64_t B, int S_q, int H, int hd, bool masked) {
   if (hd >= 256) return S_q <= 128 && B * H >= kCUs ? XB_ATTN_W8_Q16 : XB_ATTN_W4_Q16;
   if (hd == 64 && !masked && (S_q >= 16384 || (S_q > 4096 && B * H >= 32))) return XB_ATTN_PINGPONG;
-  if ((S_q + 127) / 128 * B * H <= 640) return XB_ATTN_W4_Q16;
+  if (S_q <= 64 || (S_q + 127) / 128 * B * H <= 640) return XB_ATTN_W4_Q16;
   if (hd >= 128) return XB_ATTN_W4_Q32;
   const bool many = S_q >= 16384 || (S_q >= 4096 && (S_q + 255) / 256 * B * H >= 2048);
   return many ? XB_ATTN_W4_Q64 : XB_ATTN_W4_Q32;
