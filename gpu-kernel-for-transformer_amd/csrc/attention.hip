@@ -362,7 +362,7 @@ __global__ __launch_bounds__(64 * NW * KW, 8 / (NW * KW)) void attn_kernel(const
         for (int jb = 0; jb < KB; ++jb)
           lm = fmaxf(lm, fmaxf(fmaxf(s[jb][qb][0], s[jb][qb][1]), fmaxf(s[jb][qb][2], s[jb][qb][3])));
       }
-      if (__any(unset || lm > 8.0f)) {
+      if (DECODE || __any(unset || lm > 8.0f)) {
 #pragma unroll
         for (int qb = 0; qb < NQ; ++qb) {
           float m = -INFINITY;
@@ -371,13 +371,19 @@ __global__ __launch_bounds__(64 * NW * KW, 8 / (NW * KW)) void attn_kernel(const
             m = fmaxf(m, fmaxf(fmaxf(s[jb][qb][0], s[jb][qb][1]), fmaxf(s[jb][qb][2], s[jb][qb][3])));
           // Decided per block of 16 queries, not per wave: a query's result then
           // does not depend on how many blocks its wave holds.
-          if (!__any((TRACK ? !m_set[qb] : t == 0) || m > 8.0f)) continue;
+          if (!DECODE && !__any((TRACK ? !m_set[qb] : t == 0) || m > 8.0f)) continue;
           const float mx = quad_group_max(m);
           // Until a query has seen a key its o and lacc are exactly zero: the
           // offset jumps to the first finite maximum and nothing is rescaled
           // (exp2(-sh) could overflow there).  Afterwards sh >= 0, corr <= 1.
           const bool was_set = TRACK ? m_set[qb] : t != 0;
-          const float sh = was_set ? fmaxf(mx, 0.f) : (TRACK && mx == -INFINITY ? 0.f : mx);
+          // Decode moves the offset onto every tile's own maximum, up or down (by
+          // at most 2^60, o stays FP32): the largest probability of each tile is
+          // then exactly 1 whatever the number of tiles in a range, and the cost
+          // is nothing next to the cache's bytes.
+          const float sh = !was_set ? (TRACK && mx == -INFINITY ? 0.f : mx)
+                           : !DECODE ? fmaxf(mx, 0.f)
+                           : mx == -INFINITY ? 0.f : fmaxf(mx, -60.f);
           if constexpr (TRACK) m_set[qb] = was_set || mx != -INFINITY;
           const float corr = was_set ? __builtin_amdgcn_exp2f(-sh) : 1.f;
           m_run[qb] += sh;
@@ -1006,7 +1012,12 @@ static bool attention_variant_fits(int variant, int hd, bool masked) {
 // 64.6 / 61.6 / 78.3; 8 x 2048 x 16 145 / 125 / 153; 8 x 4096 x 16 - / 347 /
 // 344; 1 x 16384 x 16 751 / 601 / 534; head_dim 128, 3 x 446 x 8 10.9 / 14.8,
 // 16 x 1024 x 8 76.8 / 69.1; 56 x 47 x 16 6.6 / 8.7 (half of each block idle).
-// So 16 up to 64 queries or 640 blocks of 128 queries, 64 from
+// So 16 up to 64 queries, or while its blocks of 64 all run at once: at
+// head_dim 128 LDS holds two blocks per CU (18 x 216 x 8, 576 blocks, 19.4 /
+// 17.3; 4 x 1000 x 8, 512, 29.5 / 29.0; 1 x 3792 x 8, 480, 73 / 87), below it
+// about four (10 x 640 x 8, 800 blocks, 13.9 / 15.8; 1 x 4000 x 16, 1008, above,
+// but 32 x 200 x 8, 1024, 11.5 / 10.4 and 16 x 500 x 8, 1024, 17.3 / 15.4, both
+// not causal; 40 x 216 x 8, 1280, 14.1 / 13.1).  64 queries per wave from
 // 16384 queries or 2048 blocks of at least 4096 queries on.  The ping-pong
 // kernel (head_dim 64, no key mask) is ahead from 16384 queries on (1 x 16384
 // x 16 530 us, 1 x 32768 x 16 2025 against 2073) and behind below (8 x 4096 x
@@ -1017,7 +1028,8 @@ static bool attention_variant_fits(int variant, int hd, bool masked) {
 static int select_attention(int64_t B, int S_q, int H, int hd, bool masked) {
   if (hd >= 256) return S_q <= 128 && B * H >= kCUs ? XB_ATTN_W8_Q16 : XB_ATTN_W4_Q16;
   if (hd == 64 && !masked && (S_q >= 16384 || (S_q > 4096 && B * H >= 32))) return XB_ATTN_PINGPONG;
-  if (S_q <= 64 || (S_q + 127) / 128 * B * H <= 640) return XB_ATTN_W4_Q16;
+  const int64_t blocks = (int64_t)(S_q + 63) / 64 * B * H;
+  if (S_q <= 64 || blocks <= (hd >= 128 ? 512 : 960)) return XB_ATTN_W4_Q16;
   if (hd >= 128) return XB_ATTN_W4_Q32;
   const bool many = S_q >= 16384 || (S_q >= 4096 && (S_q + 255) / 256 * B * H >= 2048);
   return many ? XB_ATTN_W4_Q64 : XB_ATTN_W4_Q32;
