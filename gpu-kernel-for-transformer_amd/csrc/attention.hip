@@ -124,6 +124,7 @@ __global__ __launch_bounds__(64 * NW * KW, 8 / (NW * KW)) void attn_kernel(const
   constexpr int AHEAD = DECODE || HD >= 256 || NQ > 2 ? 1 : 2;
   static_assert(NT >= BKEYS, "one thread per key stages the validity bytes");
   static_assert(KW == 1 || DECODE, "several key ranges per block: decode only");
+  static_assert(!DECODE || NQ == 1, "m_top is one value");
 
   __shared__ __attribute__((aligned(16))) half_t k_lds[KW * NBUF][BKEYS * LDK];
   __shared__ __attribute__((aligned(16))) half_t v_lds[KW * NBUF][BKEYS * LDV];
@@ -212,6 +213,7 @@ __global__ __launch_bounds__(64 * NW * KW, 8 / (NW * KW)) void attn_kernel(const
     m_run[qb] = 0.f;
     m_set[qb] = false;
   }
+  float m_top = 0.f;  // DECODE (one block of 16 queries): the largest maximum so far
   const half8_t ones8 = {1, 1, 1, 1, 1, 1, 1, 1};
 
   const int k_begin = SPLIT ? (split * KW + kw) * a.split_keys : 0;
@@ -377,13 +379,20 @@ __global__ __launch_bounds__(64 * NW * KW, 8 / (NW * KW)) void attn_kernel(const
           // offset jumps to the first finite maximum and nothing is rescaled
           // (exp2(-sh) could overflow there).  Afterwards sh >= 0, corr <= 1.
           const bool was_set = TRACK ? m_set[qb] : t != 0;
-          // Decode moves the offset onto every tile's own maximum, up or down (by
-          // at most 2^60, o stays FP32): the largest probability of each tile is
-          // then exactly 1 whatever the number of tiles in a range, and the cost
-          // is nothing next to the cache's bytes.
-          const float sh = !was_set ? (TRACK && mx == -INFINITY ? 0.f : mx)
-                           : !DECODE ? fmaxf(mx, 0.f)
-                           : mx == -INFINITY ? 0.f : fmaxf(mx, -60.f);
+          // Decode moves the offset onto every tile's own maximum, up or down: the
+          // largest probability of each tile is then exactly 1 whatever the number
+          // of tiles in a range, and the cost is nothing next to the cache's
+          // bytes.  It stays within 2^60 of the largest maximum so far (m_top), so
+          // o and lacc, which grow as it falls, stay far inside FP32.
+          float sh = !was_set ? (TRACK && mx == -INFINITY ? 0.f : mx) : fmaxf(mx, 0.f);
+          if constexpr (DECODE) {
+            if (was_set) {
+              m_top = fmaxf(m_top, m_run[qb] + mx);
+              sh = mx == -INFINITY ? 0.f : fmaxf(mx, m_top - 60.f - m_run[qb]);
+            } else {
+              m_top = m_run[qb] + mx;
+            }
+          }
           if constexpr (TRACK) m_set[qb] = was_set || mx != -INFINITY;
           const float corr = was_set ? __builtin_amdgcn_exp2f(-sh) : 1.f;
           m_run[qb] += sh;

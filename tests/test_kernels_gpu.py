@@ -687,6 +687,25 @@ def test_decode_long_cache(pkg, cuda, b, heads, hd, start):
     torch.testing.assert_close(out.cpu().float(), ref, atol=2e-3, rtol=1e-2)
 
 
+@pytest.mark.parametrize("b,heads,hd,start", [(1, 2, 64, 700), (8, 16, 64, 9000), (12, 16, 32, 9000), (40, 16, 128, 3000)])
+def test_decode_scores_fall_steeply(pkg, cuda, b, heads, hd, start):
+    """Every key tile's scores lie 2^100 below the tile before it, up again every
+    eighth tile: the softmax offset follows the tiles down without o or the row
+    sum leaving FP32.  Only the first tile of each eight counts, with equal
+    weights, so the result is the mean of V over those keys."""
+    length = start + 1
+    pos = torch.arange(length)
+    fall = -70.0 * ((pos // 64) % 8).float()  # natural-log scores
+    t = torch.randn(b, length, 3, heads, hd, generator=_gen(start))
+    t[:, :, 0] = 4.0
+    t[:, :, 1] = (fall / (4.0 * hd**0.5)).view(1, -1, 1, 1)
+    qkv_full = t.view(b, length, 3 * heads * hd).half()
+    kc, vc = _fill_cache(pkg, qkv_full, heads, length, [start, 1], cuda)
+    out = pkg.attention_kv_cache(qkv_full[:, start:].contiguous().to(cuda), kc, vc, heads, start).cpu().float()
+    ref = t[:, fall == 0, 2].half().float().mean(1).view(b, 1, heads * hd)
+    torch.testing.assert_close(out, ref, atol=2e-3, rtol=1e-2)
+
+
 @pytest.mark.parametrize("b,heads,hd,start,chunk", [
     (1, 2, 64, 6000, 17), (2, 2, 64, 5000, 130), (1, 3, 8, 4095, 64), (1, 2, 128, 3001, 100), (1, 1, 256, 2100, 33),
     (1, 2, 32, 2047, 300)])
