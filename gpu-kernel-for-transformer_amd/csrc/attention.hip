@@ -121,7 +121,10 @@ __global__ __launch_bounds__(64 * NW * KW, 8 / (NW * KW)) void attn_kernel(const
   // registers), so more of them fit on a CU.
   constexpr bool DECODE = SPLIT && NW == 1;
   constexpr int NBUF = DECODE ? 1 : 2;
-  constexpr int AHEAD = DECODE || HD >= 256 || NQ > 2 ? 1 : 2;
+  // Tiles in flight in registers: two hide a cold fetch where the registers are
+  // there; 32 queries per wave of head_dim 128 have none to spare (us, two / one:
+  // 18 x 216 x 8 17.4 / 16.5, 16 x 1024 x 8 69 to 72 / 67.4, 4 x 4096 x 8 217 / 209).
+  constexpr int AHEAD = DECODE || HD >= 256 || NQ > 2 || (HD >= 128 && NQ > 1) ? 1 : 2;
   static_assert(NT >= BKEYS, "one thread per key stages the validity bytes");
   static_assert(KW == 1 || DECODE, "several key ranges per block: decode only");
   static_assert(!DECODE || NQ == 1, "m_top is one value");
@@ -1020,13 +1023,12 @@ static bool attention_variant_fits(int variant, int hd, bool masked) {
 // heads 20.1 / 24.3 / 36.6; 1 x 4000 x 16 79.6 / 85.4 / 117; 2 x 2907 x 16
 // 64.6 / 61.6 / 78.3; 8 x 2048 x 16 145 / 125 / 153; 8 x 4096 x 16 - / 347 /
 // 344; 1 x 16384 x 16 751 / 601 / 534; head_dim 128, 3 x 446 x 8 10.9 / 14.8,
-// 16 x 1024 x 8 76.8 / 69.1; 56 x 47 x 16 6.6 / 8.7 (half of each block idle).
-// So 16 up to 64 queries, or while its blocks of 64 all run at once: at
-// head_dim 128 LDS holds two blocks per CU (18 x 216 x 8, 576 blocks, 19.4 /
-// 17.3; 4 x 1000 x 8, 512, 29.5 / 29.0; 1 x 3792 x 8, 480, 73 / 87), below it
-// about four (10 x 640 x 8, 800 blocks, 13.9 / 15.8; 1 x 4000 x 16, 1008, above,
-// but 32 x 200 x 8, 1024, 11.5 / 10.4 and 16 x 500 x 8, 1024, 17.3 / 15.4, both
-// not causal; 40 x 216 x 8, 1280, 14.1 / 13.1).  64 queries per wave from
+// 16 x 1024 x 8 78.3 / 67.4; 56 x 47 x 16 6.6 / 8.7 (half of each block idle).
+// So 16 up to 64 queries, or while its blocks of 64 all run at once with room
+// left: at head_dim 128 LDS holds two blocks per CU (18 x 216 x 8, 576 blocks,
+// 19.2 / 16.5; 4 x 1000 x 8, 512, 30.3 / 28.5), below it about four (10 x 640 x
+// 8, 800 blocks, 13.9 / 15.8; 32 x 200 x 8, 1024, 11.5 / 10.4; 16 x 500 x 8,
+// 1024, 17.3 / 15.4; 40 x 216 x 8, 1280, 14.1 / 13.1).  64 queries per wave from
 // 16384 queries or 2048 blocks of at least 4096 queries on.  The ping-pong
 // kernel (head_dim 64, no key mask) is ahead from 16384 queries on (1 x 16384
 // x 16 530 us, 1 x 32768 x 16 2025 against 2073) and behind below (8 x 4096 x
@@ -1038,7 +1040,7 @@ static int select_attention(int64_t B, int S_q, int H, int hd, bool masked) {
   if (hd >= 256) return S_q <= 128 && B * H >= kCUs ? XB_ATTN_W8_Q16 : XB_ATTN_W4_Q16;
   if (hd == 64 && !masked && (S_q >= 16384 || (S_q > 4096 && B * H >= 32))) return XB_ATTN_PINGPONG;
   const int64_t blocks = (int64_t)(S_q + 63) / 64 * B * H;
-  if (S_q <= 64 || blocks <= (hd >= 128 ? 512 : 960)) return XB_ATTN_W4_Q16;
+  if (S_q <= 64 || blocks <= (hd >= 128 ? 480 : 960)) return XB_ATTN_W4_Q16;
   if (hd >= 128) return XB_ATTN_W4_Q32;
   const bool many = S_q >= 16384 || (S_q >= 4096 && (S_q + 255) / 256 * B * H >= 2048);
   return many ? XB_ATTN_W4_Q64 : XB_ATTN_W4_Q32;
