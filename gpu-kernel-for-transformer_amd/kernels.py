@@ -544,6 +544,8 @@ def stack_forward(
     """
     _require_device(x, "stack_forward")
     batch, seq_len, _ = x.shape
+    if caches is not None and len(caches) != 2 * stack.layers:
+        raise ValueError(f"{stack.layers} layers need {2 * stack.layers} cache pointers, got {len(caches)}")
     if caches is None:
         need = _stack_workspace_bytes(batch, seq_len, stack.heads, stack.head_dim, stack.ffn_dim, variants[4])
     else:

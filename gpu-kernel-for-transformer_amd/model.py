@@ -41,8 +41,9 @@ from __future__ import annotations
 
 import ctypes
 import dataclasses
+import itertools
 import operator
-from typing import Dict, Optional, Tuple
+from typing import Dict, NamedTuple, Optional, Tuple
 
 import torch
 import torch.nn as nn
@@ -104,7 +105,9 @@ def _tensor_version(tensor: torch.Tensor) -> Optional[int]:
 # so a model's cached walk of its own tree (parameter list, LayerNorms) is
 # redone only after some tree may have changed, not on every forward.  The
 # walk itself (Module.parameters / modules) costs tens of microseconds, as
-# much as a whole small forward.
+# much as a whole small forward.  No hook sees a module leave (`del
+# model.layers[i]`, `pop`), enter by ModuleList.insert or by its parent's
+# `_modules`: the walk's children are compared with the live ones as well.
 _TREE_GENERATION = [0]
 
 
@@ -115,6 +118,20 @@ def _tree_changed(*_args) -> None:
 
 nn.modules.module.register_module_parameter_registration_hook(_tree_changed)
 nn.modules.module.register_module_module_registration_hook(_tree_changed)
+
+_CHILDREN = operator.attrgetter("_modules")
+_VALUES = operator.methodcaller("values")
+
+
+class _Tree(NamedTuple):
+    """A walk of a model's modules (the model itself left out)."""
+
+    params: Tuple[nn.Parameter, ...]
+    norms: Tuple[nn.LayerNorm, ...]
+    attentions: Tuple[nn.Module, ...]
+    generation: int
+    containers: Tuple[nn.Module, ...]  # modules with children
+    children: Tuple[nn.Module, ...]    # of the model, then of each container
 
 
 class _LayerWeights:
@@ -309,13 +326,13 @@ class UserOptimizedTransformer(nn.Module):
         for it.  The descriptors are written once and only read afterwards, so
         forwards of several threads may share them.
         """
-        params, norms = self._tree()
-        attentions = self.__dict__["_tree_cache"][3]
-        for norm in norms:  # read on each call: setting one to None calls no registration hook
+        tree = self._walk()
+        for norm in tree.norms:  # read on each call: setting one to None calls no registration hook
             registered = norm._parameters
             if registered.get("weight") is None or registered.get("bias") is None:
                 return None
-        settings = (row_block, [n.eps for n in norms], [a.scale for a in attentions])
+        params = tree.params
+        settings = (row_block, [n.eps for n in tree.norms], [a.scale for a in tree.attentions])
         try:
             key = (tuple(map(_VERSION_OF, params)), tuple(map(torch.Tensor.data_ptr, params)), settings)
         except RuntimeError:  # inference-mode parameters have no version counter: never reuse
@@ -346,14 +363,26 @@ class UserOptimizedTransformer(nn.Module):
         return value
 
     def _tree(self) -> Tuple[Tuple[nn.Parameter, ...], Tuple[nn.LayerNorm, ...]]:
-        """(parameters, LayerNorm modules) of this model, re-walked after any registration."""
+        """(parameters, LayerNorm modules) of this model, as _walk found them."""
+        tree = self._walk()
+        return tree.params, tree.norms
+
+    def _walk(self) -> _Tree:
+        """This model's modules and parameters, re-walked after any registration or change of the modules."""
         cached = self.__dict__.get("_tree_cache")
-        if cached is None or cached[0] != _TREE_GENERATION[0]:
-            cached = (_TREE_GENERATION[0], tuple(self.parameters()),
-                      tuple(m for m in self.modules() if isinstance(m, nn.LayerNorm)),
-                      tuple(layer.attention for layer in self.layers))
+        if (cached is None or cached.generation != _TREE_GENERATION[0]
+                or self._children_of(cached.containers) != cached.children):
+            modules = tuple(m for m in self.modules() if m is not self)
+            containers = tuple(m for m in modules if m._modules)
+            cached = _Tree(params=tuple(self.parameters()), norms=tuple(m for m in modules if isinstance(m, nn.LayerNorm)),
+                           attentions=tuple(layer.attention for layer in self.layers), generation=_TREE_GENERATION[0],
+                           containers=containers, children=self._children_of(containers))
             self.__dict__["_tree_cache"] = cached
-        return cached[1], cached[2]
+        return cached
+
+    def _children_of(self, containers: Tuple[nn.Module, ...]) -> Tuple[nn.Module, ...]:
+        return tuple(itertools.chain(self._modules.values(),
+                                     itertools.chain.from_iterable(map(_VALUES, map(_CHILDREN, containers)))))
 
     def _fused_stack_eligible(self) -> bool:
         """Conditions of the whole-stack kernel beyond the shape: the toggle, LayerNorm eps 1e-5 with affine."""
@@ -361,7 +390,7 @@ class UserOptimizedTransformer(nn.Module):
             return False
         # Parameters read from each module's registry directly: going through
         # nn.Module.__getattr__ for 18 of them cost microseconds per forward.
-        for norm in self._tree()[1]:
+        for norm in self._walk().norms:
             registered = norm._parameters
             if norm.eps != 1e-5 or registered.get("weight") is None or registered.get("bias") is None:
                 return False
@@ -369,7 +398,7 @@ class UserOptimizedTransformer(nn.Module):
 
     def _fused_stack_parameters(self) -> Tuple[torch.Tensor, torch.Tensor, int]:
         """Fragment-packed FP16 weights, FP32 bias/LayerNorm buffer and LayerNorm affine mask, cached by version."""
-        params = self._tree()[0]
+        params = self._walk().params
         try:
             key = (tuple(map(_VERSION_OF, params)), tuple(map(torch.Tensor.data_ptr, params)))
         except RuntimeError:  # inference-mode parameters have no version counter: never reuse

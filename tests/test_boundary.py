@@ -165,6 +165,42 @@ def test_tree_cache_follows_registrations(pkg):
     assert not model.execution_plan(2, 8).fused
 
 
+@pytest.mark.parametrize("change", ["del", "pop", "insert", "swap"])
+def test_native_descriptor_follows_the_layers(pkg, change):
+    """The native sequence runs the layers that the model has now: modules that leave or
+    enter without a registration hook are in the next descriptor, as the live loop had them."""
+    model = pkg.UserOptimizedTransformer(pkg.TransformerConfig(2, 300, 256, 4, 256, 3, True)).eval()
+    assert model._native_stack(False)[0].layers == 3
+    layers = model.layers
+    if change == "del":
+        del layers[2]
+    elif change == "pop":
+        layers.pop(0)
+    elif change == "insert":
+        layers.insert(1, layers[2])
+    else:
+        layers[1]._modules["ffn_in"] = torch.nn.Linear(256, 256)
+    stack, blocks, _ = model._native_stack(False)[:3]
+    assert stack.layers == len(blocks) == len(layers)
+    for block, layer in zip(blocks, layers):
+        assert block.norm1_g == layer.norm1.weight.data_ptr()
+    assert blocks[1].ffn_in_w == model._layer_weights(1).ffn_in_w.data_ptr()
+    assert all(any(p is q for q in model._tree()[0]) for p in layers[1].parameters())
+
+
+def test_stack_forward_wants_two_caches_per_layer(pkg, monkeypatch):
+    """The native sequence reads two cache pointers per layer: fewer are refused before the call."""
+    import importlib
+
+    kernels = importlib.import_module(pkg.__name__ + ".kernels")
+    monkeypatch.setattr(kernels, "_require_device", lambda tensor, what: None)
+    model = pkg.UserOptimizedTransformer(pkg.TransformerConfig(2, 8, 256, 4, 256, 2, True)).eval()
+    x = torch.zeros(2, 8, 256)
+    with pytest.raises(ValueError, match="2 layers need 4 cache pointers, got 2"):
+        kernels.stack_forward(x, model._native_stack(False)[0], (-1,) * 5, torch.empty_like(x),
+                              caches=(ctypes.c_void_p * 2)(16, 16), cache_capacity=8)
+
+
 def test_fused_eligibility_checks_every_layer_norm_on_each_call(pkg):
     """The whole-stack kernel needs eps 1e-5, a weight and a bias on every LayerNorm, re-read per call."""
     model = pkg.UserOptimizedTransformer(pkg.TransformerConfig(2, 8, 128, 4, 128, 2, True)).eval()
