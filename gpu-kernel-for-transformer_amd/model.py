@@ -41,6 +41,7 @@ from __future__ import annotations
 
 import ctypes
 import dataclasses
+import functools
 import itertools
 import operator
 from typing import Dict, NamedTuple, Optional, Tuple
@@ -119,8 +120,9 @@ def _tree_changed(*_args) -> None:
 nn.modules.module.register_module_parameter_registration_hook(_tree_changed)
 nn.modules.module.register_module_module_registration_hook(_tree_changed)
 
-_CHILDREN = operator.attrgetter("_modules")
+_CHILDREN, _PARAMETERS = operator.attrgetter("_modules"), operator.attrgetter("_parameters")
 _VALUES = operator.methodcaller("values")
+_IS_NONE = functools.partial(operator.is_, None)
 
 
 class _Tree(NamedTuple):
@@ -132,6 +134,12 @@ class _Tree(NamedTuple):
     generation: int
     containers: Tuple[nn.Module, ...]  # modules with children
     children: Tuple[nn.Module, ...]    # of the model, then of each container
+    holders: Tuple[nn.Module, ...]     # modules with parameters
+
+    def live_parameters(self) -> Tuple[torch.Tensor, ...]:
+        """What the holders hold now: torch.func.functional_call swaps tensors in without registering them."""
+        held = itertools.chain.from_iterable(map(_VALUES, map(_PARAMETERS, self.holders)))
+        return tuple(itertools.filterfalse(_IS_NONE, held))
 
 
 class _LayerWeights:
@@ -331,7 +339,7 @@ class UserOptimizedTransformer(nn.Module):
             registered = norm._parameters
             if registered.get("weight") is None or registered.get("bias") is None:
                 return None
-        params = tree.params
+        params = tree.live_parameters()
         settings = (row_block, [n.eps for n in tree.norms], [a.scale for a in tree.attentions])
         try:
             key = (tuple(map(_VERSION_OF, params)), tuple(map(torch.Tensor.data_ptr, params)), settings)
@@ -376,7 +384,8 @@ class UserOptimizedTransformer(nn.Module):
             containers = tuple(m for m in modules if m._modules)
             cached = _Tree(params=tuple(self.parameters()), norms=tuple(m for m in modules if isinstance(m, nn.LayerNorm)),
                            attentions=tuple(layer.attention for layer in self.layers), generation=_TREE_GENERATION[0],
-                           containers=containers, children=self._children_of(containers))
+                           containers=containers, children=self._children_of(containers),
+                           holders=tuple(m for m in modules if m._parameters))
             self.__dict__["_tree_cache"] = cached
         return cached
 

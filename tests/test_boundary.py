@@ -201,6 +201,21 @@ def test_stack_forward_wants_two_caches_per_layer(pkg, monkeypatch):
                               caches=(ctypes.c_void_p * 2)(16, 16), cache_capacity=8)
 
 
+def test_native_descriptor_follows_functional_call(pkg):
+    """Parameters swapped in for one call (torch.func.functional_call) are the ones it reads,
+    and the model's own ones are back afterwards."""
+    model = pkg.UserOptimizedTransformer(pkg.TransformerConfig(2, 300, 256, 4, 256, 1, True)).eval()
+    own = model._native_stack(False)[1][0]
+    seen = []
+    model.forward = lambda: seen.append(model._native_stack(False))
+    swapped = {name: p.detach() + 1.0 for name, p in model.named_parameters()}
+    torch.func.functional_call(model, swapped, ())
+    block, weights = seen[0][1][0], seen[0][2][0]
+    assert block.norm1_g == swapped["layers.0.norm1.weight"].data_ptr() != own.norm1_g
+    assert torch.equal(weights.out_w, swapped["layers.0.attention.out_proj.weight"].half())
+    assert model._native_stack(False)[1][0].norm1_g == own.norm1_g == model.layers[0].norm1.weight.data_ptr()
+
+
 def test_fused_eligibility_checks_every_layer_norm_on_each_call(pkg):
     """The whole-stack kernel needs eps 1e-5, a weight and a bias on every LayerNorm, re-read per call."""
     model = pkg.UserOptimizedTransformer(pkg.TransformerConfig(2, 8, 128, 4, 128, 2, True)).eval()
