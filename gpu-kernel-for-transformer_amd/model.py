@@ -340,7 +340,7 @@ class UserOptimizedTransformer(nn.Module):
             if registered.get("weight") is None or registered.get("bias") is None:
                 return None
         params = tree.live_parameters()
-        settings = (row_block, [n.eps for n in tree.norms], [a.scale for a in tree.attentions])
+        settings = (row_block, self.config, [n.eps for n in tree.norms], [a.scale for a in tree.attentions])
         try:
             key = (tuple(map(_VERSION_OF, params)), tuple(map(torch.Tensor.data_ptr, params)), settings)
         except RuntimeError:  # inference-mode parameters have no version counter: never reuse

@@ -216,6 +216,16 @@ def test_native_descriptor_follows_functional_call(pkg):
     assert model._native_stack(False)[1][0].norm1_g == own.norm1_g == model.layers[0].norm1.weight.data_ptr()
 
 
+def test_native_descriptor_follows_the_config(pkg):
+    """The descriptor's causal flag is the present config's."""
+    import dataclasses
+
+    model = pkg.UserOptimizedTransformer(pkg.TransformerConfig(2, 300, 256, 4, 256, 1, True)).eval()
+    assert model._native_stack(False)[0].causal == 1
+    model.config = dataclasses.replace(model.config, causal=False)
+    assert model._native_stack(False)[0].causal == 0
+
+
 def test_fused_eligibility_checks_every_layer_norm_on_each_call(pkg):
     """The whole-stack kernel needs eps 1e-5, a weight and a bias on every LayerNorm, re-read per call."""
     model = pkg.UserOptimizedTransformer(pkg.TransformerConfig(2, 8, 128, 4, 128, 2, True)).eval()
