@@ -208,6 +208,14 @@ class UserOptimizedTransformer(nn.Module):
         self._triton_fused_ffn_enabled = True
         self._attention_fp16_accumulation_enabled = False
 
+    # What the forward derives from the module and rebuilds when it is missing.  A copy or a
+    # saved file leaves it out: the descriptor's pointers are this process's and this model's.
+    _DERIVED = ("_native_stack_cache", "_weight_cache", "_fused_stack_cache", "_tree_cache", "_mask_cache", "_side_streams")
+
+    def __getstate__(self) -> dict:
+        """The state that copy.deepcopy, pickle and torch.save take."""
+        return {name: value for name, value in self.__dict__.items() if name not in self._DERIVED}
+
     # ----------------------------------------------------------------- toggles
     @property
     def shape_execution_plan(self) -> ShapeExecutionPlan:

@@ -188,6 +188,27 @@ def test_native_descriptor_follows_the_layers(pkg, change):
     assert all(any(p is q for q in model._tree()[0]) for p in layers[1].parameters())
 
 
+def test_model_copies_and_saves_after_a_forward(pkg):
+    """copy.deepcopy and torch.save work once the native descriptor exists; the copy keeps
+    the settings and builds a descriptor of its own parameters."""
+    import copy
+    import io
+
+    model = pkg.UserOptimizedTransformer(pkg.TransformerConfig(2, 300, 256, 4, 256, 2, True)).eval()
+    model.enable_fused_stack(False)
+    model._native_stack(False)
+    file = io.BytesIO()
+    torch.save(model, file)
+    file.seek(0)
+    for twin in (copy.deepcopy(model), torch.load(file, weights_only=False)):
+        assert twin._fused_stack_enabled is False and not twin.training
+        for p, q in zip(model.parameters(), twin.parameters()):
+            assert torch.equal(p, q) and p.data_ptr() != q.data_ptr()
+        _, blocks, weights = twin._native_stack(False)[:3]
+        assert blocks[1].norm1_g == twin.layers[1].norm1.weight.data_ptr()
+        assert torch.equal(weights[1].ffn_in_w, model.layers[1].ffn_in.weight.half())
+
+
 def test_stack_forward_wants_two_caches_per_layer(pkg, monkeypatch):
     """The native sequence reads two cache pointers per layer: fewer are refused before the call."""
     import importlib
