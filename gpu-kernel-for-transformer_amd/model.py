@@ -209,12 +209,16 @@ class UserOptimizedTransformer(nn.Module):
         self._attention_fp16_accumulation_enabled = False
 
     # What the forward derives from the module and rebuilds when it is missing.  A copy or a
-    # saved file leaves it out: the descriptor's pointers are this process's and this model's.
+    # saved file leaves it out (the descriptor's pointers are this process's and this model's),
+    # and what a file saved with it holds is not taken over.
     _DERIVED = ("_native_stack_cache", "_weight_cache", "_fused_stack_cache", "_tree_cache", "_mask_cache", "_side_streams")
 
     def __getstate__(self) -> dict:
         """The state that copy.deepcopy, pickle and torch.save take."""
         return {name: value for name, value in self.__dict__.items() if name not in self._DERIVED}
+
+    def __setstate__(self, state: dict) -> None:
+        super().__setstate__({name: value for name, value in state.items() if name not in self._DERIVED})
 
     # ----------------------------------------------------------------- toggles
     @property

@@ -209,6 +209,16 @@ def test_model_copies_and_saves_after_a_forward(pkg):
         assert torch.equal(weights[1].ffn_in_w, model.layers[1].ffn_in.weight.half())
 
 
+def test_caches_of_an_older_file_are_dropped(pkg):
+    """A model pickled with its derived caches inside loads without them: their form is not this code's."""
+    model = pkg.UserOptimizedTransformer(pkg.TransformerConfig(2, 300, 256, 4, 256, 1, True)).eval()
+    walk = (0, tuple(model.parameters()), tuple(m for m in model.modules() if isinstance(m, torch.nn.LayerNorm)))
+    loaded = pkg.UserOptimizedTransformer.__new__(pkg.UserOptimizedTransformer)
+    loaded.__setstate__({**model.__getstate__(), "_tree_cache": walk, "_weight_cache": {0: ((), None)}})
+    assert "_tree_cache" not in loaded.__dict__ and "_weight_cache" not in loaded.__dict__
+    assert loaded._native_stack(False)[0].layers == 1
+
+
 def test_stack_forward_wants_two_caches_per_layer(pkg, monkeypatch):
     """The native sequence reads two cache pointers per layer: fewer are refused before the call."""
     import importlib
