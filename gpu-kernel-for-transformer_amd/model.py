@@ -336,15 +336,36 @@ class UserOptimizedTransformer(nn.Module):
             cache[index] = cached
         return cached[1]
 
-    def _native_stack(self, row_block: bool) -> Optional[Tuple[_capi.XbStack, object, object]]:
-        """(xb_stack, its xb_block array, the tensors they point into), cached by parameter version.
+    def _fits_config(self) -> bool:
+        """Whether every parameter is what the native kernels index it as: of the config's
+        sizes, all on one device, LayerNorms in contiguous float32."""
+        d, f = self.config.d_model, self.config.ffn_dim
+        device = self.final_norm.weight.device
+        norms = [self.final_norm]
+        for layer in self.layers:
+            att = layer.attention
+            norms += [layer.norm1, layer.norm2]
+            for lin, n, k in ((att.q_proj, d, d), (att.k_proj, d, d), (att.v_proj, d, d), (att.out_proj, d, d),
+                              (layer.ffn_in, f, d), (layer.ffn_out, d, f)):
+                if lin.bias is None or tuple(lin.weight.shape) != (n, k) or tuple(lin.bias.shape) != (n,):
+                    return False
+                if lin.weight.device != device or lin.bias.device != device:
+                    return False
+        return all(p.numel() == d and p.dtype == torch.float32 and p.device == device and p.is_contiguous()
+                   for norm in norms for p in (norm.weight, norm.bias))
+
+    def _native_stack(self, row_block: bool) -> Optional[Tuple[_capi.XbStack, object, object, torch.device]]:
+        """(xb_stack, its xb_block array, the tensors they point into, their device), cached by parameter version.
 
         row_block: with fragment-packed weights for xb_row_block instead of
         the FP16 copies the GEMMs read.
 
-        None when a LayerNorm has no weight or bias: the wrappers then raise
-        for it.  The descriptors are written once and only read afterwards, so
-        forwards of several threads may share them.
+        None when a LayerNorm has no weight or bias, or a parameter does not
+        fit the config (_fits_config): the kernels would take its size from
+        the config.  The wrappers, which take each size from the tensor
+        itself, then run the forward or raise.  The descriptors are written
+        once and only read afterwards, so forwards of several threads may
+        share them.
         """
         tree = self._walk()
         for norm in tree.norms:  # read on each call: setting one to None calls no registration hook
@@ -360,6 +381,9 @@ class UserOptimizedTransformer(nn.Module):
         cached = self.__dict__.get("_native_stack_cache")
         if key is not None and cached is not None and cached[0] == key:
             return cached[1]
+        if not self._fits_config():
+            self.__dict__["_native_stack_cache"] = (key, None)
+            return None
         cfg = self.config
         blocks = (_capi.XbBlock * len(self.layers))()
         weights = [_RowBlockWeights(layer) if row_block else self._layer_weights(i)
@@ -378,7 +402,7 @@ class UserOptimizedTransformer(nn.Module):
                               final_eps=final.eps, final_affine=int(self._layer_norm_uses_affine(final)),
                               layers=len(self.layers), heads=cfg.num_heads, head_dim=cfg.head_dim,
                               ffn_dim=cfg.ffn_dim, causal=int(cfg.causal))
-        value = (stack, blocks, weights)
+        value = (stack, blocks, weights, final.weight.device)
         self.__dict__["_native_stack_cache"] = (key, value)
         return value
 
@@ -715,7 +739,7 @@ class UserOptimizedTransformer(nn.Module):
         if plan.row_block and self.config.d_model == 32 and x.data_ptr() % 16:
             x = x.clone()  # this width's LayerNorm takes any alignment, the row blocks 16 bytes
         native = None if kernels.recording() else self._native_stack(plan.row_block)
-        if native is None:
+        if native is None or native[3] != x.device:
             return self._per_op_forward_stepwise(x, plan, out, token_valid, cache_start)
         if out is None:
             out = torch.empty_like(x)
@@ -742,7 +766,7 @@ class UserOptimizedTransformer(nn.Module):
                                  token_valid: Optional[torch.Tensor], cache_start: Optional[int]) -> torch.Tensor:
         """_per_op_forward, one wrapper call per launch."""
         native = self._native_stack(True) if plan.row_block else None
-        if native is not None:
+        if native is not None and native[3] == x.device:
             return self._row_block_forward_stepwise(x, native[0], plan, out, token_valid, cache_start)
         cfg = self.config
         batch, seq_len, d_model = x.shape
@@ -776,8 +800,11 @@ class UserOptimizedTransformer(nn.Module):
                 residual_in, update, layer.norm2.weight, layer.norm2.bias, layer.norm2.eps, f16,
                 apply_affine=self._layer_norm_uses_affine(layer.norm2), residual_out=residual,
             )
-            hidden = kernels.linear(norm2, w.ffn_in_w, w.ffn_in_b, gelu=True, variant=plan.ffn_in_variant)
-            update = kernels.linear(hidden, w.ffn_out_w, w.ffn_out_b, variant=plan.ffn_out_variant)
+            planned = w.ffn_in_w.shape[0] == cfg.ffn_dim  # the plan's tiles are for the config's width
+            hidden = kernels.linear(norm2, w.ffn_in_w, w.ffn_in_b, gelu=True,
+                                    variant=plan.ffn_in_variant if planned else _capi.XB_VARIANT_AUTO)
+            update = kernels.linear(hidden, w.ffn_out_w, w.ffn_out_b,
+                                    variant=plan.ffn_out_variant if planned else _capi.XB_VARIANT_AUTO)
             last = index == num_layers - 1
             following = self.final_norm if last else self.layers[index + 1].norm1
             residual_in, norm = kernels.fused_residual_layer_norm(

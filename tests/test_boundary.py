@@ -209,6 +209,30 @@ def test_model_copies_and_saves_after_a_forward(pkg):
         assert torch.equal(weights[1].ffn_in_w, model.layers[1].ffn_in.weight.half())
 
 
+@pytest.mark.parametrize("misfit", ["narrow_ffn", "wide_ffn", "norm", "final_norm", "half_norm", "projection", "bias"])
+def test_native_descriptor_only_for_parameters_of_the_configs_sizes(pkg, misfit):
+    """The native kernels take every size from the config: a parameter of another size, or a
+    LayerNorm that isn't float32, gives no descriptor (the wrappers then run it or raise)."""
+    model = pkg.UserOptimizedTransformer(pkg.TransformerConfig(2, 300, 256, 4, 512, 2, True)).eval()
+    layer = model.layers[1]
+    assert model._native_stack(False)[0].ffn_dim == 512
+    if misfit.endswith("ffn"):
+        width = 256 if misfit == "narrow_ffn" else 1024
+        layer.ffn_in, layer.ffn_out = torch.nn.Linear(256, width), torch.nn.Linear(width, 256)
+    elif misfit == "norm":
+        layer.norm2 = torch.nn.LayerNorm(64)
+    elif misfit == "final_norm":
+        model.final_norm = torch.nn.LayerNorm(512)
+    elif misfit == "half_norm":
+        layer.norm1.half()
+    elif misfit == "projection":
+        layer.attention.k_proj = torch.nn.Linear(256, 64)
+    else:
+        layer.ffn_in.bias = None
+    assert model._native_stack(False) is None and model._native_stack(True) is None
+    assert model._native_stack(False) is None
+
+
 def test_caches_of_an_older_file_are_dropped(pkg):
     """A model pickled with its derived caches inside loads without them: their form is not this code's."""
     model = pkg.UserOptimizedTransformer(pkg.TransformerConfig(2, 300, 256, 4, 256, 1, True)).eval()

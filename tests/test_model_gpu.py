@@ -928,3 +928,26 @@ def test_unaligned_input_and_norms(pkg, cuda, geom):
             norm.bias.data = off_by_one(norm.bias.data)
         out = model(x)
         assert float((out - ref).norm() / ref.norm()) < 1e-3
+
+
+@pytest.mark.parametrize("geom", [(2, 150, 256, 4, 512, 2), (3, 200, 64, 4, 128, 2), (2, 40, 512, 8, 512, 2)])
+@pytest.mark.parametrize("width", [96, 1200])
+def test_ffn_of_another_width_in_one_layer(pkg, cuda, geom, width):
+    """A layer whose FFN pair has another width than the config's runs with its own sizes,
+    and a LayerNorm of the wrong width is refused."""
+    config = pkg.TransformerConfig(*geom, True)
+    torch.manual_seed(21)
+    baseline = BaselineTransformer(config).eval()
+    model = pkg.UserOptimizedTransformer(config)
+    for m in (baseline, model):
+        m.layers[1].ffn_in, m.layers[1].ffn_out = torch.nn.Linear(geom[2], width), torch.nn.Linear(width, geom[2])
+    copy_model_weights(baseline, model)
+    model = model.to(cuda).eval()
+    x = torch.randn(*geom[:3], generator=torch.Generator().manual_seed(2))
+    mask = torch.ones(geom[0], geom[1], dtype=torch.bool)
+    with torch.inference_mode():
+        result = compare_outputs(baseline(x, mask), model(x.to(cuda)).cpu())
+    assert result.passed, result.summary()
+    model.layers[0].norm2 = torch.nn.LayerNorm(geom[2] // 2).to(cuda)
+    with torch.inference_mode(), pytest.raises(ValueError, match="do not match the input width"):
+        model(x.to(cuda))
