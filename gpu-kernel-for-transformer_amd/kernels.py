@@ -96,6 +96,13 @@ def _check_buffer(t: torch.Tensor, shape, dtype: torch.dtype, device: torch.devi
         raise ValueError(f"{what} must be a contiguous {dtype} tensor of shape {tuple(shape)} on {device}")
 
 
+def _check_norm_parameters(weight: torch.Tensor, bias: torch.Tensor, device: torch.device) -> None:
+    """LayerNorm parameters as the kernels read them (when they apply the affine at all)."""
+    for t in (weight, bias):
+        if t.dtype != torch.float32 or t.device != device or not t.is_contiguous():
+            raise ValueError(f"LayerNorm parameters must be contiguous float32 tensors on {device}")
+
+
 def _ptr(tensor: Optional[torch.Tensor]) -> Optional[int]:
     return None if tensor is None else tensor.data_ptr()
 
@@ -115,6 +122,8 @@ def layer_norm(
         raise ValueError("LayerNorm parameters do not match the input width")
     if inputs.dtype != torch.float32:
         raise ValueError("layer_norm expects float32 inputs")
+    if apply_affine:
+        _check_norm_parameters(weight, bias, inputs.device)
     inputs = inputs.contiguous()
     output = torch.empty_like(inputs, dtype=output_dtype)
     rows = inputs.numel() // n_cols
@@ -164,6 +173,10 @@ def fused_residual_layer_norm(
         raise ValueError("the residual stream must be float32")
     if not residual.is_contiguous() or not update.is_contiguous():
         raise ValueError("residual and update must be contiguous")
+    if update.device != residual.device:
+        raise ValueError("residual and update must be on the same device")
+    if apply_affine:
+        _check_norm_parameters(weight, bias, residual.device)
     n_cols = residual.shape[-1]
     if store_residual:
         if residual_out is None:
@@ -242,8 +255,10 @@ def linear(
         raise ValueError("bias must be float32 with one entry per output feature")
     if inputs.dtype != torch.float16 or weight.dtype != torch.float16:
         raise ValueError("linear expects float16 inputs and weights")
-    if not inputs.is_contiguous() or not weight.is_contiguous():
-        raise ValueError("linear expects contiguous inputs and weights")
+    if not inputs.is_contiguous() or not weight.is_contiguous() or (bias is not None and not bias.is_contiguous()):
+        raise ValueError("linear expects contiguous inputs, weights and bias")
+    if weight.device != inputs.device or (bias is not None and bias.device != inputs.device):
+        raise ValueError("linear expects its weights on the inputs' device")
     m = inputs.numel() // k
     if out is None:
         out = torch.empty((*inputs.shape[:-1], n), device=inputs.device, dtype=torch.float16)

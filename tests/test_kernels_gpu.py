@@ -749,3 +749,21 @@ def test_decode_workspace_too_small(pkg, cuda):
     code = lib.xb_attention_kv_cache(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), out.data_ptr(), b, 1, heads, hd,
                                      start, start + 1, 0.125, None, 0, None)
     assert code == -1
+
+
+def test_parameters_elsewhere_are_refused(pkg, cuda):
+    """Weights on another device, and LayerNorm parameters in another type, are refused
+    before any launch; a LayerNorm that isn't applied may have any type."""
+    x = torch.randn(4, 64, device=cuda)
+    w, b = torch.randn(64, device=cuda), torch.randn(64, device=cuda)
+    for bad in (w.cpu(), w.half(), w.double(), torch.randn(128, device=cuda)[::2]):
+        with pytest.raises(ValueError, match="LayerNorm parameters must be"):
+            pkg.layer_norm(x, bad, b, 1e-5, F16)
+        with pytest.raises(ValueError, match="LayerNorm parameters must be"):
+            pkg.fused_residual_layer_norm(x, x, w, bad, 1e-5, F16)
+    out = pkg.layer_norm(x, w.half(), b.half(), 1e-5, F16, apply_affine=False)
+    assert torch.equal(out, pkg.layer_norm(x, w, b, 1e-5, F16, apply_affine=False))
+    xh, wh = x.half(), torch.randn(32, 64, device=cuda).half()
+    for weight, bias in ((wh.cpu(), None), (wh, torch.randn(32)), (wh, torch.randn(64, device=cuda)[::2])):
+        with pytest.raises(ValueError):
+            pkg.linear(xh, weight, bias)
