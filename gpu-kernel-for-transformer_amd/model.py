@@ -324,16 +324,20 @@ class UserOptimizedTransformer(nn.Module):
         return self._kv_cache_length
 
     # ------------------------------------------------------------ parameter caches
-    def _layer_weights(self, index: int) -> _LayerWeights:
-        """Packed FP16 weights, rebuilt when any source parameter changes (TTB:524-641)."""
+    def _layer_weights(self, index: int, form: type = _LayerWeights):
+        """Packed FP16 weights of a layer in one form, rebuilt when any source parameter changes (TTB:524-641).
+
+        Each form is kept by the parameters alone: a captured graph reads these buffers, so no
+        setting (the row-block toggle, a LayerNorm's eps, the attention scale) may replace them.
+        """
         layer = self.layers[index]
         params = list(layer.attention.parameters()) + list(layer.ffn_in.parameters()) + list(layer.ffn_out.parameters())
         key = tuple((p.data_ptr(), _tensor_version(p), p.device, p.dtype) for p in params)
-        cache: Dict[int, Tuple[tuple, _LayerWeights]] = self.__dict__.setdefault("_weight_cache", {})
-        cached = cache.get(index)
+        cache: Dict[Tuple[int, type], Tuple[tuple, object]] = self.__dict__.setdefault("_weight_cache", {})
+        cached = cache.get((index, form))
         if cached is None or cached[0] != key or any(k[1] is None for k in key):
-            cached = (key, _LayerWeights(layer))
-            cache[index] = cached
+            cached = (key, form(layer))
+            cache[(index, form)] = cached
         return cached[1]
 
     def _fits_config(self) -> bool:
@@ -386,8 +390,8 @@ class UserOptimizedTransformer(nn.Module):
             return None
         cfg = self.config
         blocks = (_capi.XbBlock * len(self.layers))()
-        weights = [_RowBlockWeights(layer) if row_block else self._layer_weights(i)
-                   for i, layer in enumerate(self.layers)]
+        form = _RowBlockWeights if row_block else _LayerWeights
+        weights = [self._layer_weights(i, form) for i in range(len(self.layers))]
         for block, layer, w in zip(blocks, self.layers, weights):
             for name in w.__slots__:
                 setattr(block, name, getattr(w, name).data_ptr())

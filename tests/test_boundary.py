@@ -233,6 +233,31 @@ def test_native_descriptor_only_for_parameters_of_the_configs_sizes(pkg, misfit)
     assert model._native_stack(False) is None
 
 
+def test_packed_weights_outlive_a_change_of_settings(pkg, monkeypatch):
+    """Row-block weights belong to the parameters, not to the descriptor: a LayerNorm eps, the
+    attention scale and the path toggle leave them where a captured graph reads them."""
+    import importlib
+
+    kernels = importlib.import_module(pkg.__name__ + ".kernels")
+    monkeypatch.setattr(kernels, "pack_linear_fragments", lambda w, out: out.copy_(w.detach().flatten()))
+    model = pkg.UserOptimizedTransformer(pkg.TransformerConfig(2, 300, 64, 4, 64, 2, True)).eval()
+    packed = [w.packed for w in model._native_stack(True)[2]]
+    model.layers[0].norm2.eps = 0.25
+    model._native_stack(True)
+    model.layers[1].attention.scale = 0.5
+    model._native_stack(True)
+    model._native_stack(False)                        # the per-op form between two row-block ones
+    held = [entry[1] for entry in model._weight_cache.values()]
+    assert all(any(getattr(w, "packed", None) is p for w in held) for p in packed)
+    again = model._native_stack(True)
+    assert all(w.packed is p for w, p in zip(again[2], packed))
+    assert again[1][0].norm2_eps == 0.25 and again[1][1].scale == 0.5
+    with torch.no_grad():
+        model.layers[0].ffn_in.weight.add_(1.0)
+    changed = [w.packed for w in model._native_stack(True)[2]]
+    assert changed[0] is not packed[0] and changed[1] is packed[1]
+
+
 def test_caches_of_an_older_file_are_dropped(pkg):
     """A model pickled with its derived caches inside loads without them: their form is not this code's."""
     model = pkg.UserOptimizedTransformer(pkg.TransformerConfig(2, 300, 256, 4, 256, 1, True)).eval()

@@ -125,6 +125,32 @@ def test_captured_per_op_forward_overlaps_half_batches(pkg, cuda, geom, masked):
             assert torch.equal(model(x, mask), eager)
 
 
+@pytest.mark.parametrize("geom", [(3, 90, 32, 4, 64, 2), (2, 200, 128, 4, 128, 2)])
+def test_captured_row_blocks_keep_their_weights(pkg, cuda, geom):
+    """A captured narrow model replays its own weights after eager calls with another
+    LayerNorm eps and without row blocks, and after their memory would have been used again."""
+    graphs, _, _ = _runners(pkg)
+    _, model = _models(pkg, pkg.TransformerConfig(*geom, True), cuda)
+    x = torch.randn(*geom[:3], generator=torch.Generator(device=cuda).manual_seed(3), device=cuda)
+    assert model.execution_plan(*geom[:2]).row_block
+    with torch.inference_mode():
+        eager = model(x).clone()
+    graphed = graphs.FixedInputCUDAGraph(model, x, None)
+    with torch.inference_mode():
+        for change in ("eps", "toggle", "back"):
+            if change == "eps":
+                model.layers[0].norm1.eps = 0.5
+            else:
+                model.enable_fused_stack(change == "back")
+                model.layers[0].norm1.eps = 1e-5
+            model(x)
+            junk = [torch.full((n,), float("nan"), device=cuda) for n in (1 << 10, 1 << 12, 1 << 14, 1 << 16) for _ in range(8)]
+            out = graphed(x, None)
+            torch.cuda.synchronize()
+            assert torch.equal(out, eager), change
+            del junk
+
+
 def test_maybe_cuda_graph_refuses_a_failed_handoff(pkg, cuda, monkeypatch):
     """A graph whose check run counted a failed split-form K/V hand-off (its
     rows would be NaN) is refused with the cause named, and the forward stays
