@@ -1372,10 +1372,11 @@ extern "C" int xb_attention_kv_cache(const void* qkv, const void* k_cache, const
                                      void* stream) {
   return attention_kv_cache(qkv, k_cache, v_cache, out, batch, chunk, heads, head_dim, start, capacity, scale, stream,
                             [&](int64_t need, bool optional, void** ptr) {
-                              if (optional && (!workspace || workspace_bytes < need)) return XB_OK;
+                              const bool aligned = ((uintptr_t)workspace & 15u) == 0;
+                              if (optional && (!workspace || workspace_bytes < need || !aligned)) return XB_OK;
                               if (!workspace) return XB_ERR_NULL_POINTER;
                               if (workspace_bytes < need) return XB_ERR_WORKSPACE;
-                              if ((uintptr_t)workspace & 15u) return XB_ERR_MISALIGNED;
+                              if (!aligned) return XB_ERR_MISALIGNED;
                               *ptr = workspace;
                               return XB_OK;
                             });

@@ -508,7 +508,8 @@ def attention_kv_cache(
             )
         return out
     need = kv_cache_workspace_bytes(batch, chunk, num_heads, head_dim, start)
-    if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
+    if need and (workspace is None or workspace.device != qkv.device or not workspace.is_contiguous()
+                 or workspace.numel() * workspace.element_size() < need):
         workspace = torch.empty(need, device=qkv.device, dtype=torch.uint8)
     ws_ptr = workspace.data_ptr() if need else None
     ws_bytes = workspace.numel() * workspace.element_size() if need else 0

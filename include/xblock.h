@@ -228,8 +228,8 @@ int xb_attention_causal_vt(const void* qkv, const void* vt, void* out,
  * the keys over the GPU and needs a caller-provided workspace of
  * xb_attention_kv_cache_workspace_bytes(...) bytes (16-byte aligned); a
  * smaller one gives XB_ERR_WORKSPACE.  Longer chunks need none: with the bytes
- * the function gives (0 where there is nothing to gain) they split the keys
- * too, with less or NULL they don't.
+ * the function gives (0 where there is nothing to gain), 16-byte aligned, they
+ * split the keys too, with any other workspace or NULL they don't.
  */
 int xb_kv_cache_append(const void* qkv, void* k_cache, void* v_cache,
                        int32_t batch, int64_t chunk, int32_t heads,

@@ -734,6 +734,30 @@ def test_chunk_over_long_cache(pkg, cuda, b, heads, hd, start, chunk):
     assert torch.equal(pkg.attention_kv_cache(q, kc, vc, heads, start, no_alloc=True), out)
 
 
+def test_long_chunk_takes_any_workspace(pkg, cuda):
+    """A chunk that needs no workspace is not refused for the one it is given: an unaligned one
+    leaves the keys unsplit, and one on another device is replaced."""
+    b, heads, hd, start, chunk = 1, 2, 64, 6000, 40
+    length = start + chunk
+    qkv = torch.randn(b, length, 3 * heads * hd, generator=_gen(8)).half()
+    kc, vc = _fill_cache(pkg, qkv, heads, length, [start, chunk], cuda)
+    q = qkv[:, start:].contiguous().to(cuda)
+    need = pkg.kernels.kv_cache_workspace_bytes(b, chunk, heads, hd, start)
+    ws = torch.empty(need + 16, device=cuda, dtype=torch.uint8)[8:8 + need]
+    assert need > 0 and ws.data_ptr() % 16 == 8
+
+    def call(ptr, size):
+        out = torch.empty(b, chunk, heads * hd, device=cuda, dtype=F16)
+        assert pkg._capi.lib().xb_attention_kv_cache(
+            q.data_ptr(), kc.data_ptr(), vc.data_ptr(), out.data_ptr(), b, chunk, heads, hd, start, length, hd**-0.5,
+            ptr, size, pkg._capi.stream_handle(q.device)) == 0
+        return out
+
+    assert torch.equal(call(ws.data_ptr(), need), call(None, 0))
+    assert torch.equal(pkg.attention_kv_cache(q, kc, vc, heads, start, workspace=torch.empty(need, dtype=torch.uint8)),
+                       pkg.attention_kv_cache(q, kc, vc, heads, start))
+
+
 def test_decode_workspace_too_small(pkg, cuda):
     b, heads, hd, start = 1, 2, 64, 300
     qkv_full = torch.randn(b, start + 1, 3 * heads * hd, generator=_gen(3)).half()
