@@ -160,8 +160,12 @@ def kernel_costs(name: str, config, rows: int):
         # split form: per sequence and layer, K and V of tokens 0..63 (FP16) written once and read once
         handoff = b * layers * 2 * (2 * 64 * d * 2) if name.endswith("_split") else 0
         return rows * 8 * d + weights + handoff, 2.0 * rows * layers * (4 * d * d + 2 * d * f) + attn
-    if name.startswith("row_block"):  # context, residual stream in and out, next QKV
-        return rows * 16 * d, 2.0 * rows * (4 * d * d + 2 * d * f)
+    if name.startswith("row_block"):
+        if name.endswith("_first"):   # x in; QKV out
+            return rows * 10 * d, 2.0 * rows * 3 * d * d
+        if name.endswith("_last"):    # context, residual stream in; y out
+            return rows * 10 * d, 2.0 * rows * (d * d + 2 * d * f)
+        return rows * 16 * d, 2.0 * rows * (4 * d * d + 2 * d * f)  # context, residual stream in and out, next QKV
     if name.startswith("gemm_"):
         parts = name.split("_")
         n, k = int(parts[1][1:]), int(parts[2][1:])

@@ -601,8 +601,9 @@ def row_block(
         if t is not None:
             _check_buffer(t, shape, dtype, residual.device, what)
     valid = None if row_valid is None else _byte_mask(row_valid, rows, residual.device, "row_valid")
+    form = "first" if layer < 0 else "last" if layer + 1 == stack.layers else "mid"
     check(
-        _launch(f"row_block_{d}", lambda: lib().xb_row_block(
+        _launch(f"row_block_{d}_{form}", lambda: lib().xb_row_block(
             ctypes.addressof(stack), layer, residual.data_ptr(), _ptr(ctx), _ptr(residual_out), _ptr(qkv), _ptr(out),
             _ptr(valid), rows, stream_handle(residual.device))),
         "xb_row_block",

@@ -58,6 +58,18 @@ def test_kernel_costs_match_the_formulas(pkg):
     assert bench.kernel_costs("kv_append_hd64", cfg2, m2) == (0.0, 0.0)
 
 
+@pytest.mark.parametrize("layers", [1, 2, 4])
+def test_row_block_costs_add_up_to_the_forward(pkg, layers):
+    """The three forms of a row-block launch: a forward's first, layers - 1 middle and last launch
+    do the stack's products once, and move x in, y out, and QKV, the residual stream and the context
+    between them."""
+    config = pkg.TransformerConfig(3, 200, 64, 4, 256, layers, True)
+    m, d, f = 600, 64, 256
+    first, mid, last = (bench.kernel_costs(f"row_block_64_{form}", config, m) for form in ("first", "mid", "last"))
+    assert first[1] + (layers - 1) * mid[1] + last[1] == 2.0 * m * layers * (4 * d * d + 2 * d * f)
+    assert first[0] == m * d * (4 + 6) and mid[0] == m * d * (2 + 4 + 4 + 6) and last[0] == m * d * (2 + 4 + 4)
+
+
 def test_trial_rows_follow_the_reference_trials(pkg):
     shapes = pkg.OFFICIAL_BENCHMARK_SHAPES
     for shape_id in (1, 8, 11):                       # small configs: every sequence of each trial

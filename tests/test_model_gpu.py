@@ -951,3 +951,17 @@ def test_ffn_of_another_width_in_one_layer(pkg, cuda, geom, width):
     model.layers[0].norm2 = torch.nn.LayerNorm(geom[2] // 2).to(cuda)
     with torch.inference_mode(), pytest.raises(ValueError, match="do not match the input width"):
         model(x.to(cuda))
+
+
+@pytest.mark.parametrize("layers", [1, 3])
+def test_row_block_launches_are_recorded_by_form(pkg, cuda, layers):
+    """The recorder names a forward's first, middle and last row-block launches apart: they move
+    and compute different amounts."""
+    kernels = __import__(pkg.__name__ + ".kernels", fromlist=["LaunchRecorder"])
+    model = pkg.UserOptimizedTransformer(pkg.TransformerConfig(2, 150, 64, 4, 64, layers, True)).to(cuda).eval()
+    x = torch.randn(2, 150, 64, device=cuda)
+    with torch.inference_mode(), kernels.LaunchRecorder() as recorder:
+        model(x)
+    torch.cuda.synchronize()
+    counts = {name: len(times) for name, times in recorder.durations_ms().items() if name.startswith("row_block")}
+    assert counts == {"row_block_64_first": 1, "row_block_64_last": 1, **({"row_block_64_mid": layers - 1} if layers > 1 else {})}
