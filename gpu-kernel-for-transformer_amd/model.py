@@ -41,7 +41,6 @@ from __future__ import annotations
 
 import ctypes
 import dataclasses
-import functools
 import itertools
 import operator
 from typing import Dict, NamedTuple, Optional, Tuple
@@ -120,26 +119,27 @@ def _tree_changed(*_args) -> None:
 nn.modules.module.register_module_parameter_registration_hook(_tree_changed)
 nn.modules.module.register_module_module_registration_hook(_tree_changed)
 
-_CHILDREN, _PARAMETERS = operator.attrgetter("_modules"), operator.attrgetter("_parameters")
-_VALUES = operator.methodcaller("values")
-_IS_NONE = functools.partial(operator.is_, None)
+_FLATTEN = itertools.chain.from_iterable
 
 
 class _Tree(NamedTuple):
-    """A walk of a model's modules (the model itself left out)."""
+    """A walk of a model's modules.  The registries are the modules' own dicts, so looking
+    through them again costs 1 to 2 us where walking the modules costs tens."""
 
     params: Tuple[nn.Parameter, ...]
     norms: Tuple[nn.LayerNorm, ...]
     attentions: Tuple[nn.Module, ...]
     generation: int
-    containers: Tuple[nn.Module, ...]  # modules with children
-    children: Tuple[nn.Module, ...]    # of the model, then of each container
-    holders: Tuple[nn.Module, ...]     # modules with parameters
+    children: Tuple[nn.Module, ...]
+    child_registries: Tuple[dict, ...]      # `_modules` of every module that has children
+    parameter_registries: Tuple[dict, ...]  # `_parameters` of every module that has some
 
-    def live_parameters(self) -> Tuple[torch.Tensor, ...]:
-        """What the holders hold now: torch.func.functional_call swaps tensors in without registering them."""
-        held = itertools.chain.from_iterable(map(_VALUES, map(_PARAMETERS, self.holders)))
-        return tuple(itertools.filterfalse(_IS_NONE, held))
+    def live_children(self) -> Tuple[nn.Module, ...]:
+        return tuple(_FLATTEN(map(dict.values, self.child_registries)))
+
+    def live_parameters(self) -> Tuple[Optional[torch.Tensor], ...]:
+        """What the modules hold now: torch.func.functional_call swaps tensors in without registering them."""
+        return tuple(_FLATTEN(map(dict.values, self.parameter_registries)))
 
 
 class _LayerWeights:
@@ -235,7 +235,9 @@ class UserOptimizedTransformer(nn.Module):
         eligibility (the enable_fused_stack toggle, LayerNorm eps and affine);
         per_op=True asks for the per-op sequence (KV-cached steps).
         """
-        key = (int(batch), int(seq_len), bool(padded), self._fused_stack_eligible() and not per_op, bool(per_op),
+        # Only a width-128 model can be eligible: the others don't pay for the question.
+        eligible = not per_op and self.config.d_model == 128 and self._fused_stack_eligible()
+        key = (int(batch), int(seq_len), bool(padded), eligible, bool(per_op),
                self._fused_stack_enabled)
         plans = self.__dict__.setdefault("_plans", {})
         plan = plans.get(key)
@@ -344,19 +346,22 @@ class UserOptimizedTransformer(nn.Module):
         """Whether every parameter is what the native kernels index it as: of the config's
         sizes, all on one device, LayerNorms in contiguous float32."""
         d, f = self.config.d_model, self.config.ffn_dim
-        device = self.final_norm.weight.device
-        norms = [self.final_norm]
+        square, norms, held = (d, d), [self.final_norm], []
         for layer in self.layers:
             att = layer.attention
             norms += [layer.norm1, layer.norm2]
-            for lin, n, k in ((att.q_proj, d, d), (att.k_proj, d, d), (att.v_proj, d, d), (att.out_proj, d, d),
-                              (layer.ffn_in, f, d), (layer.ffn_out, d, f)):
-                if lin.bias is None or tuple(lin.weight.shape) != (n, k) or tuple(lin.bias.shape) != (n,):
+            for lin, shape in ((att.q_proj, square), (att.k_proj, square), (att.v_proj, square), (att.out_proj, square),
+                               (layer.ffn_in, (f, d)), (layer.ffn_out, (d, f))):
+                weight, bias = lin.weight, lin.bias
+                if bias is None or weight.shape != shape or bias.shape != shape[:1]:
                     return False
-                if lin.weight.device != device or lin.bias.device != device:
+                held += [weight, bias]
+        for norm in norms:
+            for p in (norm.weight, norm.bias):
+                if p is None or p.numel() != d or p.dtype != torch.float32 or not p.is_contiguous():
                     return False
-        return all(p.numel() == d and p.dtype == torch.float32 and p.device == device and p.is_contiguous()
-                   for norm in norms for p in (norm.weight, norm.bias))
+                held.append(p)
+        return len({p.device for p in held}) == 1
 
     def _native_stack(self, row_block: bool) -> Optional[Tuple[_capi.XbStack, object, object, torch.device]]:
         """(xb_stack, its xb_block array, the tensors they point into, their device), cached by parameter version.
@@ -364,7 +369,7 @@ class UserOptimizedTransformer(nn.Module):
         row_block: with fragment-packed weights for xb_row_block instead of
         the FP16 copies the GEMMs read.
 
-        None when a LayerNorm has no weight or bias, or a parameter does not
+        None when a parameter is missing or does not
         fit the config (_fits_config): the kernels would take its size from
         the config.  The wrappers, which take each size from the tensor
         itself, then run the forward or raise.  The descriptors are written
@@ -372,14 +377,12 @@ class UserOptimizedTransformer(nn.Module):
         share them.
         """
         tree = self._walk()
-        for norm in tree.norms:  # read on each call: setting one to None calls no registration hook
-            registered = norm._parameters
-            if registered.get("weight") is None or registered.get("bias") is None:
-                return None
         params = tree.live_parameters()
         settings = (row_block, self.config, [n.eps for n in tree.norms], [a.scale for a in tree.attentions])
         try:
             key = (tuple(map(_VERSION_OF, params)), tuple(map(torch.Tensor.data_ptr, params)), settings)
+        except AttributeError:  # one is None (setting it calls no registration hook)
+            return None
         except RuntimeError:  # inference-mode parameters have no version counter: never reuse
             key = None
         cached = self.__dict__.get("_native_stack_cache")
@@ -419,19 +422,15 @@ class UserOptimizedTransformer(nn.Module):
         """This model's modules and parameters, re-walked after any registration or change of the modules."""
         cached = self.__dict__.get("_tree_cache")
         if (cached is None or cached.generation != _TREE_GENERATION[0]
-                or self._children_of(cached.containers) != cached.children):
-            modules = tuple(m for m in self.modules() if m is not self)
-            containers = tuple(m for m in modules if m._modules)
+                or cached.live_children() != cached.children):
+            modules = tuple(self.modules())
+            registries = tuple(m._modules for m in modules if m._modules)
             cached = _Tree(params=tuple(self.parameters()), norms=tuple(m for m in modules if isinstance(m, nn.LayerNorm)),
                            attentions=tuple(layer.attention for layer in self.layers), generation=_TREE_GENERATION[0],
-                           containers=containers, children=self._children_of(containers),
-                           holders=tuple(m for m in modules if m._parameters))
+                           children=tuple(_FLATTEN(map(dict.values, registries))), child_registries=registries,
+                           parameter_registries=tuple(m._parameters for m in modules if m._parameters))
             self.__dict__["_tree_cache"] = cached
         return cached
-
-    def _children_of(self, containers: Tuple[nn.Module, ...]) -> Tuple[nn.Module, ...]:
-        return tuple(itertools.chain(self._modules.values(),
-                                     itertools.chain.from_iterable(map(_VALUES, map(_CHILDREN, containers)))))
 
     def _fused_stack_eligible(self) -> bool:
         """Conditions of the whole-stack kernel beyond the shape: the toggle, LayerNorm eps 1e-5 with affine."""
