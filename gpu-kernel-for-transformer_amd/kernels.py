@@ -76,9 +76,10 @@ def _device_is_gfx950(index: int) -> bool:
 
 def _require_device(tensor: torch.Tensor, what: str) -> None:
     lib()
-    if tensor.device.type != "cuda":
+    device = tensor.device
+    if device.type != "cuda":
         raise ValueError(f"{what} requires GPU tensors")
-    if not _device_is_gfx950(tensor.device.index if tensor.device.index is not None else torch.cuda.current_device()):
+    if not _device_is_gfx950(device.index if device.index is not None else torch.cuda.current_device()):
         raise RuntimeError(f"{what}: the xblock kernels are built for gfx950 only")
 
 
@@ -560,6 +561,7 @@ def stack_forward(
     """
     _require_device(x, "stack_forward")
     batch, seq_len, _ = x.shape
+    device = x.device
     if caches is not None and len(caches) != 2 * stack.layers:
         raise ValueError(f"{stack.layers} layers need {2 * stack.layers} cache pointers, got {len(caches)}")
     if caches is None:
@@ -569,11 +571,11 @@ def stack_forward(
                                                   variants[4], cache_start))
     if need < 0:
         check(need, "xb_stack_workspace_bytes")
-    workspace = torch.empty(need, device=x.device, dtype=torch.uint8)
+    workspace = torch.empty(need, device=device, dtype=torch.uint8)
     check(
         lib().xb_stack_forward(
             ctypes.addressof(stack), x.data_ptr(), out.data_ptr(), _ptr(token_valid), batch, seq_len, *variants,
-            caches, cache_start, cache_capacity, workspace.data_ptr(), need, stream_handle(x.device)),
+            caches, cache_start, cache_capacity, workspace.data_ptr(), need, stream_handle(device)),
         "xb_stack_forward",
     )
     return out

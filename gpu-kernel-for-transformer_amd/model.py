@@ -90,6 +90,7 @@ class TransformerBlockParameters(nn.Module):
         raise RuntimeError("run blocks through UserOptimizedTransformer.forward")
 
 
+_DEVICE_OF, _EPS_OF, _SCALE_OF = map(operator.attrgetter, ("device", "eps", "scale"))
 _VERSION_OF = operator.attrgetter("_version")  # raises RuntimeError on inference tensors, as _version does
 
 
@@ -207,6 +208,7 @@ class UserOptimizedTransformer(nn.Module):
         self._triton_fused_norm_enabled = True
         self._triton_fused_ffn_enabled = True
         self._attention_fp16_accumulation_enabled = False
+        self._walk()
 
     # What the forward derives from the module and rebuilds when it is missing.  A copy or a
     # saved file leaves it out (the descriptor's pointers are this process's and this model's),
@@ -346,25 +348,31 @@ class UserOptimizedTransformer(nn.Module):
         """Whether every parameter is what the native kernels index it as: of the config's
         sizes, all on one device, LayerNorms in contiguous float32."""
         d, f = self.config.d_model, self.config.ffn_dim
-        square, norms, held = (d, d), [self.final_norm], []
+        square, vector = (d, d), (d,)
+        tensors, norms = [], [self.final_norm]
         for layer in self.layers:
-            att = layer.attention
-            norms += [layer.norm1, layer.norm2]
-            for lin, shape in ((att.q_proj, square), (att.k_proj, square), (att.v_proj, square), (att.out_proj, square),
-                               (layer.ffn_in, (f, d)), (layer.ffn_out, (d, f))):
-                weight, bias = lin.weight, lin.bias
+            parts = layer._modules  # read directly: nn.Module.__getattr__ made this a tenth of a first forward
+            projections = parts["attention"]._modules
+            norms += (parts["norm1"], parts["norm2"])
+            for module, shape in ((projections["q_proj"], square), (projections["k_proj"], square),
+                                  (projections["v_proj"], square), (projections["out_proj"], square),
+                                  (parts["ffn_in"], (f, d)), (parts["ffn_out"], (d, f))):
+                held = module._parameters
+                weight, bias = held.get("weight"), held.get("bias")
+                if weight is None or bias is None:
+                    weight, bias = module.weight, module.bias  # parametrized, or missing
                 if bias is None or weight.shape != shape or bias.shape != shape[:1]:
                     return False
-                held += [weight, bias]
+                tensors += (weight, bias)
         for norm in norms:
             for p in (norm.weight, norm.bias):
-                if p is None or p.numel() != d or p.dtype != torch.float32 or not p.is_contiguous():
+                if p is None or p.shape != vector or p.dtype != torch.float32 or not p.is_contiguous():
                     return False
-                held.append(p)
-        return len({p.device for p in held}) == 1
+                tensors.append(p)
+        return len(set(map(_DEVICE_OF, tensors))) == 1
 
-    def _native_stack(self, row_block: bool) -> Optional[Tuple[_capi.XbStack, object, object, torch.device]]:
-        """(xb_stack, its xb_block array, the tensors they point into, their device), cached by parameter version.
+    def _native_stack(self, row_block: bool) -> Optional[Tuple[_capi.XbStack, object, object, int]]:
+        """(xb_stack, its xb_block array, the tensors they point into, their GPU), cached by parameter version.
 
         row_block: with fragment-packed weights for xb_row_block instead of
         the FP16 copies the GEMMs read.
@@ -378,7 +386,7 @@ class UserOptimizedTransformer(nn.Module):
         """
         tree = self._walk()
         params = tree.live_parameters()
-        settings = (row_block, self.config, [n.eps for n in tree.norms], [a.scale for a in tree.attentions])
+        settings = (row_block, self.config, tuple(map(_EPS_OF, tree.norms)), tuple(map(_SCALE_OF, tree.attentions)))
         try:
             key = (tuple(map(_VERSION_OF, params)), tuple(map(torch.Tensor.data_ptr, params)), settings)
         except AttributeError:  # one is None (setting it calls no registration hook)
@@ -409,7 +417,7 @@ class UserOptimizedTransformer(nn.Module):
                               final_eps=final.eps, final_affine=int(self._layer_norm_uses_affine(final)),
                               layers=len(self.layers), heads=cfg.num_heads, head_dim=cfg.head_dim,
                               ffn_dim=cfg.ffn_dim, causal=int(cfg.causal))
-        value = (stack, blocks, weights, final.weight.device)
+        value = (stack, blocks, weights, final.weight.get_device())
         self.__dict__["_native_stack_cache"] = (key, value)
         return value
 
@@ -552,6 +560,9 @@ class UserOptimizedTransformer(nn.Module):
 
     def _forward_impl(self, x: torch.Tensor, valid_token_mask: Optional[torch.Tensor],
                       out: Optional[torch.Tensor]) -> torch.Tensor:
+        if torch.is_grad_enabled():  # entering no_grad costs 1 us: only where it changes anything
+            with torch.no_grad():
+                return self._forward_impl(x, valid_token_mask, out)
         if x.device.type != "cuda":
             raise RuntimeError(
                 "UserOptimizedTransformer runs only on the gfx950 HIP path; move the model and "
@@ -587,21 +598,19 @@ class UserOptimizedTransformer(nn.Module):
         if self._kv_cache_enabled:
             if token_valid is not None:
                 raise ValueError("KV-cached decoding does not support padding")
-            with torch.no_grad():
-                result = self._forward_hip_cached(x)
+            result = self._forward_hip_cached(x)
             return result if out is None else out.copy_(result)
         plan = self.execution_plan(x.shape[0], x.shape[1])
         chunk = self._large_batch_chunk_size or plan.batch_chunk_size  # as _chunk_size
-        with torch.no_grad():
-            if chunk and x.shape[0] > chunk:
-                output = torch.empty_like(x) if out is None else out
-                for start in range(0, x.shape[0], chunk):
-                    end = min(start + chunk, x.shape[0])
-                    self._forward_hip(x[start:end], out=output[start:end],
-                                      token_valid=None if token_valid is None else token_valid[start:end])
-                return output
-            # An unpadded whole batch runs the plan just looked up.
-            return self._forward_hip(x, out=out, token_valid=token_valid, plan=plan if token_valid is None else None)
+        if chunk and x.shape[0] > chunk:
+            output = torch.empty_like(x) if out is None else out
+            for start in range(0, x.shape[0], chunk):
+                end = min(start + chunk, x.shape[0])
+                self._forward_hip(x[start:end], out=output[start:end],
+                                  token_valid=None if token_valid is None else token_valid[start:end])
+            return output
+        # An unpadded whole batch runs the plan just looked up.
+        return self._forward_hip(x, out=out, token_valid=token_valid, plan=plan if token_valid is None else None)
 
     def _forward_hip(self, x: torch.Tensor, out: Optional[torch.Tensor] = None,
                      token_valid: Optional[torch.Tensor] = None,
@@ -742,7 +751,7 @@ class UserOptimizedTransformer(nn.Module):
         if plan.row_block and self.config.d_model == 32 and x.data_ptr() % 16:
             x = x.clone()  # this width's LayerNorm takes any alignment, the row blocks 16 bytes
         native = None if kernels.recording() else self._native_stack(plan.row_block)
-        if native is None or native[3] != x.device:
+        if native is None or native[3] != x.get_device():
             return self._per_op_forward_stepwise(x, plan, out, token_valid, cache_start)
         if out is None:
             out = torch.empty_like(x)
@@ -769,7 +778,7 @@ class UserOptimizedTransformer(nn.Module):
                                  token_valid: Optional[torch.Tensor], cache_start: Optional[int]) -> torch.Tensor:
         """_per_op_forward, one wrapper call per launch."""
         native = self._native_stack(True) if plan.row_block else None
-        if native is not None and native[3] == x.device:
+        if native is not None and native[3] == x.get_device():
             return self._row_block_forward_stepwise(x, native[0], plan, out, token_valid, cache_start)
         cfg = self.config
         batch, seq_len, d_model = x.shape
