@@ -410,11 +410,12 @@ class UserOptimizedTransformer(nn.Module):
                 setattr(block, which + "_g", norm.weight.data_ptr())
                 setattr(block, which + "_b", norm.bias.data_ptr())
                 setattr(block, which + "_eps", norm.eps)
-                setattr(block, which + "_affine", int(self._layer_norm_uses_affine(norm)))
+                # The row blocks always apply it; asking costs two reads from the device.
+                setattr(block, which + "_affine", int(row_block or self._layer_norm_uses_affine(norm)))
             block.scale = layer.attention.scale
         final = self.final_norm
         stack = _capi.XbStack(blocks=blocks, final_g=final.weight.data_ptr(), final_b=final.bias.data_ptr(),
-                              final_eps=final.eps, final_affine=int(self._layer_norm_uses_affine(final)),
+                              final_eps=final.eps, final_affine=int(row_block or self._layer_norm_uses_affine(final)),
                               layers=len(self.layers), heads=cfg.num_heads, head_dim=cfg.head_dim,
                               ffn_dim=cfg.ffn_dim, causal=int(cfg.causal))
         value = (stack, blocks, weights, final.weight.get_device())

@@ -479,3 +479,19 @@ def test_stack_forward_argument_checks(capi):
     assert call(valid=16, caches=16) == -2 and call(caches=16, start=-1) == -2
     stack.layers = 0
     assert call() == -2
+
+
+def test_row_block_descriptor_reads_nothing_from_the_device(pkg, monkeypatch):
+    """Row blocks apply every LayerNorm's affine: their descriptor doesn't ask whether it is (1, 0),
+    which takes two reads from the device per LayerNorm, and the per-op one does."""
+    import importlib
+
+    kernels = importlib.import_module(pkg.__name__ + ".kernels")
+    monkeypatch.setattr(kernels, "pack_linear_fragments", lambda w, out: out.copy_(w.detach().flatten()))
+    model = pkg.UserOptimizedTransformer(pkg.TransformerConfig(2, 300, 64, 4, 64, 2, True)).eval()
+    asked = []
+    monkeypatch.setattr(type(model), "_layer_norm_uses_affine", staticmethod(lambda norm: asked.append(norm) or False))
+    stack, blocks, _ = model._native_stack(True)[:3]
+    assert not asked and stack.final_affine == blocks[0].norm1_affine == blocks[1].norm2_affine == 1
+    stack, blocks, _ = model._native_stack(False)[:3]
+    assert len(asked) == 5 and stack.final_affine == blocks[0].norm1_affine == 0
