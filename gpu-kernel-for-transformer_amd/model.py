@@ -40,7 +40,6 @@ reference (TTB:503-508) there is no sequence-length limit: the key mask is a
 from __future__ import annotations
 
 import ctypes
-import dataclasses
 import itertools
 import operator
 from typing import Dict, NamedTuple, Optional, Tuple
@@ -213,7 +212,7 @@ class UserOptimizedTransformer(nn.Module):
     # What the forward derives from the module and rebuilds when it is missing.  A copy or a
     # saved file leaves it out (the descriptor's pointers are this process's and this model's),
     # and what a file saved with it holds is not taken over.
-    _DERIVED = ("_native_stack_cache", "_weight_cache", "_fused_stack_cache", "_tree_cache", "_mask_cache", "_side_streams")
+    _DERIVED = ("_native_stack_cache", "_weight_cache", "_fused_stack_cache", "_tree_cache", "_mask_cache")
 
     def __getstate__(self) -> dict:
         """The state that copy.deepcopy, pickle and torch.save take."""
@@ -634,82 +633,17 @@ class UserOptimizedTransformer(nn.Module):
                                               split=plan.fused_variant == _capi.XB_FUSED_SPLIT,
                                               strict=self._strict_handoff_checks)
 
-        # Not for row blocks: nine short launches gain nothing from running beside nine more
-        # (64 x 128 tokens of width 32: 47 us in one stream, 82 us in two).
-        streams = None if plan.row_block else self._overlap_streams(x)
-        if streams is not None and torch.cuda.is_current_stream_capturing():
-            return self._per_op_forward_overlapped(x, plan, streams, out, token_valid)
         return self._per_op_forward(x, plan, out=out, token_valid=token_valid)
 
-    # A small per-op forward captured into a hipGraph runs as two half-batches
-    # on two streams forked from the capturing stream and joined back into it.
-    # Each half takes the GEMM tiles the plan picks for its own row count for
-    # the output projection and the FFN (128 x 128 at 4096 rows: 256 tiles,
-    # every CU, instead of 128 x 256 tiles that leave half of them idle at
-    # that size), so the two halves' single-round grids run side by side and
-    # fill each other's ramp-up and drain; the QKV projection and the
-    # attention keep the whole batch's variants.  Every direct-to-LDS tile
-    # gives the same bits, and batch elements are independent, so the rows
-    # equal the whole batch's bit for bit.  Measured under graph replay, in
-    # one call: cfg3 725.8 -> 681.3 us; D = 1024 with 16 heads of 64 at the
-    # same size 730.5 -> 694.9 us.  With both halves on the whole batch's
-    # tiles the overlap gained nothing (734.7 us), and four streams no more
-    # than two.  Eager calls stay on one stream: there the host's per-launch
-    # cost, paid twice, outweighs it.
-    _OVERLAP_MAX_TOKENS = 32768
-
-    def _overlap_streams(self, x: torch.Tensor) -> Optional[Tuple[torch.cuda.Stream, torch.cuda.Stream]]:
-        """The two side streams of x's device for an overlapped capture, or None when x does not qualify.
-
-        Made on the first qualifying call outside capture (the eager warm-up
-        calls before a capture are such calls), at the default priority.
-        """
-        if x.shape[0] < 2 or x.shape[0] * x.shape[1] > self._OVERLAP_MAX_TOKENS:
-            return None
-        per_device = self.__dict__.setdefault("_side_streams", {})
-        streams = per_device.get(x.device.index)
-        if streams is None and not torch.cuda.is_current_stream_capturing():
-            streams = (torch.cuda.Stream(device=x.device), torch.cuda.Stream(device=x.device))
-            per_device[x.device.index] = streams
-        return streams
-
     def captured_overlap(self, batch: int, seq_len: int, padded: bool = False) -> Optional[str]:
-        """What a forward of [batch, seq_len] captured into a hipGraph runs beyond its plan, or None.
+        """What a captured forward of [batch, seq_len] runs beyond its plan: None, the plan's launches on one stream.
 
-        A captured small per-op forward runs as two half-batches on two
-        streams, each with its own GEMM tiles for the output projection and
-        the FFN (see _OVERLAP_MAX_TOKENS); this names them.
+        Two half-batches on two streams are slower at every size tried (us per replay, two
+        streams / one: 64 x 128 tokens of width 1024, 4 layers 684 / 663; 16 x 512, width 768,
+        2 layers 415 / 376; 4 x 128, width 256, 4 layers 285 / 112): the GEMM tiles already put
+        two blocks on a CU, and a graph with two branches costs more per launch.
         """
-        plan = self.execution_plan(batch, seq_len, padded=padded)
-        if (plan.fused or plan.row_block or batch < 2 or batch * seq_len > self._OVERLAP_MAX_TOKENS
-                or self._kv_cache_enabled):
-            return None
-        halves = sorted({(batch + 1) // 2, batch // 2}, reverse=True)
-        own = [self.execution_plan(h, seq_len, padded=padded, per_op=True) for h in halves]
-        names = ", ".join(f"{h} sequences: out {p.projection_strategy.split('out ')[-1]}, FFN {p.ffn_strategy}"
-                          for h, p in zip(halves, own))
-        return f"two half-batch streams under capture ({names}); QKV and attention as planned"
-
-    def _per_op_forward_overlapped(self, x: torch.Tensor, plan: ShapeExecutionPlan,
-                                   streams: Tuple[torch.cuda.Stream, torch.cuda.Stream],
-                                   out: Optional[torch.Tensor], token_valid: Optional[torch.Tensor]) -> torch.Tensor:
-        """_per_op_forward of each half of the batch on its own stream, joined back into the current one."""
-        batch, seq_len = x.shape[0], x.shape[1]
-        if out is None:
-            out = torch.empty_like(x)
-        main = torch.cuda.current_stream(x.device)
-        half = (batch + 1) // 2
-        for stream, (start, end) in zip(streams, ((0, half), (half, batch))):
-            valid = None if token_valid is None else token_valid[start:end]
-            own = self.execution_plan(end - start, seq_len, padded=token_valid is not None, per_op=True)
-            half_plan = dataclasses.replace(plan, out_variant=own.out_variant, ffn_in_variant=own.ffn_in_variant,
-                                            ffn_out_variant=own.ffn_out_variant)
-            stream.wait_stream(main)
-            with torch.cuda.stream(stream):
-                self._per_op_forward(x[start:end], half_plan, out=out[start:end], token_valid=valid)
-        for stream in streams:
-            main.wait_stream(stream)
-        return out
+        return None
 
     def _forward_hip_cached(self, x: torch.Tensor) -> torch.Tensor:
         """One KV-cached step: append this chunk's keys/values per layer, attend over the cache.
