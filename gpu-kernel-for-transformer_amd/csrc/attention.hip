@@ -1031,14 +1031,16 @@ static bool attention_variant_fits(int variant, int hd, bool masked) {
 // 1024, 17.3 / 15.4; 40 x 216 x 8, 1280, 14.1 / 13.1).  64 queries per wave from
 // 16384 queries or 2048 blocks of at least 4096 queries on.  The ping-pong
 // kernel (head_dim 64, no key mask) is ahead from 16384 queries on (1 x 16384
-// x 16 530 us, 1 x 32768 x 16 2025 against 2073) and behind below (8 x 4096 x
-// 16 388 against 344, 1 x 8000 x 16 206 against 177); with 32 heads and more
-// it keeps the plans past 4096 queries, where it is within 2 to 9 % (2 x 4128
-// x 16 120 with V handed over transposed, 126 without, against 117; 4 x 8192 x
-// 16 629 and 643 against 620).
+// x 16 530 us, 1 x 32768 x 16 2025 against 2073), with 32 heads and more from
+// 12288 on, and behind below (ping-pong / 32 / 64 queries per wave: 2 x 4128 x
+// 16 132 / 115 / 128, 2 x 8192 x 16 376 / 316 / 365, 4 x 10000 x 16 898 / 884 /
+// 887, 2 x 12288 x 16 657 / 667 / 641, 2 x 14336 x 16 804 / 914 / 822, 8 x 14336
+// x 16 3276 / 3506 / 3444).  V handed over transposed does not move that line:
+// one layer of width 1024 takes 673 against 611 us at 2 x 8192 tokens, 9441
+// against 9368 at 32 x 8192 and 8466 against 8619 at 16 x 12288.
 static int select_attention(int64_t B, int S_q, int H, int hd, bool masked) {
   if (hd >= 256) return S_q <= 128 && B * H >= kCUs ? XB_ATTN_W8_Q16 : XB_ATTN_W4_Q16;
-  if (hd == 64 && !masked && (S_q >= 16384 || (S_q > 4096 && B * H >= 32))) return XB_ATTN_PINGPONG;
+  if (hd == 64 && !masked && (S_q >= 16384 || (S_q >= 12288 && B * H >= 32))) return XB_ATTN_PINGPONG;
   const int64_t blocks = (int64_t)(S_q + 63) / 64 * B * H;
   if (S_q <= 64 || blocks <= (hd >= 128 ? 480 : 960)) return XB_ATTN_W4_Q16;
   if (hd >= 128) return XB_ATTN_W4_Q32;

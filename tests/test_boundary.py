@@ -86,6 +86,9 @@ def test_variant_selection_abi(capi):
     assert lib.xb_select_attention(8, 128, 4, 256, 0) == 0           # too few blocks for that
     assert lib.xb_select_attention(32, 100000, 16, 64, 0) == 4
     assert lib.xb_select_attention(32, 100000, 16, 64, 1) == 2
+    # head_dim 64 without a mask: the ping-pong kernel from 16384 queries on, from 12288 with 32 heads
+    for batch, s, variant in ((2, 4128, 1), (2, 12287, 1), (4, 12287, 2), (2, 12288, 4), (1, 12288, 1), (1, 16384, 4)):
+        assert lib.xb_select_attention(batch, s, 16, 64, 0) == variant, (batch, s)
     assert lib.xb_select_attention(1, 8, 2, 24, 0) == -4
     assert lib.xb_select_fused_d128(64, 128, 4, 128, 1, 0) == 1
     assert lib.xb_select_fused_d128(10000, 128, 4, 128, 1, 0) == 0

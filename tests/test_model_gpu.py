@@ -119,20 +119,21 @@ def test_transposed_v_forward_matches_plain_plan(pkg, cuda):
     """A long head_dim-64 causal forward takes V transposed from the QKV GEMM
     (plan: flash_pingpong_vt); the same model with the plan resolved without
     it (plain QKV GEMM + ping-pong attention) gives the same output bit for
-    bit, here at S = 4128 (rows padded to 4160)."""
+    bit, here at S = 12320 (rows padded to 12352)."""
     capi = pkg._capi
-    config = pkg.TransformerConfig(2, 4128, 1024, 16, 1024, 2, True)
+    config = pkg.TransformerConfig(4, 12320, 1024, 16, 1024, 2, True)
     _, optimized = _models(pkg, config, cuda)
-    x = torch.randn(2, 4128, 1024, generator=torch.Generator(device=cuda).manual_seed(11), device=cuda)
-    plan = optimized.execution_plan(2, 4128)
+    x = torch.randn(4, 12320, 1024, generator=torch.Generator(device=cuda).manual_seed(11), device=cuda)
+    plan = optimized.execution_plan(4, 12320)
     assert plan.attention_variant == capi.XB_ATTN_PINGPONG_VT and "flash_pingpong_vt" in plan.describe()
     with torch.inference_mode():
         out_vt = optimized(x).clone()
-        optimized._large_batch_chunk_size = 1  # one sequence per slice, each with its own V^T buffer
+        optimized._large_batch_chunk_size = 2  # two sequences per slice, each slice with its own V^T buffer
+        assert optimized.execution_plan(2, 12320).attention_variant == capi.XB_ATTN_PINGPONG_VT
         assert torch.equal(optimized(x), out_vt)
         optimized._large_batch_chunk_size = 0
     key = next(k for k, v in optimized._plans.items() if v is plan)
-    optimized._plans[key] = pkg.resolve_shape_execution_plan(config, 2, 4128, transposed_v_allowed=False)
+    optimized._plans[key] = pkg.resolve_shape_execution_plan(config, 4, 12320, transposed_v_allowed=False)
     assert optimized._plans[key].attention_variant == capi.XB_ATTN_PINGPONG
     with torch.inference_mode():
         out_plain = optimized(x)
@@ -778,7 +779,7 @@ def test_random_geometries_against_oracle(pkg, cuda, geom):
     ((3, 70, 64, 4, 96, 3), True, False), ((3, 70, 64, 4, 96, 3), False, True),
     ((3, 70, 64, 4, 128, 3), False, True), ((2, 200, 128, 4, 256, 2), True, True),   # row blocks
     ((2, 129, 256, 8, 2048, 2), True, True),
-    ((2, 4128, 256, 4, 256, 1), True, False),      # V handed over transposed
+    ((8, 12288, 256, 4, 256, 1), True, False),     # V handed over transposed
     ((1, 1, 512, 8, 512, 2), True, False)])
 def test_native_sequence_is_the_stepwise_one(pkg, cuda, geom, causal, padded):
     """The native call issues the launches the wrappers issue one by one: the same
@@ -793,6 +794,7 @@ def test_native_sequence_is_the_stepwise_one(pkg, cuda, geom, causal, padded):
         valid = torch.ones(geom[0], geom[1], dtype=torch.uint8, device=cuda)
         valid[0, geom[1] // 2:] = 0
     plan = model.execution_plan(geom[0], geom[1], padded=padded)
+    assert (plan.attention_variant == pkg._capi.XB_ATTN_PINGPONG_VT) == (geom[1] == 12288)
 
     def both():
         with torch.no_grad():
