@@ -278,15 +278,15 @@ def test_causal_attention_long(pkg, cuda, hd, s):
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("b,s,h", [(2, 4096, 2), (1, 4133, 3), (1, 8703, 1)])
 def test_attention_long_hd64_ping_pong(pkg, cuda, b, s, h, causal):
-    """head_dim 64, S >= 4096, no mask: the ping-pong kernel (two wave groups, K/V
-    ring loaded straight into LDS).  FP32 reference, and bitwise equal to the
-    four-wave kernel, which an all-valid key mask selects: same 64-query waves,
-    same tile order and the same wave-uniform rescale decisions."""
+    """The ping-pong kernel (two wave groups, K/V ring loaded straight into LDS) at
+    lengths of few and ragged tiles.  FP32 reference, and bitwise equal to the
+    four-wave kernel, which an all-valid key mask selects: the same tile order
+    and the same rescale decisions per block of 16 queries."""
     hd = 64
     qkv = torch.randn(b, s, 3 * h * hd, generator=_gen(s + h)).half()
     ref = _attention_reference(qkv, h, causal=causal)
     qg = qkv.to(cuda)
-    out = pkg.attention(qg, h, causal=causal)
+    out = pkg.attention(qg, h, causal=causal, variant=pkg._capi.XB_ATTN_PINGPONG)
     torch.testing.assert_close(out.cpu().float(), ref, atol=2e-3, rtol=1e-2)
     ones = torch.ones(b, s, dtype=torch.bool, device=cuda)
     assert torch.equal(out, pkg.attention(qg, h, key_valid=ones, causal=causal))
