@@ -83,13 +83,16 @@ def test_maybe_cuda_graph_reasons(pkg, cuda):
     assert "KV-cache" in graphs.maybe_cuda_graph(model, x, None, enabled=True)[2]
     model.enable_kv_cache(False)
     assert "GPU input" in graphs.maybe_cuda_graph(model, x.cpu(), None, enabled=True)[2]
-    # with a padded mask the forward also converts the mask (two launches): captured
+    # a padded mask is read as it is: one kernel too, except where it has to be made contiguous first
     mask = torch.ones(4, 64, dtype=torch.bool, device=cuda)
     mask[1, 50:] = False
     runner, graphed, reason = graphs.maybe_cuda_graph(model, x, mask, enabled=True)
+    assert runner is model and not graphed and "one-kernel" in reason
+    strided = mask.t().contiguous().t()
+    runner, graphed, reason = graphs.maybe_cuda_graph(model, x, strided, enabled=True)
     assert graphed and runner is not model, reason
     with torch.inference_mode():
-        assert torch.equal(runner(x, mask), model(x, mask))
+        assert torch.equal(runner(x, strided), model(x, mask))
 
 
 @pytest.mark.parametrize("geom,masked", [((5, 96, 256, 4, 512, 2), False), ((7, 64, 1024, 4, 1024, 1), True),
