@@ -454,9 +454,11 @@ class UserOptimizedTransformer(nn.Module):
 
     def _fused_stack_parameters(self) -> Tuple[torch.Tensor, torch.Tensor, int]:
         """Fragment-packed FP16 weights, FP32 bias/LayerNorm buffer and LayerNorm affine mask, cached by version."""
-        params = self._walk().params
+        params = self._walk().live_parameters()
         try:
             key = (tuple(map(_VERSION_OF, params)), tuple(map(torch.Tensor.data_ptr, params)))
+        except AttributeError:  # a bias is None: the packing below raises for it
+            key = None
         except RuntimeError:  # inference-mode parameters have no version counter: never reuse
             key = None
         cached = self.__dict__.get("_fused_stack_cache")

@@ -299,6 +299,25 @@ def test_native_descriptor_follows_functional_call(pkg):
     assert model._native_stack(False)[1][0].norm1_g == own.norm1_g == model.layers[0].norm1.weight.data_ptr()
 
 
+def test_whole_stack_parameters_follow_functional_call(pkg, monkeypatch):
+    """The whole-stack form packs the parameters of the call as well."""
+    import importlib
+
+    kernels = importlib.import_module(pkg.__name__ + ".kernels")
+    monkeypatch.setattr(kernels, "pack_linear_fragments", lambda w, scale: (w.detach() * scale).half().flatten())
+    model = pkg.UserOptimizedTransformer(pkg.TransformerConfig(2, 64, 128, 4, 128, 1, True)).eval()
+    own = model._fused_stack_parameters()
+    assert model._fused_stack_parameters()[0] is own[0]
+    seen = []
+    model.forward = lambda: seen.append(model._fused_stack_parameters())
+    swapped = {name: p.detach() + 1.0 for name, p in model.named_parameters()}
+    torch.func.functional_call(model, swapped, ())
+    assert not torch.equal(seen[0][0], own[0]) and not torch.equal(seen[0][1], own[1])
+    assert torch.equal(seen[0][1][-256:-128], swapped["final_norm.weight"])
+    again = model._fused_stack_parameters()
+    assert torch.equal(again[0], own[0]) and torch.equal(again[1], own[1])
+
+
 def test_native_descriptor_follows_the_config(pkg):
     """The descriptor's causal flag is the present config's."""
     import dataclasses
