@@ -531,12 +531,9 @@ class UserOptimizedTransformer(nn.Module):
             padded = not self._all_tokens_valid(valid_token_mask, x.shape[1])
             if padded and not valid_token_mask.is_contiguous():
                 return False
-        chunk = self._chunk_size(x.shape[0], x.shape[1])
-        return self.execution_plan(x.shape[0], x.shape[1], padded=padded).fused and not (chunk and x.shape[0] > chunk)
-
-    def _chunk_size(self, batch: int, seq_len: int) -> int:
-        """Batch slice per launch sequence: the caller's _large_batch_chunk_size (TTB:1740), else the plan's."""
-        return self._large_batch_chunk_size or self.execution_plan(batch, seq_len).batch_chunk_size
+        plan = self.execution_plan(x.shape[0], x.shape[1], padded=padded)
+        chunk = self._large_batch_chunk_size or plan.batch_chunk_size  # the caller's (TTB:1740), else the plan's
+        return plan.fused and not (chunk and x.shape[0] > chunk)
 
     def _all_tokens_valid(self, valid_token_mask: Optional[torch.Tensor], seq_len: int) -> bool:
         """Mask inspection cached by identity + version + length (TTB:464-522)."""
@@ -606,8 +603,8 @@ class UserOptimizedTransformer(nn.Module):
                 raise ValueError("KV-cached decoding does not support padding")
             result = self._forward_hip_cached(x)
             return result if out is None else out.copy_(result)
-        plan = self.execution_plan(x.shape[0], x.shape[1])
-        chunk = self._large_batch_chunk_size or plan.batch_chunk_size  # as _chunk_size
+        plan = self.execution_plan(x.shape[0], x.shape[1], padded=token_valid is not None)
+        chunk = self._large_batch_chunk_size or plan.batch_chunk_size
         if chunk and x.shape[0] > chunk:
             output = torch.empty_like(x) if out is None else out
             for start in range(0, x.shape[0], chunk):
@@ -615,8 +612,7 @@ class UserOptimizedTransformer(nn.Module):
                 self._forward_hip(x[start:end], out=output[start:end],
                                   token_valid=None if token_valid is None else token_valid[start:end])
             return output
-        # An unpadded whole batch runs the plan just looked up.
-        return self._forward_hip(x, out=out, token_valid=token_valid, plan=plan if token_valid is None else None)
+        return self._forward_hip(x, out=out, token_valid=token_valid, plan=plan)
 
     def _forward_hip(self, x: torch.Tensor, out: Optional[torch.Tensor] = None,
                      token_valid: Optional[torch.Tensor] = None,
