@@ -238,15 +238,20 @@ def resolve_shape_execution_plan(
     # width divides D, so every tile is all Q/K or all V.
     if (transposed_v_allowed and attn == _capi.XB_ATTN_PINGPONG and config.causal and s % 32 == 0
             and d % 128 == 0 and d >= 256):
-        widths = {_capi.XB_LINEAR_DMA_256x256: 256, _capi.XB_LINEAR_DMA_128x256: 256, _capi.XB_LINEAR_DMA_128x128: 128}
+        widths = {_capi.XB_LINEAR_DMA_256x256: 256, _capi.XB_LINEAR_DMA_128x128: 128}
         if d % widths.get(qkv, d + 1) != 0:
             wide = d % 256 == 0 and qkv in (_capi.XB_LINEAR_DMA_256x256, _capi.XB_LINEAR_DMA_256x192)
             qkv = _capi.XB_LINEAR_DMA_256x256 if wide else _capi.XB_LINEAR_DMA_128x128
         attn = _capi.XB_ATTN_PINGPONG_VT
     lin = lambda v: _variant_name(lib, _capi.XB_OP_LINEAR, v)  # noqa: E731
+    # A few rows: xb_stack_forward's choice for 16-byte aligned inputs and LayerNorms.
+    norm_inside = lib.xb_select_norm_linear(rows, 3 * d, d) == 0 and lib.xb_select_norm_linear(rows, f, d) == 0
+    sequence = ("LayerNorm inside the QKV GEMM, attention, out GEMM, residual LayerNorm inside the FFN-in GEMM, FFN-out GEMM "
+                "per layer, final residual LayerNorm" if norm_inside else
+                "LayerNorm, QKV GEMM, attention, out GEMM, residual LayerNorm, FFN GEMMs per layer")
     return ShapeExecutionPlan(
         official_shape_id=shape_id, batch=b, seq_len=s, masked=masked, batch_chunk_size=chunk,
-        forward_strategy="per_op (LayerNorm, QKV GEMM, attention, out GEMM, residual LayerNorm, FFN GEMMs per layer)",
+        forward_strategy=f"per_op ({sequence})",
         ffn_strategy=f"{lin(ffn_in)}+gelu_erf / {lin(ffn_out)}",
         attention_strategy=_variant_name(lib, _capi.XB_OP_ATTENTION, attn),
         projection_strategy=f"qkv {lin(qkv)}, out {lin(out)}",

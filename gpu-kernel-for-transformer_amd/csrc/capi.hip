@@ -32,7 +32,7 @@ extern "C" const char* xb_variant_name(int op, int variant) {
     case XB_OP_LINEAR:
       switch (variant) {
         case XB_LINEAR_DMA_256x256: return "mfma_gemm_dma_256x256";
-        case XB_LINEAR_DMA_256x192: return "mfma_gemm_dma_256x192";
+        case XB_LINEAR_DMA_256x192: return "mfma_gemm_dma_256x192_by_2x128x192";
         case XB_LINEAR_DMA_128x256: return "mfma_gemm_dma_128x256";
         case XB_LINEAR_DMA_128x128: return "mfma_gemm_dma_128x128";
         case XB_LINEAR_NT_128x128: return "mfma_gemm_nt_128x128";

@@ -55,6 +55,7 @@ def test_shape_plan(pkg, capi):
     # D=1024: per-op kernels; the QKV GEMM's tile is the cost model's (256 x 192 for N = 3072)
     cfg3 = pkg.resolve_shape_execution_plan(shapes[8])
     assert not cfg3.fused and cfg3.qkv_variant == 1 and "mfma_gemm_dma_256x192" in cfg3.projection_strategy
+    assert "2x128x192" in cfg3.projection_strategy                                # the blocks that it launches
     assert cfg3.attention_strategy == "flash_8wave_128q"
     cfg5 = pkg.resolve_shape_execution_plan(shapes[14])
     assert cfg5.attention_strategy == "flash_pingpong_vt_8wave_512q" and cfg5.batch_chunk_size == 0
@@ -72,6 +73,11 @@ def test_shape_plan(pkg, capi):
     big = pkg.TransformerConfig(400, 100000, 1024, 16, 1024, 2, True)
     chunked = pkg.resolve_shape_execution_plan(big)
     assert 0 < chunked.batch_chunk_size < 400 and "batch_chunk=" in chunked.describe()
+    # up to 8 rows of some widths: LayerNorms inside the products
+    few = pkg.TransformerConfig(4, 2, 1024, 16, 1024, 2, True)
+    assert "LayerNorm inside the QKV GEMM" in pkg.resolve_shape_execution_plan(few).describe()
+    for more in (pkg.TransformerConfig(9, 1, 1024, 16, 1024, 2, True), pkg.TransformerConfig(4, 2, 256, 4, 256, 2, True)):
+        assert "per_op (LayerNorm, QKV GEMM" in pkg.resolve_shape_execution_plan(more).describe()
     general = pkg.resolve_shape_execution_plan(pkg.TransformerConfig(3, 5, 8, 2, 8, 1, True))
     assert general.official_shape_id is None and general.describe().startswith("general:")
 
@@ -99,8 +105,8 @@ def test_variant_selection_abi(capi):
     assert lib.xb_linear_v(16, 16, None, 16, 8192, 1024, 1024, 0, 1, None) == -10    # 256 x 192 needs N % 192
     assert lib.xb_attention_v(16, 16, None, 2, 64, 2, 32, 0.1, 1, 4, None) == -10     # ping-pong: head_dim 64 only
     assert lib.xb_attention_v(16, 16, 16, 2, 64, 2, 64, 0.1, 1, 4, None) == -10       # nor with a key mask
-    names = {lib.xb_variant_name(op, v) for op, n in ((0, 6), (1, 5), (2, 3)) for v in range(n)}
-    assert None not in names and len(names) == 14
+    names = {lib.xb_variant_name(op, v) for op, n in ((0, 8), (1, 6), (2, 3)) for v in range(n)}
+    assert None not in names and len(names) == 17
     assert lib.xb_variant_name(0, 99) is None
 
 
