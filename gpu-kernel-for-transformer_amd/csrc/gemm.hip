@@ -183,12 +183,16 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_nt_kernel(
 //
 // What is left over is each tile's start (the first slab's latency) and end
 // (the output stores), which nothing hides while a CU holds one tile: for
-// 8192 x 3072 x 1024 time against K put 17 of 55 us there.  So the tiles below
-// 256 x 256 are eight waves of at most 128 registers and at most 80 KB of LDS,
-// and a CU runs two of them, one starting or storing while the other
-// multiplies: 8192 x 3072 x 1024 54.5 -> 50.2 us (256 x 192 by one block ->
-// two of 128 x 192), 3001 x 3072 x 1024 26.1 -> 23.2 us, 8192 x 1024 x 1024
-// 21.0 -> 19.4 us (128 x 128 by four waves -> by eight).
+// 8192 x 3072 x 1024 time against K put 17 of 55 us there.  So the library
+// chooses, below 256 x 256, tiles of which a CU runs two and more, one
+// starting or storing while another multiplies: 128 x 192 and 128 x 128 by
+// eight waves (123 and 98 registers, 80 and 64 KB of LDS; two blocks) and 64 x
+// 64 (by eight waves with three stages, 43 registers and 48 KB: three blocks;
+// by four waves with two stages, 64 registers: five).  8192 x 3072 x 1024 54.5
+// -> 50.2 us (256 x 192 by one block -> two of 128 x 192), 3001 x 3072 x 1024
+// 26.1 -> 23.2 us, 8192 x 1024 x 1024 21.0 -> 19.4 us (128 x 128 by four waves
+// -> by eight).  128 x 256 (151 registers, 96 KB: one block) runs only when a
+// caller asks for it.
 //
 // LDS slab layout: the A rows (BM) and then the W rows (BN), 128 bytes each
 // (64 halves = eight 16-byte chunks).  Chunk c of row r lives at slot
@@ -621,8 +625,8 @@ static hipError_t launch_gemm(const half_t* a, const half_t* w, const float* bia
 }
 
 // Variants (XB_LINEAR_*): the gemm_dma_kernel tiles need K % 64 == 0 and K >=
-// 256 (256 x 192 also N % 192 == 0); the gemm_nt_kernel tiles take any K % 8
-// == 0; gemm_rows_kernel a few rows.
+// 256 (256 x 192, a pair of 128 x 192 blocks on a CU, also N % 192 == 0); the
+// gemm_nt_kernel tiles take any K % 8 == 0; gemm_rows_kernel a few rows.
 static bool linear_variant_fits(int variant, int64_t m, int n, int k) {
   const bool dma = k % 64 == 0 && k >= 256;
   switch (variant) {

@@ -69,7 +69,7 @@ const char* xb_strerror(int code);
  * and gemm_rows_kernel (ROWS). */
 #define XB_LINEAR_DMA_256x256 0
 #define XB_LINEAR_DMA_256x192 1   /* two 128 x 192 blocks per CU; also N % 192 == 0 */
-#define XB_LINEAR_DMA_128x256 2
+#define XB_LINEAR_DMA_128x256 2   /* on request only: never the library's choice */
 #define XB_LINEAR_DMA_128x128 3
 #define XB_LINEAR_NT_128x128 4
 #define XB_LINEAR_NT_64x64 5
@@ -248,10 +248,11 @@ int xb_attention_kv_cache(const void* qkv, const void* k_cache,
 /*
  * xb_attention_kv_cache without a workspace argument, for callers that cannot
  * allocate (code under hipGraph capture, tight serving loops, harnesses that
- * forbid hipMalloc).  No counterpart in the reference.  A decode chunk's
- * split partials go to a static device buffer of XB_DECODE_SCRATCH_BYTES
- * that the library holds on each GPU it runs on until the process ends; the
- * call allocates nothing.  The partials take
+ * forbid hipMalloc).  No counterpart in the reference.  The split partials,
+ * of a decode chunk and of a longer one whose keys are split, go to a static
+ * device buffer of XB_DECODE_SCRATCH_BYTES that the library holds on each GPU
+ * it runs on until the process ends; the call allocates nothing.  A decode
+ * chunk's partials take
  *   batch * heads * n_splits * 16 * (4 * head_dim + 8) bytes,
  * and the split count n_splits (>= 1; the same in both entry points, which
  * is what keeps their results equal) is capped so that this stays within
@@ -262,11 +263,13 @@ int xb_attention_kv_cache(const void* qkv, const void* k_cache,
  * head_dim 8 / 16 / 32 / 64 / 128 / 256.  Such a call returns
  * XB_ERR_SCRATCH_TOO_SMALL without launching; use xb_attention_kv_cache with
  * a workspace then (xb_attention_kv_cache_workspace_bytes gives the bytes
- * either call needs).  The stream must belong to the current device
+ * either call needs).  A longer chunk's partials always fit: its keys stay
+ * unsplit where two ranges would not.  The stream must belong to the current device
  * (XB_ERR_WRONG_DEVICE otherwise).  All calls on one GPU share its buffer:
  * calls that overlap in time on one GPU (different streams, or concurrent
- * graph replays) race and must not be issued.  Results equal
- * xb_attention_kv_cache's bit for bit.
+ * graph replays) race and must not be issued, long chunks included.  Results
+ * equal those of xb_attention_kv_cache with its full workspace bit for bit (a
+ * long chunk without one keeps its keys unsplit, which sums in another order).
  */
 #define XB_DECODE_SCRATCH_BYTES (32LL << 20)
 int xb_attention_kv_cache_noalloc(const void* qkv, const void* k_cache,
