@@ -167,12 +167,14 @@ def test_linear_every_variant(pkg, cuda, m, n, k, gelu):
     ag, wg, bg = a.to(cuda), w.to(cuda), bias.to(cuda)
     outs = {}
     for variant in (capi.XB_LINEAR_DMA_256x256, capi.XB_LINEAR_DMA_256x192, capi.XB_LINEAR_DMA_128x256,
-                    capi.XB_LINEAR_DMA_128x128, capi.XB_LINEAR_NT_128x128, capi.XB_LINEAR_NT_64x64):
+                    capi.XB_LINEAR_DMA_128x128, capi.XB_LINEAR_DMA_64x64, capi.XB_LINEAR_NT_128x128,
+                    capi.XB_LINEAR_NT_64x64):
         out = pkg.linear(ag, wg, bg, gelu=gelu, variant=variant)
         torch.testing.assert_close(out.cpu().float(), ref, atol=2e-3, rtol=2e-3,
                                    msg=lambda e, v=variant: f"variant {v}: {e}")
         outs[variant] = out
-    dma = [capi.XB_LINEAR_DMA_256x256, capi.XB_LINEAR_DMA_256x192, capi.XB_LINEAR_DMA_128x256, capi.XB_LINEAR_DMA_128x128]
+    dma = [capi.XB_LINEAR_DMA_256x256, capi.XB_LINEAR_DMA_256x192, capi.XB_LINEAR_DMA_128x256, capi.XB_LINEAR_DMA_128x128,
+           capi.XB_LINEAR_DMA_64x64]
     for v in dma[1:]:
         assert torch.equal(outs[v], outs[dma[0]]), f"variant {v} differs from {dma[0]}"
     assert torch.equal(outs[capi.XB_LINEAR_NT_64x64], outs[capi.XB_LINEAR_NT_128x128])
@@ -463,9 +465,9 @@ def test_qkv_vt_argument_errors(pkg, cuda):
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("hd,b,s,h,variants", [
     (256, 2, 300, 2, ("XB_ATTN_W4_Q16", "XB_ATTN_W8_Q16")),
-    (128, 1, 333, 2, ("XB_ATTN_W4_Q32",)),
-    (64, 2, 4100, 1, ("XB_ATTN_W4_Q32", "XB_ATTN_W4_Q64", "XB_ATTN_PINGPONG")),
-    (32, 1, 1100, 3, ("XB_ATTN_W4_Q32", "XB_ATTN_W4_Q64")),
+    (128, 1, 333, 2, ("XB_ATTN_W4_Q16", "XB_ATTN_W4_Q32")),
+    (64, 2, 4100, 1, ("XB_ATTN_W4_Q16", "XB_ATTN_W4_Q32", "XB_ATTN_W4_Q64", "XB_ATTN_PINGPONG")),
+    (32, 1, 1100, 3, ("XB_ATTN_W4_Q16", "XB_ATTN_W4_Q32", "XB_ATTN_W4_Q64")),
 ])
 def test_attention_every_variant(pkg, cuda, causal, hd, b, s, h, variants):
     """Every attention kernel the plan can name (xb_attention_v), forced on a
