@@ -11,8 +11,8 @@
 // matrix work, so it is bound by memory traffic and, on small batches, by the
 // number of launches; here a token's row stays in registers from the context
 // to the next projection and HBM sees ctx, x (in and out) and q, k, v only:
-// 16 D bytes per token instead of 44 D.  65536 tokens of width 128: 93 -> 37.5 us
-// per layer (3.6 TB/s; the reads come first and the writes last in every block,
+// 16 D bytes per token instead of 44 D.  65536 tokens of width 128: 93 -> 34 us
+// per layer (4.0 TB/s; the reads come first and the writes last in every block,
 // and one round of blocks fills the chip, so they overlap little); the 32-wide
 // model's 29 launches become 9.
 //
