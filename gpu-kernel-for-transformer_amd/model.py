@@ -212,7 +212,8 @@ class UserOptimizedTransformer(nn.Module):
     # What the forward derives from the module and rebuilds when it is missing.  A copy or a
     # saved file leaves it out (the descriptor's pointers are this process's and this model's),
     # and what a file saved with it holds is not taken over.
-    _DERIVED = ("_native_stack_cache", "_weight_cache", "_fused_stack_cache", "_tree_cache", "_mask_cache")
+    _DERIVED = ("_native_stack_cache", "_weight_cache", "_fused_stack_cache", "_tree_cache", "_mask_cache",
+                "_plans", "_plans_config")
 
     def __getstate__(self) -> dict:
         """The state that copy.deepcopy, pickle and torch.save take."""
@@ -240,7 +241,9 @@ class UserOptimizedTransformer(nn.Module):
         eligible = not per_op and self.config.d_model == 128 and self._fused_stack_eligible()
         key = (int(batch), int(seq_len), bool(padded), eligible, bool(per_op),
                self._fused_stack_enabled)
-        plans = self.__dict__.setdefault("_plans", {})
+        if self.__dict__.get("_plans_config") is not self.config:  # replaced: its plans with it
+            self.__dict__["_plans_config"], self.__dict__["_plans"] = self.config, {}
+        plans = self.__dict__["_plans"]
         plan = plans.get(key)
         if plan is None:
             plan = resolve_shape_execution_plan(self.config, batch, seq_len, masked=padded, fused_allowed=key[3],

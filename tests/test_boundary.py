@@ -325,13 +325,15 @@ def test_whole_stack_parameters_follow_functional_call(pkg, monkeypatch):
 
 
 def test_native_descriptor_follows_the_config(pkg):
-    """The descriptor's causal flag is the present config's."""
+    """The descriptor's causal flag and the plans are the present config's."""
     import dataclasses
 
     model = pkg.UserOptimizedTransformer(pkg.TransformerConfig(2, 300, 256, 4, 256, 1, True)).eval()
     assert model._native_stack(False)[0].causal == 1
+    assert "pingpong_vt" in model.execution_plan(8, 12288).attention_strategy
     model.config = dataclasses.replace(model.config, causal=False)
     assert model._native_stack(False)[0].causal == 0
+    assert model.execution_plan(8, 12288).attention_strategy == "flash_pingpong_8wave_512q"   # V^T is for causal only
 
 
 def test_fused_eligibility_checks_every_layer_norm_on_each_call(pkg):
