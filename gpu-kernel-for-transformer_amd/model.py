@@ -399,7 +399,7 @@ class UserOptimizedTransformer(nn.Module):
         if key is not None and cached is not None and cached[0] == key:
             return cached[1]
         if not self._fits_config():
-            self.__dict__["_native_stack_cache"] = (key, None)
+            self.__dict__["_native_stack_cache"] = (key, None, params)
             return None
         cfg = self.config
         blocks = (_capi.XbBlock * len(self.layers))()
@@ -421,7 +421,9 @@ class UserOptimizedTransformer(nn.Module):
                               layers=len(self.layers), heads=cfg.num_heads, head_dim=cfg.head_dim,
                               ffn_dim=cfg.ffn_dim, causal=int(cfg.causal))
         value = (stack, blocks, weights, final.weight.get_device())
-        self.__dict__["_native_stack_cache"] = (key, value)
+        # With the tensors that the key names: while it is compared against, nothing else can
+        # come to lie at their addresses (tensors swapped in for one call are freed after it).
+        self.__dict__["_native_stack_cache"] = (key, value, params)
         return value
 
     def _tree(self) -> Tuple[Tuple[nn.Parameter, ...], Tuple[nn.LayerNorm, ...]]:
@@ -485,7 +487,7 @@ class UserOptimizedTransformer(nn.Module):
             wpack = torch.cat(weights).contiguous()
             ppack = torch.cat(vectors).contiguous()
         affine_mask = self._fused_affine_mask()
-        self.__dict__["_fused_stack_cache"] = (key, wpack, ppack, affine_mask)
+        self.__dict__["_fused_stack_cache"] = (key, wpack, ppack, affine_mask, params)  # held as in _native_stack
         return wpack, ppack, affine_mask
 
     def _fused_affine_mask(self) -> int:

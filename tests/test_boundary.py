@@ -324,6 +324,28 @@ def test_whole_stack_parameters_follow_functional_call(pkg, monkeypatch):
     assert torch.equal(again[0], own[0]) and torch.equal(again[1], own[1])
 
 
+@pytest.mark.parametrize("form", ["native", "whole_stack"])
+def test_cached_addresses_stay_taken(pkg, monkeypatch, form):
+    """What was derived from tensors swapped in for one call is keyed by their addresses, so
+    they stay alive until it is replaced: the next call's cannot lie where they lay."""
+    import importlib
+    import weakref
+
+    kernels = importlib.import_module(pkg.__name__ + ".kernels")
+    monkeypatch.setattr(kernels, "pack_linear_fragments", lambda w, scale=1.0: (w.detach() * scale).half().flatten())
+    d = 128 if form == "whole_stack" else 256
+    model = pkg.UserOptimizedTransformer(pkg.TransformerConfig(2, 64, d, 4, d, 1, True)).eval()
+    derive = model._fused_stack_parameters if form == "whole_stack" else lambda: model._native_stack(False)
+    model.forward = derive
+    swapped = {name: p.detach() + 1.0 for name, p in model.named_parameters()}
+    refs = [weakref.ref(t) for t in swapped.values()]
+    torch.func.functional_call(model, swapped, ())
+    del swapped
+    assert all(ref() is not None for ref in refs)
+    derive()
+    assert all(ref() is None for ref in refs)
+
+
 def test_native_descriptor_follows_the_config(pkg):
     """The descriptor's causal flag and the plans are the present config's."""
     import dataclasses
