@@ -367,7 +367,8 @@ class UserOptimizedTransformer(nn.Module):
                     return False
                 tensors += (weight, bias)
         for norm in norms:
-            for p in (norm.weight, norm.bias):
+            held = norm._parameters  # a parametrized one is made anew on each access: nothing to point at
+            for p in (held.get("weight"), held.get("bias")):
                 if p is None or p.shape != vector or p.dtype != torch.float32 or not p.is_contiguous():
                     return False
                 tensors.append(p)

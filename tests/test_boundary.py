@@ -346,6 +346,18 @@ def test_cached_addresses_stay_taken(pkg, monkeypatch, form):
     assert all(ref() is None for ref in refs)
 
 
+def test_native_descriptor_only_for_its_own_norms(pkg):
+    """A parametrized LayerNorm weight is another tensor on each access: no descriptor points at one."""
+    model = pkg.UserOptimizedTransformer(pkg.TransformerConfig(2, 64, 256, 4, 256, 1, True)).eval()
+    torch.nn.utils.parametrize.register_parametrization(model.layers[0].norm2, "weight", torch.nn.Identity())
+    assert model._native_stack(False) is None
+    weight = model.layers[0].attention.out_proj
+    torch.nn.utils.parametrize.remove_parametrizations(model.layers[0].norm2, "weight")
+    torch.nn.utils.parametrize.register_parametrization(weight, "weight", torch.nn.Identity())
+    stack, _, weights = model._native_stack(False)[:3]     # a projection's is copied
+    assert torch.equal(weights[0].out_w, weight.weight.half())
+
+
 def test_native_descriptor_follows_the_config(pkg):
     """The descriptor's causal flag and the plans are the present config's."""
     import dataclasses
