@@ -967,3 +967,35 @@ def test_row_block_launches_are_recorded_by_form(pkg, cuda, layers):
     torch.cuda.synchronize()
     counts = {name: len(times) for name, times in recorder.durations_ms().items() if name.startswith("row_block")}
     assert counts == {"row_block_64_first": 1, "row_block_64_last": 1, **({"row_block_64_mid": layers - 1} if layers > 1 else {})}
+
+
+@pytest.mark.parametrize("geom", [(3, 60, 128, 4, 128, 3), (3, 60, 64, 4, 64, 3), (3, 60, 256, 4, 512, 3)])
+def test_forward_follows_the_model(pkg, cuda, geom):
+    """The next forward runs what the model is then, in the one-launch, row-block and per-op
+    forms: parameters swapped in for one call (freed ones' addresses used again), a layer taken
+    out, a copy; each equals a fresh model with the same state bit for bit."""
+    import copy
+
+    config = pkg.TransformerConfig(*geom, True)
+    torch.manual_seed(4)
+    model = pkg.UserOptimizedTransformer(config).to(cuda).eval()
+    x = torch.randn(*geom[:3], generator=torch.Generator().manual_seed(5)).to(cuda)
+
+    def fresh(state, layers=geom[5]):
+        twin = pkg.UserOptimizedTransformer(pkg.TransformerConfig(*geom[:5], layers, True)).to(cuda).eval()
+        twin.load_state_dict(state)
+        return twin(x)
+
+    with torch.no_grad():
+        own = model(x).clone()
+        for scale in (0.5, 1.5, 0.75, 1.25):
+            swapped = {name: p * scale for name, p in model.named_parameters()}
+            out = torch.func.functional_call(model, swapped, (x,))
+            assert torch.equal(out, fresh(swapped)), scale
+            del swapped
+        assert torch.equal(model(x), own)
+        twin = copy.deepcopy(model)
+        twin.layers[1].ffn_in.weight.mul_(0.5)
+        assert torch.equal(twin(x), fresh(twin.state_dict())) and torch.equal(model(x), own)
+        model.layers.pop(1)
+        assert torch.equal(model(x), fresh(model.state_dict(), 2))
