@@ -688,8 +688,10 @@ class UserOptimizedTransformer(nn.Module):
         """LN -> per layer (QKV GEMM, attention, out GEMM, residual LN, FFN) -> final LN, issued natively.
 
         cache_start: None, or the position in the KV cache of x's first token.
-        While a LaunchRecorder is active the same launches go through the
-        wrappers one by one, so that each is bracketed by its events.
+        While a LaunchRecorder is active the same sequence goes through the
+        wrappers one by one, so that each launch is bracketed by its events
+        (a few rows' LayerNorms and cache appends are then launches of their
+        own, with the same bits).
         """
         if plan.row_block and self.config.d_model == 32 and x.data_ptr() % 16:
             x = x.clone()  # this width's LayerNorm takes any alignment, the row blocks 16 bytes
